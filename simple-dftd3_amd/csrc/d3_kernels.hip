@@ -1022,9 +1022,9 @@ __global__ void atm_acc_kernel(DevBatch b, const double4* __restrict__ acc, doub
 
 // Three-body hot path: x**y for x > 0, 1/x and 1/sqrt(x) for normal x > 0.
 // FP32 uses the hardware approximations (v_exp_f32, v_log_f32, v_rcp_f32,
-// v_rsq_f32, about 1 ulp); FP64 the device-library functions, except 1/x:
-// the hardware reciprocal refined by two Newton steps (about 1 ulp, not the
-// correctly rounded division).
+// v_rsq_f32, about 1 ulp); FP64 the device-library functions for the power,
+// and the hardware estimates of 1/x and 1/sqrt(x) refined by one third-order
+// step each (about 1 ulp, not correctly rounded).
 template <typename R> __device__ __forceinline__ R pow_pos(R x, R y);
 template <> __device__ __forceinline__ double pow_pos<double>(double x, double y) { return exp2(y * log2(x)); }
 template <> __device__ __forceinline__ float pow_pos<float>(float x, float y) {
@@ -1032,32 +1032,32 @@ template <> __device__ __forceinline__ float pow_pos<float>(float x, float y) {
 }
 // x**(-8/3) for normal x > 0, the damping power of the default alp = 14
 // (alp + 2 = 16, (r0/r)^((alp + 2)/3) with x = r^2): the FP32 hardware
-// estimate scaled into range in FP64, then two Newton steps on
-// t^6 x^16 = 1, t <- t + t (1 - t^6 x^16) / 6 (quadratic convergence from
-// ~2e-7: about one ulp).  The general power costs the device library's
-// log2 and exp2 in FP64.
+// estimate scaled into range in FP64, then one third-order step on
+// h = 1 - t^3 x^8, t <- t (1 + h / 3 + 2 h^2 / 9) (the estimate is good to
+// 2e-6, so the h^3 term dropped is below 1e-17): 9 FP64 operations where two
+// Newton steps on t^6 x^16 took 16.  The general power costs the device
+// library's log2 and exp2 in FP64.
 __device__ __forceinline__ double pow_m8_3(double x) {
   const float e = (-8.0f / 3.0f) * __builtin_amdgcn_logf(static_cast<float>(x));
   const float k = __builtin_rintf(e);
-  double t = ldexp(static_cast<double>(__builtin_amdgcn_exp2f(e - k)), static_cast<int>(k));
-  const double x2 = x * x, x4 = x2 * x2, x8 = x4 * x4, x16 = x8 * x8;
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const double t2 = t * t, t6 = t2 * t2 * t2;
-    const double r = fma(-t6, x16, 1.0);
-    t = fma(t * r, 1.0 / 6.0, t);
-  }
-  return t;
+  const double t = ldexp(static_cast<double>(__builtin_amdgcn_exp2f(e - k)), static_cast<int>(k));
+  const double x2 = x * x, x4 = x2 * x2, x8 = x4 * x4;
+  const double h = fma(-(t * t * t), x8, 1.0);
+  return fma(t * h, fma(h, 2.0 / 9.0, 1.0 / 3.0), t);
 }
 template <typename R> __device__ __forceinline__ R rcp_fast(R x);
-template <> __device__ __forceinline__ double rcp_fast<double>(double x) {  // v_rcp_f64, two Newton steps
-  double r = __builtin_amdgcn_rcp(x);
-  r = fma(r, fma(-x, r, 1.0), r);
-  return fma(r, fma(-x, r, 1.0), r);
+template <> __device__ __forceinline__ double rcp_fast<double>(double x) {  // v_rcp_f64, one third-order step
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 }
 template <> __device__ __forceinline__ float rcp_fast<float>(float x) { return __builtin_amdgcn_rcpf(x); }
 template <typename R> __device__ __forceinline__ R rsqrt_fast(R x);
-template <> __device__ __forceinline__ double rsqrt_fast<double>(double x) { return rsqrt(x); }
+template <> __device__ __forceinline__ double rsqrt_fast<double>(double x) {  // v_rsq_f64, one third-order step
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
 template <> __device__ __forceinline__ float rsqrt_fast<float>(float x) { return __builtin_amdgcn_rsqf(x); }
 
 // atm.f90:625-825 get_atm_dispersion_derivs (kGrad) and atm.f90:500-621,
