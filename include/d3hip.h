@@ -230,7 +230,7 @@ D3HIP_API void d3hip_get_dispersion_batch(dftd3_error error, dftd3_model workspa
  * which keeps the last call's contents.  Same arguments and results as
  * d3hip_get_dispersion_batch otherwise (including the read-back of the
  * three-body list size). */
-#define D3HIP_NOALLOC_BYTES (64u << 20)
+#define D3HIP_NOALLOC_BYTES (65u << 20)
 D3HIP_API void d3hip_get_dispersion_batch_noalloc(dftd3_error error, int nsys, const int* natoms,
                                                   const int* numbers, const double* lattices, const bool* periodic,
                                                   const double* params, const double* cutoffs, int precision,

@@ -202,6 +202,7 @@ struct Prepared {
   bool smooth = false;         // some three-body system has a nonzero width3
   bool periodic_atm = false;   // some three-body system has lattice images
   bool partitioned = false;    // some system evaluates one part of a work partition
+  bool any_cull = false;       // some system is a molecule of more than 8 tiles
   bool fixed_order = false;    // one system of at most 8 tiles: storage order = atom order, no sort
   long long slot_bound = 0;    // sum over three-body systems of (il + 1) * images
   long long atm_atoms = 0;     // atoms of the systems with a three-body term
@@ -355,7 +356,7 @@ AtmShape per_call_shape(bool mixed, bool periodic, long long items) {
 
 struct Workspace {
   DeviceBuffer meta, pos, rank, order, sort_tmp, cn, gw, dgw, pair, e_atom, dedcn, grad, sig, atm_acc, cnt, off,
-      item_off, slots, gw_rank, sp_rank, pos_rank, tbox, counts, counter, flag, pair3s, hbuf, e_out, ew_tab, ew_c6l, ew_lc6l, ew_ldc6l, ew_part,
+      item_off, items, slots, gw_rank, sp_rank, pos_rank, tbox, counts, counter, flag, pair3s, hbuf, e_out, ew_tab, ew_c6l, ew_lc6l, ew_ldc6l, ew_part,
       ew_phi, ew_f, ew_s, sp_base, sp_theta, sp_dtheta, sp_q, sp_qh, sp_th, sp_k, sp_dm, sp_dmir;
   // batched real <-> half-complex 3D transforms of the particle mesh (one per
   // species), kept while the mesh and the species count stay the same
@@ -392,7 +393,7 @@ struct Workspace {
   Arena* arena = nullptr;
   std::vector<DeviceBuffer*> buffers() {
     return {&meta, &pos, &rank, &order, &sort_tmp, &cn, &gw, &dgw, &pair, &e_atom, &dedcn, &grad, &sig, &atm_acc, &cnt, &off,
-            &item_off, &slots, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
+            &item_off, &items, &slots, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
             &e_out, &ew_tab, &ew_c6l, &ew_lc6l, &ew_ldc6l, &ew_part, &ew_phi, &ew_f, &ew_s, &sp_base, &sp_theta,
             &sp_dtheta, &sp_q, &sp_qh, &sp_th, &sp_k, &sp_dm, &sp_dmir};
   }
@@ -434,7 +435,7 @@ struct Workspace {
   }
   DevWork work(const Prepared& pb, bool mixed, bool grad, const BatchOutput& out, const BatchDebug* debug);
   // count -> scans of the list sizes and of their work items (three-body lists of every atom)
-  void list_offsets(const Prepared& pb, const void* pair, bool mixed, double4* acc, hipStream_t stream);
+  void list_offsets(const DevBatch& db, const void* pair, bool mixed, double4* acc, int2* items, hipStream_t stream);
   // pack .. disp2; then the three-body lists and kernel; then the chain
   // rule and the reduction.  capacity < 0: read the list size back and size
   // the slot buffer to it; otherwise use the fixed capacity and item bound.
@@ -570,6 +571,7 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
     // tile culling for molecules of more than 8 tiles (in smaller ones every
     // tile is usually within the cutoffs and the box tests only cost)
     g.cull = !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2]) && sd.natoms > 8 * kTile;
+    pb.any_cull = pb.any_cull || g.cull;
     for (int t = 0; t * kTile < sd.natoms; ++t)
       tiles.push_back(make_int2(g.atom_begin + t * kTile, std::min(kTile, sd.natoms - t * kTile)));
     if (std::fabs(sd.param.s9) >= kEps) {
@@ -803,22 +805,28 @@ DevWork Workspace::work(const Prepared& pb, bool mixed, bool grad, const BatchOu
   return w;
 }
 
-void Workspace::list_offsets(const Prepared& pb, const void* pair_records, bool mixed, double4* acc,
+void Workspace::list_offsets(const DevBatch& db, const void* pair_records, bool mixed, double4* acc, int2* items,
                              hipStream_t stream) {
-  const int natoms = pb.db.natoms;
+  const int natoms = db.natoms;
   long long* c = cnt.as<long long>(natoms);
   long long* o = off.as<long long>(natoms + 1);
   long long* io = item_off.as<long long>(natoms + 1);
   timed("atm_list", stream, [&] {
-    launch_atm_count(pb.db, pair_records, mixed, c, acc, stream);
-    launch_list_scan(c, natoms, o, io, stream);
+    launch_atm_count(db, pair_records, mixed, c, acc, stream);
+    launch_list_scan(db, c, o, io, items, stream);
   });
 }
 
 void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool order_atoms, bool mixed, bool grad,
                          bool smooth, const BatchOutput& out, const BatchDebug* debug, RunStats* stats,
                          long long capacity, long long max_items, const AtmShape& shape, hipStream_t stream) {
-  const DevBatch& db = pb.db;
+  DevBatch db = pb.db;
+  // the Hessian (stats) and the work partition go by the reference's triangle
+  db.rank_own = pb.any_cull && !pb.partitioned && !stats;
+  // lists of lattice images, taken atom by atom, gain nothing from an XCD's own
+  // range (2,000-atom cell, mixed: 14.1 ms with one queue, 14.7 with eight;
+  // batch of 1,024 molecules, FP64: 6.0 and 5.7 ms)
+  db.xcd_queues = !pb.periodic_atm;
   const int natoms = db.natoms;
   pack(pb, positions_dev, stream, order_atoms);
   const DevWork w = work(pb, mixed, grad, out, debug);
@@ -885,15 +893,18 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
     timed("ewald_atom", stream, [&] { launch_ewald_atom(e, grad, w, ew, stream); });
   }
   if (pb.any_atm) {
-    list_offsets(pb, w.pair, mixed, w.atm_acc, stream);
+    const long long bound_bytes = pb.slot_bound * static_cast<long long>(slot_record_bytes(mixed));
+    // molecules whose exact list bound (j <= i: il + 1 slots per atom) fits a
+    // modest buffer: no read-back of the list size, so the call does not wait
+    // for the device here
+    const bool bounded = capacity < 0 && !stats && !arena && !pb.periodic_atm && bound_bytes <= kUnsyncedSlotBytes;
+    int2* it = nullptr;
+    if (bounded && list_scan_writes_items(db)) it = items.as<int2>(std::max<long long>(pb.item_bound, 1));
+    list_offsets(db, w.pair, mixed, w.atm_acc, it, stream);
     long long* o = off.as<long long>(natoms + 1);
     long long* io = item_off.as<long long>(natoms + 1);
     void* s = nullptr;
-    const long long bound_bytes = pb.slot_bound * static_cast<long long>(slot_record_bytes(mixed));
-    if (capacity < 0 && !stats && !arena && !pb.periodic_atm && bound_bytes <= kUnsyncedSlotBytes) {
-      // molecules whose exact list bound (j <= i: il + 1 slots per atom)
-      // fits a modest buffer: no read-back of the list size, so the call
-      // does not wait for the device here
+    if (bounded) {
       capacity = std::max<long long>(pb.slot_bound, 1);
       max_items = pb.item_bound;
       s = slots.get(capacity * slot_record_bytes(mixed));
@@ -909,11 +920,17 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
       s = slots.get(std::max<long long>(capacity, 1) * slot_record_bytes(mixed));
       launch_atm_guard(db, o, capacity, io, flag.as<int>(1), w, grad, stream);
     }
-    timed("atm_list", stream, [&] { launch_atm_fill(db, w.pair, mixed, o, s, capacity, stream); });
+    timed("atm_list", stream, [&] {
+      if (!it) {
+        it = items.as<int2>(std::max<long long>(max_items, 1));
+        launch_item_table(db, cnt.as<long long>(natoms), io, it, stream);
+      }
+      launch_atm_fill(db, w.pair, mixed, o, s, capacity, stream);
+    });
     const AtmShape sh = shape.waves == 0 ? per_call_shape(mixed, pb.periodic_atm, max_items) : shape;
-    unsigned long long* wc = sh.blocks_per_cu > 0 ? counter.as<unsigned long long>(1) : nullptr;
+    unsigned long long* wc = sh.blocks_per_cu > 0 ? counter.as<unsigned long long>(kXcd * kCounterStride) : nullptr;
     timed("atm", stream,
-          [&] { launch_atm(db, mixed, grad, smooth, pb.partitioned, sh, io, max_items, o, s, w, wc, stream); });
+          [&] { launch_atm(db, mixed, grad, smooth, pb.partitioned, sh, io, it, max_items, o, s, w, wc, stream); });
   }
   if (grad) timed("cn_chain", stream, [&] { launch_cn_chain(db, mixed, w, stream); });
   timed("reduce", stream, [&] { launch_reduce(db, w, out.energy, grad ? out.sigma : nullptr, stream); });
@@ -996,16 +1013,20 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
   } else {
     double* S = m.pair3s.as<double>(static_cast<size_t>(pb.pair_total));
     hip_check(hipMemsetAsync(S, 0, bytes, stream), "hipMemsetAsync");
-    m.list_offsets(pb, w.pair, mixed, nullptr, stream);
+    m.list_offsets(db, w.pair, mixed, nullptr, nullptr, stream);
     long long* o = m.off.as<long long>(natoms + 1);
     long long* io = m.item_off.as<long long>(natoms + 1);
     long long total = 0;
     hip_check(hipMemcpyAsync(&total, o + natoms, sizeof total, hipMemcpyDeviceToHost, stream), "list size");
     hip_check(hipStreamSynchronize(stream), "list size sync");
     void* sl = m.slots.get(std::max<long long>(total, 1) * slot_record_bytes(mixed));
-    m.timed("atm_list", stream, [&] { launch_atm_fill(db, w.pair, mixed, o, sl, total, stream); });
+    int2* it = m.items.as<int2>(static_cast<size_t>(total / kTile + natoms));
+    m.timed("atm_list", stream, [&] {
+      launch_item_table(db, m.cnt.as<long long>(natoms), io, it, stream);
+      launch_atm_fill(db, w.pair, mixed, o, sl, total, stream);
+    });
     m.timed("atm", stream, [&] {
-      launch_atm_pairs(db, mixed, pb.smooth, io, total / kTile + natoms, o, sl, w, S, stream);
+      launch_atm_pairs(db, mixed, pb.smooth, io, it, total / kTile + natoms, o, sl, w, S, stream);
       launch_pair3_finalize(db, S, pair3, stream);
     });
   }
@@ -1075,7 +1096,7 @@ void Engine::count_terms(const std::vector<SystemDesc>& systems, const int* numb
   hip_check(hipMemsetAsync(dc, 0, sizeof(unsigned long long) * 3 * pb.db.nsys, stream), "hipMemsetAsync");
   launch_count_pairs(pb.db, dc, stream);
   // lists without the C6 test: every pair within the cutoff is a slot
-  m.list_offsets(pb, nullptr, false, nullptr, stream);
+  m.list_offsets(pb.db, nullptr, false, nullptr, nullptr, stream);
   long long* o = m.off.as<long long>(natoms + 1);
   long long total = 0;
   hip_check(hipMemcpyAsync(&total, o + natoms, sizeof total, hipMemcpyDeviceToHost, stream), "list size");
@@ -1138,7 +1159,7 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
         launch_cn(s.pb.db, s.mixed, w.cn, stream);
         launch_weights(s.pb.db, w.cn, w.gw, w.dgw, stream);
         launch_pair(s.pb.db, s.mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, stream);
-        s.ws.list_offsets(s.pb, w.pair, s.mixed, w.atm_acc, stream);
+        s.ws.list_offsets(s.pb.db, w.pair, s.mixed, w.atm_acc, nullptr, stream);
         long long total = 0;
         hip_check(hipMemcpyAsync(&total, s.ws.off.as<long long>(natoms + 1) + natoms, sizeof total,
                                  hipMemcpyDeviceToHost, stream),
@@ -1153,7 +1174,8 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
       s.shape.blocks_per_cu = a.blocks_per_cu;
       // size every buffer now, so that an evaluation allocates nothing
       (void)s.ws.slots.get(std::max<long long>(cap, 1) * slot_record_bytes(s.mixed));
-      (void)s.ws.counter.as<unsigned long long>(1);
+      (void)s.ws.items.as<int2>(std::max<long long>(s.max_items, 1));
+      (void)s.ws.counter.as<unsigned long long>(kXcd * kCounterStride);
     }
     (void)s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
     hip_check(hipStreamSynchronize(stream), "plan sync");

@@ -158,6 +158,32 @@ __device__ __forceinline__ unsigned long long near_tiles(const DevBatch& b, cons
   return __ballot(near);
 }
 
+// The three-body lists of a system hold j <= i (the reference's triangle), or,
+// in an energy evaluation of a large molecule, the atoms before i in the
+// storage order: neighbouring atoms then have nearly the same list, and a tile
+// holds a compact, gap-free run of that order (20,000-atom ellipsoid, mixed
+// three-body kernel: 78 ms with j <= i, 62 ms with the storage order).  The
+// triple set is the same, but a distance that the reference forms from
+// another atom of the triple can round to the other side of the cutoff, so
+// distances within kBand of it are decided by triple_in_range.
+constexpr double kBand = 1.0e-9;
+__device__ __forceinline__ bool rank_owned(const DevBatch& b, const SysGeom& g) { return b.rank_own && g.cull; }
+
+// Whether the reference takes the triple of three different atoms of a system
+// without lattice images: the distances of the atom with the largest index
+// from the other two and, from these vectors, the third (atm.f90:706-724).
+__device__ __attribute__((noinline)) bool triple_in_range(const double4* __restrict__ pos, int i, int j, int k,
+                                                          double cut2) {
+  const int o = max(i, max(j, k));
+  const int p = o == i ? j : i, q = o == k ? j : k;
+  const double4 xo = pos[o], t0 = make_double4(0.0, 0.0, 0.0, 0.0);
+  double p0, p1, p2, q0, q1, q2, d0, d1, d2;
+  const double rp = atm_vec(pos[p], t0, xo, p0, p1, p2);
+  const double rq = atm_vec(pos[q], t0, xo, q0, q1, q2);
+  const double rd = diff_norm2(q0, q1, q2, p0, p1, p2, d0, d1, d2);
+  return rp <= cut2 && rp >= kEps && rq <= cut2 && rq >= kEps && rd <= cut2 && rd >= kEps;
+}
+
 // cutoff.f90:73-99 smooth_cutoff
 template <typename R>
 __device__ __forceinline__ void smooth_cutoff(R r, R cutoff, R width, R& sw, R& dswdr) {
@@ -768,11 +794,12 @@ __global__ __launch_bounds__(kBlock) void atm_list_kernel(DevBatch b, const R4<R
     if (!kFill && lane == 0) count[i] = 0;
     return;
   }
-  const double cut2 = p.cut3 * p.cut3;
+  const bool by_rank = rank_owned(b, g);
+  const double cut2 = p.cut3 * p.cut3 * (by_rank ? 1.0 + kBand : 1.0);
   const R malp6 = -(R(p.alp) + R(2)) / R(6);  // exponent of r2 in (r0/r)^(alp/3)
   const double4 xi = b.pos[i];
-  const int n = g.natoms;
-  const R4<R>* row = pair ? pair + g.c6_begin + static_cast<long long>(b.rank[i]) * n : nullptr;
+  const int n = by_rank ? b.rank[i] : g.natoms;  // partners: the positions before n
+  const R4<R>* row = pair ? pair + g.c6_begin + static_cast<long long>(b.rank[i]) * g.natoms : nullptr;
   Slot<R>* out = kFill ? slots + offset[i] : nullptr;
   long long total = 0;
   unsigned long long near = 0;
@@ -783,7 +810,7 @@ __global__ __launch_bounds__(kBlock) void atm_list_kernel(DevBatch b, const R4<R
     const int r = r0 + lane;
     const int j = r < n ? b.order[g.atom_begin + r] : i + 1;
     int cnt = 0;
-    bool valid = j <= i;
+    bool valid = by_rank ? r < n : j <= i;
     R4<R> q{};
     if (valid && row) {
       q = row[r];
@@ -828,25 +855,65 @@ __global__ __launch_bounds__(kBlock) void atm_list_kernel(DevBatch b, const R4<R
   if (!kFill && lane == 0) count[i] = total;
 }
 
-// The list offsets and the work-item offsets of n atoms in one block:
-// offset[0..n] = exclusive scan of the list sizes count[k], item_off[0..n] =
-// exclusive scan of their tile counts ceil(count[k] / 64).  Each thread sums
-// a chunk of consecutive atoms; the chunk sums are scanned across the
-// wavefronts (wavefront scans, then a scan of the wavefront totals).
-constexpr int kScanBlock = 1024;
-__global__ __launch_bounds__(kScanBlock) void list_scan_kernel(const long long* __restrict__ count, int n,
-                                                                long long* __restrict__ offset,
-                                                                long long* __restrict__ item_off) {
-  __shared__ long long wtot[2][kScanBlock / kWave];
-  const int tid = threadIdx.x, lane = wave_lane(), w = tid >> 6;
-  const int chunk = (n + kScanBlock - 1) / kScanBlock;
-  const int lo = min(n, tid * chunk), hi = min(n, lo + chunk);
-  long long s0 = 0, s1 = 0;
-  for (int k = lo; k < hi; ++k) {
-    const long long c = count[k];
-    s0 += c;
-    s1 += (c + kTile - 1) / kTile;
+__device__ __forceinline__ long long tiles_of(long long slots) { return (slots + kTile - 1) / kTile; }
+
+// The work items (atom i, 64-slot tile P of its list) in the order the
+// three-body kernel takes them, the last atoms of the storage order (the
+// longest lists) first.  Systems without lattice images: the atoms in groups
+// of kWave positions, within a group P by P, so that items taken at about the
+// same time pair the same slots for neighbouring atoms and read the same pair
+// records (see atm_body; batch of 1,024 molecules, FP64: 5.7 against 6.0 ms
+// atom by atom).  Lists of lattice images: atom by atom (the records repeat
+// within a tile, and the group order makes the slot sums of 64 atoms meet in
+// the same cache lines: 2,000-atom cell, mixed 14.1 against 15.2 ms).
+// Wavefront per 64-position tile.
+__device__ __forceinline__ void emit_items(const DevBatch& b, int t, const long long* count, const long long* item_off,
+                                           long long total, int2* items) {
+  const int lane = wave_lane();
+  const int2 tile = b.tiles[t];
+  int i = 0, nb = 0;
+  long long end = 0;
+  if (lane < tile.y) {
+    i = b.order[tile.x + lane];
+    nb = static_cast<int>(tiles_of(count[i]));
+    end = item_off[tile.x + lane] + nb;
   }
+  if (b.geom[b.sys[b.order[tile.x]]].img3_count > 1) {
+    for (int P = 0; P < nb; ++P) items[total - end + P] = make_int2(i, P);
+    return;
+  }
+  long long out = total - __shfl(end, tile.y - 1, kWave);
+  for (int P = 0;; ++P) {
+    const unsigned long long has = __ballot(P < nb);
+    if (!has) break;
+    if (P < nb) items[out + __popcll(has & ((1ull << lane) - 1))] = make_int2(i, P);
+    out += __popcll(has);
+  }
+}
+
+// The list offsets and the work-item offsets of n atoms: offset[0..n] =
+// exclusive scan of the list sizes count[i] over the atoms, item_off[0..n] =
+// exclusive scan of their tile counts ceil(count[order[x]] / 64) over the
+// storage positions x.  One thread per element; a block first sums all
+// elements before its own (coalesced, from the L2), so one launch without a
+// serial chain over the blocks does both scans.  With items (a launch of one
+// block, kScanBlock atoms or fewer) it writes the item table too.
+constexpr int kScanBlock = 1024;
+__global__ __launch_bounds__(kScanBlock) void list_scan_kernel(DevBatch b, const long long* count, long long* offset,
+                                                                long long* item_off, int2* items) {
+  const int n = b.natoms;
+  const int* __restrict__ order = b.order;
+  constexpr int kNw = kScanBlock / kWave;
+  __shared__ long long wtot[2][kNw], before[2][kNw];
+  const int tid = threadIdx.x, lane = wave_lane(), w = tid >> 6;
+  const int base = blockIdx.x * kScanBlock;
+  long long b0 = 0, b1 = 0;
+  for (int k = tid; k < base; k += kScanBlock) {  // before this block, any order of the atoms
+    b0 += count[k];
+    b1 += tiles_of(count[order[k]]);
+  }
+  const int k = base + tid;
+  const long long s0 = k < n ? count[k] : 0, s1 = k < n ? tiles_of(count[order[k]]) : 0;
   long long i0 = s0, i1 = s1;  // inclusive scans within the wavefront
 #pragma unroll
   for (int off = 1; off < kWave; off <<= 1) {
@@ -856,41 +923,46 @@ __global__ __launch_bounds__(kScanBlock) void list_scan_kernel(const long long* 
       i1 += y1;
     }
   }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    b0 += __shfl_xor(b0, off, kWave);
+    b1 += __shfl_xor(b1, off, kWave);
+  }
   if (lane == kWave - 1) {
     wtot[0][w] = i0;
     wtot[1][w] = i1;
+    before[0][w] = b0;
+    before[1][w] = b1;
   }
   __syncthreads();
-  if (w == 0) {  // exclusive scan of the wavefront totals
-    constexpr int kNw = kScanBlock / kWave;
-    long long t0 = lane < kNw ? wtot[0][lane] : 0, t1 = lane < kNw ? wtot[1][lane] : 0;
-    const long long e0 = t0, e1 = t1;
-#pragma unroll
-    for (int off = 1; off < kNw; off <<= 1) {
-      const long long y0 = __shfl_up(t0, off, kWave), y1 = __shfl_up(t1, off, kWave);
-      if (lane >= off) {
-        t0 += y0;
-        t1 += y1;
-      }
-    }
-    if (lane < kNw) {
-      wtot[0][lane] = t0 - e0;
-      wtot[1][lane] = t1 - e1;
-    }
-    if (lane == kNw - 1) {
-      offset[n] = t0;
-      item_off[n] = t1;
-    }
+  long long r0 = i0 - s0, r1 = i1 - s1;
+  for (int q = 0; q < kNw; ++q) {
+    r0 += before[0][q] + (q < w ? wtot[0][q] : 0);
+    r1 += before[1][q] + (q < w ? wtot[1][q] : 0);
   }
-  __syncthreads();
-  long long r0 = wtot[0][w] + i0 - s0, r1 = wtot[1][w] + i1 - s1;
-  for (int k = lo; k < hi; ++k) {
-    const long long c = count[k];
+  if (k < n) {
     offset[k] = r0;
     item_off[k] = r1;
-    r0 += c;
-    r1 += (c + kTile - 1) / kTile;
   }
+  if (k == n - 1) {
+    offset[n] = r0 + s0;
+    item_off[n] = r1 + s1;
+  }
+  if (!items) return;
+  __shared__ long long total;
+  if (k == n - 1) total = r1 + s1;
+  __syncthreads();
+  for (int t = w; t < b.ntiles; t += kNw) emit_items(b, t, count, item_off, total, items);
+}
+
+// Wavefront per tile; nothing when item_off[natoms] is 0: no list, or lists
+// that do not fit.
+__global__ __launch_bounds__(kBlock) void item_table_kernel(DevBatch b, const long long* __restrict__ count,
+                                                            const long long* __restrict__ item_off,
+                                                            int2* __restrict__ items) {
+  const int t = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  const long long total = item_off[b.natoms];
+  if (t < b.ntiles && total > 0) emit_items(b, t, count, item_off, total, items);
 }
 
 // --------------------------------------------------------- three-body term
@@ -941,7 +1013,8 @@ __device__ __forceinline__ int load_tile(TileSlots<R>* T, const Slot<R>* __restr
   // fails every distance test
   vx = 1e30; vy = 1e30; vz = 1e30;
   if (T) {
-    T->g0[l] = make_r4<R>(R(0), R(0), R(0), R(0));
+    const R far = sizeof(R) == 8 ? R(1e30) : R(0);
+    T->g0[l] = make_r4<R>(far, far, far, R(0));
     T->g1[l] = make_r4<R>(R(0), R(0), R(0), R(0));
     T->rank[l] = 0;
   }
@@ -1060,6 +1133,65 @@ template <> __device__ __forceinline__ double rsqrt_fast<double>(double x) {  //
 }
 template <> __device__ __forceinline__ float rsqrt_fast<float>(float x) { return __builtin_amdgcn_rsqf(x); }
 
+// One triple of atom i: A = r_ij^2, B = r_ik^2, C = r_jk^2, the slots' and
+// the (j, k) pair's records, pjk = (r0_jk/r_jk)^(alp/3), both: the two slots
+// are images of atom i.  dE with the weight of the triple; with kGrad the
+// radial factors f_X (dG_X = f_X v_X).  Formulas at atm_body.
+template <typename R>
+struct TripleTerm {
+  R dE, fA, fB, fC;
+};
+template <typename R, bool kGrad, bool kSmooth>
+__device__ __forceinline__ TripleTerm<R> triple_term(R A, R B, R C, const R4<R>& a1, const R4<R>& b1, const R4<R>& q,
+                                                     R pjk, bool both, R ns9, R alp2, R cutr, R width) {
+  TripleTerm<R> t{R(0), R(0), R(0), R(0)};
+  const R AB = A * B;
+  const R S = AB * C;
+  const R ir1 = rsqrt_fast(S);
+  const R ir2 = ir1 * ir1;
+  const R ir5 = ir2 * ir2 * ir1;
+  const R dab = A - B;
+  const R t1 = (A + B) - C, t2 = dab + C, t3 = C - dab;
+  const R u = t2 * t3, v = t1 * t3, wv = t1 * t2;
+  const R Pt = t1 * u;
+  const R core = R(0.375) * Pt + S;
+  const R ang = ir5 * core;
+  const R pp = a1.x * b1.x * (q.w * pjk);
+  const R fd = rcp_fast(R(1) + R(6) * pp);
+  R c9 = ns9 * a1.y * b1.y * q.x;
+  if (both) c9 *= R(4.0 / 3.0);  // j == k == i
+  const R cwf = c9 * fd;
+  t.dE = ang * cwf;
+  R sw = R(1), swa = R(1), dswa = R(0), swb = R(1), dswb = R(0), swc = R(1), dswc = R(0);
+  if (kSmooth) {
+    const R ra = d_sqrt(A), rb = d_sqrt(B), rc = d_sqrt(C);
+    smooth_cutoff(ra, cutr, width, swa, dswa);
+    smooth_cutoff(rb, cutr, width, swb, dswb);
+    smooth_cutoff(rc, cutr, width, swc, dswc);
+    dswa /= ra; dswb /= rb; dswc /= rc;
+    sw = swa * swb * swc;
+  }
+  if (kGrad) {
+    const R Y = alp2 * pp * fd;
+    const R sgm = u + v + wv;
+    const R K1 = R(-1.875) * Pt - R(3) * S + Y * core;
+    const R hA = R(0.75) * A * (sgm - R(2) * wv) + K1;
+    const R hB = R(0.75) * B * (sgm - R(2) * v) + K1;
+    const R hC = R(0.75) * C * (sgm - R(2) * u) + K1;
+    const R om = -cwf * ir5 * ir2;  // 1/X = (S/X) / S
+    t.fA = om * hA * (B * C);
+    t.fB = om * hB * (A * C);
+    t.fC = om * hC * AB;
+    if (kSmooth) {  // atm.f90:754-790, switching-function terms
+      t.fA = sw * t.fA - t.dE * dswa * swb * swc;
+      t.fB = sw * t.fB - t.dE * dswb * swa * swc;
+      t.fC = sw * t.fC - t.dE * dswc * swa * swb;
+    }
+  }
+  if (kSmooth) t.dE *= sw;
+  return t;
+}
+
 // atm.f90:625-825 get_atm_dispersion_derivs (kGrad) and atm.f90:500-621,
 // with rs9 = 4/3 and alp + 2 (rational.f90:563, zero.f90:602).
 //
@@ -1093,9 +1225,27 @@ template <> __device__ __forceinline__ float rsqrt_fast<float>(float x) { return
 // kSmooth adds the switching function of a nonzero width3 (cutoff.f90:73-99,
 // atm.f90:720-790).
 //
-// Work items are taken in reverse order (the longest slot lists first):
-// block k takes item total-1-k, or, with a work counter (persistent launch),
-// the items total-1-c for the counter values c it draws until none is left.
+// Work items come from the item table (emit_items), the longest slot lists
+// first: block k takes item k, or, with a work counter (persistent launch),
+// the items it draws until none is left.
+//
+// kDense (batches with a system of more than 8 tiles and no lattice images):
+// tile pairs of which most sampled slot pairs are within the cutoff skip the
+// ring.  Every group of 8 lanes takes a row of the A tile and walks the
+// B tile in blocks of 8 consecutive slots (b = l xor 8k), so the group's pair
+// records lie in two or three cache lines where the ring's lanes each read a
+// line of their own; the a-slot's sums stay in registers (summed over the 8
+// lanes once per row) and the b-slots' LDS additions hit distinct addresses.
+// In large molecules the gather of the pair records from beyond the L2 was
+// the limit (without it 56 of 99 ms, 20,000-atom ellipsoid, mixed); the
+// lists by storage order and the item order let neighbouring atoms share
+// lines.  20,000-atom ellipsoid, mixed, whole step 111.8 -> 78.1 ms;
+// 1,501-atom molecule, FP64 energy 2.55 -> 1.81 ms.  Where a tile pair is
+// mostly out of range the ring's compaction is cheaper: the share at which
+// the dense form is taken, 0.6 of the sample, is the middle of a flat range
+// (0.45, 0.6, 0.75: 79.2, 78.3, 79.2 ms).  Batches of smaller molecules and
+// of cells keep the ring alone, whose kernel needs fewer registers (2,000-atom
+// cell, mixed: 14.1 against 15.0 ms with both forms in one kernel).
 //
 // kPairs (energy only) distributes every triple term over the pairs of its
 // atoms, the pairwise three-body energy of atm.f90:829-950: a sixth of the
@@ -1106,6 +1256,10 @@ template <> __device__ __forceinline__ float rsqrt_fast<float>(float x) { return
 // pair-record index, {i, s} per slot s at (rank_i, rank_s) when the slot is
 // flushed.  The pair energy of (x, y) is then pair3s(rx, ry) + pair3s(ry, rx)
 // (pair3_finalize_kernel).
+// A tile pair of which kDenseShare or more of the kSample * 64 sampled slot
+// pairs are within the cutoff is evaluated densely.
+constexpr int kSample = 8;
+constexpr int kDenseShare = kSample * kWave * 6 / 10;
 constexpr int kAccPairs = 1;  // per-slot sums of the pairwise mode: sum t
 
 // Lane l receives the value of lane (l + 1) mod 64 (DPP wave_rol:1; every
@@ -1115,13 +1269,24 @@ __device__ __forceinline__ double wave_rotate1(double v) {
   return __hiloint2double(wave_rotate1(__double2hiint(v)), wave_rotate1(__double2loint(v)));
 }
 
-template <typename R, bool kGrad, bool kSmooth, int kW, bool kPairs, bool kPart = false>
+// The double of another lane of the same row of 16, by DPP control C.
+template <int C>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int hi = __double2hiint(v), lo = __double2loint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, C, 0xF, 0xF, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, C, 0xF, 0xF, false));
+}
+
+template <typename R, bool kGrad, bool kSmooth, int kW, bool kPairs, bool kPart = false, bool kDense = false>
 __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict__ item_off,
+                                         const int2* __restrict__ items,
                                          const long long* __restrict__ offset, const Slot<R>* __restrict__ slots,
                                          const R4<R>* __restrict__ pair, double* __restrict__ e_atom,
                                          double* __restrict__ dedcn, double* __restrict__ grad,
                                          double* __restrict__ sig_atom, double4* __restrict__ slot_acc,
-                                         unsigned long long* __restrict__ work_counter, double* __restrict__ pair3s) {
+                                         unsigned long long* __restrict__ work_counter, double* __restrict__ pair3s,
+                                         int queues) {
+  static_assert(!(kDense && (kPairs || kPart)), "dense tile pairs: energy kernels only");
   static_assert(!(kGrad && kPairs), "the pairwise mode is energy only");
   constexpr int kNAcc = kGrad ? kAcc : (kPairs ? kAccPairs : 0);
   constexpr int kAccLen = kNAcc > 0 ? kNAcc * kTile : 1;
@@ -1135,25 +1300,34 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   __shared__ PairEntry<R> ring[kW][kQueue];
   __shared__ double red[kW];
   __shared__ long long next_item;
+  // FP64 vectors of the tiles' slots (dense FP32 instantiations)
+  __shared__ double avec[3][kDense ? kTile : 1];
+  __shared__ double bvec[kDense && sizeof(R) == 4 ? kW : 1][3][kDense ? kTile : 1];
   // the atoms of the A tile and of each wavefront's B tile (work partition only)
   __shared__ int part_atom[kPart ? (kW + 1) * kTile : 1];
   const long long total = item_off[b.natoms];
+  // Persistent launch: the items in `queues` ranges, one per XCD (blocks go
+  // to the XCDs in turn), so that the blocks of an XCD share its L2's lines;
+  // a block whose range is empty goes on with the next.
+  int steal = 0;
+  auto draw = [&]() {
+    for (; steal < queues; ++steal) {
+      const int q = (blockIdx.x + steal) % queues;
+      const long long at =
+          total * q / queues + static_cast<long long>(atomicAdd(work_counter + q * kCounterStride, 1ull));
+      if (at < total * (q + 1) / queues) return at;
+    }
+    return total;
+  };
   long long k_item = blockIdx.x;
   if (work_counter) {
-    if (threadIdx.x == 0) next_item = static_cast<long long>(atomicAdd(work_counter, 1ull));
+    if (threadIdx.x == 0) next_item = draw();
     __syncthreads();
     k_item = next_item;
   }
   for (; k_item < total;) {
-  const long long item = total - 1 - k_item;
-  int lo = 0, hi = b.natoms;
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (item_off[mid] <= item) lo = mid;
-    else hi = mid;
-  }
-  const int i = lo;
-  const int P = static_cast<int>(item - item_off[i]);
+  const int2 it = items[k_item];
+  const int i = __builtin_amdgcn_readfirstlane(it.x), P = __builtin_amdgcn_readfirstlane(it.y);
   const int s = b.sys[i];
   const SysGeom g = b.geom[s];
   const SysParam p = b.par[s];
@@ -1161,7 +1335,12 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   const long long L0 = offset[i];
   const int m = static_cast<int>(offset[i + 1] - L0);
   const int nb = (m + kTile - 1) / kTile;
-  const double cut2 = p.cut3 * p.cut3;
+  // lists by storage order: pairs within the rounding band of the cutoff are
+  // taken first and decided by triple_in_range
+  const bool by_rank = kDense && rank_owned(b, g);
+  const double cut2x = p.cut3 * p.cut3;
+  const double cut2 = by_rank ? cut2x * (1.0 + kBand) : cut2x;
+  const double cut2_lo = cut2x * (1.0 - kBand);
   const R alp = R(p.alp) + R(2);
   const R alp2 = R(2) * alp;
   const R malp6 = -alp / R(6);
@@ -1169,17 +1348,24 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   const R ns9 = -R(p.s9);
   const R cutr = R(p.cut3), width = R(p.width3);
   const R4<R>* __restrict__ prow = pair + g.c6_begin;  // n x n pair records of the system
+  auto pair_power = [&](R C) { return alp14 ? R(pow_m8_3(double(C))) : pow_pos(C, malp6); };
   // wavefront index as a uniform value, so the tile loop, the ring counters
   // and the LDS tile addresses live in scalar registers
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = wave_lane();
 
   // A tile (shared)
+  const bool jat_valid = P * kTile + l < m;
   double* __restrict__ accB = accBw[w];
   int jat = -1;  // atom of a-slot l
   double ax, ay, az;  // FP64 vector of a-slot l (every wavefront holds them)
   if (w == 0) {
     jat = load_tile(&tileA, slots, L0, P * kTile + l, m, l, ax, ay, az);
     if (kPart) part_atom[l] = jat < 0 ? i : jat;
+    if (kDense && sizeof(R) == 4) {
+      avec[0][l] = ax;
+      avec[1][l] = ay;
+      avec[2][l] = az;
+    }
     for (int c = 0; c < kNAcc; ++c) accA[c * kTile + l] = 0.0;
   } else {
     load_tile<R>(nullptr, slots, L0, P * kTile + l, m, l, ax, ay, az);
@@ -1193,6 +1379,9 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   // in a step of its own after the loop over the others.
   const double cut2_half = l < kTile / 2 ? cut2 : -1.0;
   const int arank = tileA.rank[l];
+  const int* __restrict__ sys_order = b.order + g.atom_begin;
+  // a-slots in the band
+  const bool a_band = by_rank && __ballot(jat_valid && ax * ax + ay * ay + az * az > cut2_lo) != 0ull;
   const int ri = b.rank[i];  // storage index of atom i: slots with this rank are its images
   const unsigned lane_tag = static_cast<unsigned>(l) * 257u;  // entry word a | a << 8
   const long long irow = kPairs ? static_cast<long long>(ri) * n : 0;  // pairs {i, s} in pair3s
@@ -1209,16 +1398,136 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
     int katl = -1;                          // atom of b-slot l of this tile
     double vbx = 0.0, vby = 0.0, vbz = 0.0;  // and its FP64 vector
     if (!diag) katl = load_tile(&TB, slots, L0, Q * kTile + l, m, l, vbx, vby, vbz);
+    // FP64 vectors of the tile's slots in LDS (dense instantiations): FP64
+    // tiles hold them (1e30 past the list's end), FP32 tiles have bvec beside
+    if (kDense && sizeof(R) == 4 && !diag) {
+      bvec[w][0][l] = vbx;
+      bvec[w][1][l] = vby;
+      bvec[w][2][l] = vbz;
+    }
+    auto b_vector = [&](int k, double& x, double& y, double& z) {
+      if (sizeof(R) == 4) {
+        const double(*v)[kDense ? kTile : 1] = diag ? avec : bvec[w];
+        x = v[0][k];
+        y = v[1][k];
+        z = v[2][k];
+      } else {
+        const R4<R> v = TB.g0[k];
+        x = double(v.x);
+        y = double(v.y);
+        z = double(v.z);
+      }
+    };
     if (kPart && !diag) part_atom[(w + 1) * kTile + l] = katl < 0 ? i : katl;
     const int* __restrict__ batom = part_atom + (kPart && !diag ? (w + 1) * kTile : 0);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
     const int s0 = diag ? 1 : 0, s1 = diag ? kTile / 2 : kTile - 1;
-    int st = s0, head = 0, tail = 0;
     // the b-slot of lane l at step st is (l + st) mod 64: its vector rotates
     // by one lane after every step
     double bx = vbx, by = vby, bz = vbz;
-    if (diag) {
+    // the pairs of tiles with a slot in the band are all decided exactly
+    const bool exact = by_rank && (a_band || (!diag && __ballot(katl >= 0 && vbx * vbx + vby * vby + vbz * vbz >
+                                                                                 cut2_lo) != 0ull));
+    if (kDense && !diag && !exact) {
+      // the share of a sample of the slot pairs that pass the distance test
+      int near = 0;
+      const R4<R> c0 = tileA.g0[l];
+#pragma unroll
+      for (int k = 0; k < kSample; ++k) {
+        const R4<R> b0 = TB.g0[(l + 8 * k + 5) & (kTile - 1)];
+        const R dx = b0.x - c0.x, dy = b0.y - c0.y, dz = b0.z - c0.z;
+        // (a slot past the list's end has r^2 = 0)
+        near += __popcll(__ballot(dx * dx + dy * dy + dz * dz <= cutr * cutr && c0.w > R(0) && b0.w > R(0)));
+      }
+      if (near >= kDenseShare) {
+        // row 8 (l / 8) + m8 of the A tile for each group of 8 lanes
+        for (int m8 = 0; m8 < 8; ++m8) {
+          const int a = (l & ~7) + m8;
+          const R4<R> a0 = tileA.g0[a], a1 = tileA.g1[a];
+          const int ka = tileA.rank[a];
+          const R4<R>* __restrict__ arow = prow + static_cast<long long>(ka) * n;
+          const bool aself = ka == ri;
+          double sax, say, saz;
+          if (sizeof(R) == 4) {
+            sax = __shfl(ax, a, kWave);
+            say = __shfl(ay, a, kWave);
+            saz = __shfl(az, a, kWave);
+          } else {
+            sax = double(a0.x);
+            say = double(a0.y);
+            saz = double(a0.z);
+          }
+          double sGx = 0.0, sGy = 0.0, sGz = 0.0, sD = 0.0;
+          int kb = TB.rank[l];
+          R4<R> qn = arow[kb];
+          int kn = TB.rank[l ^ 8];
+#pragma unroll 1
+          for (int k = 0; k < 8; ++k) {
+            const int bl = l ^ (8 * k);
+            const R4<R> q = qn;
+            const bool both = aself && kb == ri;
+            const R4<R> b0 = TB.g0[bl], b1 = TB.g1[bl];
+            kb = kn;
+            qn = arow[kb];  // the next step's pair record
+            kn = TB.rank[l ^ ((8 * k + 16) & 63)];
+            double v0, v1, v2, x0, x1, x2;
+            b_vector(bl, x0, x1, x2);
+            const double Cd = diff_norm2(x0, x1, x2, sax, say, saz, v0, v1, v2);
+            bool ok = Cd <= cut2 && Cd >= kEps;
+            if (by_rank && ok && Cd > cut2_lo)
+              ok = triple_in_range(b.pos, i, sys_order[ka], sys_order[TB.rank[bl]], cut2x);
+            if (ok) {
+              const R C = R(Cd);
+              const TripleTerm<R> tt = triple_term<R, kGrad, kSmooth>(a0.w, b0.w, C, a1, b1, q, pair_power(C), both,
+                                                                      ns9, alp2, cutr, width);
+              ei -= double(tt.dE);
+              if (kGrad) {
+                const R fA = tt.fA, fB = tt.fB, fC = tt.fC;
+                di += double(tt.dE * (a1.z + b1.z));
+                const R cx = fC * (a0.x - b0.x), cy = fC * (a0.y - b0.y), cz = fC * (a0.z - b0.z);
+                sGx += double(fA * a0.x + cx);
+                sGy += double(fA * a0.y + cy);
+                sGz += double(fA * a0.z + cz);
+                sD += double(tt.dE * (a1.w + q.y));
+                atomicAdd(&accb[0 * kTile + bl], double(fB * b0.x - cx));
+                atomicAdd(&accb[1 * kTile + bl], double(fB * b0.y - cy));
+                atomicAdd(&accb[2 * kTile + bl], double(fB * b0.z - cz));
+                atomicAdd(&accb[3 * kTile + bl], double(tt.dE * (b1.w + q.z)));
+              }
+            }
+          }
+          if (kGrad) {
+            double sv[4] = {sGx, sGy, sGz, sD};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              sv[c] += dpp_move<0xB1>(sv[c]);   // quad_perm [1,0,3,2]
+              sv[c] += dpp_move<0x4E>(sv[c]);   // quad_perm [2,3,0,1]
+              sv[c] += dpp_move<0x141>(sv[c]);  // row_half_mirror
+            }
+            if ((l & 7) < 4) {
+              const double x = (l & 3) == 0 ? sv[0] : (l & 3) == 1 ? sv[1] : (l & 3) == 2 ? sv[2] : sv[3];
+              atomicAdd(&accA[(l & 3) * kTile + a], x);
+            }
+          }
+        }
+        if (kGrad) {  // flush the b-slots of this tile pair
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+          __builtin_amdgcn_wave_barrier();
+          const double Gx = accB[0 * kTile + l], Gy = accB[1 * kTile + l], Gz = accB[2 * kTile + l];
+          const double D = accB[3 * kTile + l];
+          for (int c = 0; c < kAcc; ++c) accB[c * kTile + l] = 0.0;
+          b_vector(l, vbx, vby, vbz);
+          flush_tile(Gx, Gy, Gz, D, vbx, vby, vbz, Q * kTile + l < m ? TB.rank[l] : -1, TB.rank[l],
+                     slot_acc + g.atom_begin, gi, sg);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        continue;
+      }
+    }
+    int st = s0, head = 0, tail = 0;
+    if (!kDense && diag) {
       bx = wave_rotate1(ax);
       by = wave_rotate1(ay);
       bz = wave_rotate1(az);
@@ -1228,11 +1537,19 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
     auto test_step = [&](double thr) {
       const int bl = (l + st) & (kTile - 1);
       double v0, v1, v2;
+      if (kDense) b_vector(bl, bx, by, bz);
       const double Cd = diff_norm2(bx, by, bz, ax, ay, az, v0, v1, v2);
       const bool in_c = Cd <= thr, in_e = Cd >= kEps;
       bool ok = in_c & in_e;
       // the ballot from the two compares' lane masks (no VALU copy of ok)
       unsigned long long bal = __builtin_amdgcn_ballot_w64(in_c) & __builtin_amdgcn_ballot_w64(in_e);
+      if (by_rank) {
+        const bool band = ok && (exact || Cd > cut2_lo);
+        if (__builtin_amdgcn_ballot_w64(band) != 0ull) {
+          if (band) ok = triple_in_range(b.pos, i, sys_order[arank], sys_order[TB.rank[bl]], cut2x);
+          bal = __ballot(ok);
+        }
+      }
       if (kPart) {  // atm.f90:709: the triple belongs to the pair (i, larger partner)
         ok = ok && owns_pair(p, i - g.atom_begin, max(part_atom[l], batom[bl]) - g.atom_begin);
         bal = __ballot(ok);
@@ -1247,9 +1564,11 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
         q_ring[pos & (kQueue - 1)] = e;
       }
       tail += __popcll(bal);
-      bx = wave_rotate1(bx);
-      by = wave_rotate1(by);
-      bz = wave_rotate1(bz);
+      if (!kDense) {
+        bx = wave_rotate1(bx);
+        by = wave_rotate1(by);
+        bz = wave_rotate1(bz);
+      }
       ++st;
     };
     // the steps before the half step of a diagonal tile, or all 64
@@ -1274,50 +1593,11 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
           const R C = e.C;
           const R4<R> a0 = tileA.g0[a], a1 = tileA.g1[a];
           const R4<R> b0 = TB.g0[bb], b1 = TB.g1[bb];
-          const R A = a0.w, B = b0.w;
-          const R AB = A * B;
-          const R S = AB * C;
-          const R ir1 = rsqrt_fast(S);
-          const R ir2 = ir1 * ir1;
-          const R ir5 = ir2 * ir2 * ir1;
-          const R dab = A - B;
-          const R t1 = (A + B) - C, t2 = dab + C, t3 = C - dab;
-          const R u = t2 * t3, v = t1 * t3, wv = t1 * t2;
-          const R Pt = t1 * u;
-          const R core = R(0.375) * Pt + S;
-          const R ang = ir5 * core;
-          const R pp = a1.x * b1.x * (q.w * (alp14 ? R(pow_m8_3(double(C))) : pow_pos(C, malp6)));
-          const R fd = rcp_fast(R(1) + R(6) * pp);
-          R c9 = ns9 * a1.y * b1.y * q.x;
-          if (ka == ri && kb == ri) c9 *= R(4.0 / 3.0);  // j == k == i
-          const R cwf = c9 * fd;
-          R dE = ang * cwf;
-          R sw = R(1), swa = R(1), dswa = R(0), swb = R(1), dswb = R(0), swc = R(1), dswc = R(0);
-          if (kSmooth) {
-            const R ra = d_sqrt(A), rb = d_sqrt(B), rc = d_sqrt(C);
-            smooth_cutoff(ra, cutr, width, swa, dswa);
-            smooth_cutoff(rb, cutr, width, swb, dswb);
-            smooth_cutoff(rc, cutr, width, swc, dswc);
-            dswa /= ra; dswb /= rb; dswc /= rc;
-            sw = swa * swb * swc;
-          }
+          const TripleTerm<R> tt = triple_term<R, kGrad, kSmooth>(a0.w, b0.w, C, a1, b1, q, pair_power(C),
+                                                                  ka == ri && kb == ri, ns9, alp2, cutr, width);
+          const R dE = tt.dE;
           if (kGrad) {
-            const R Y = alp2 * pp * fd;
-            const R sgm = u + v + wv;
-            const R K1 = R(-1.875) * Pt - R(3) * S + Y * core;
-            const R hA = R(0.75) * A * (sgm - R(2) * wv) + K1;
-            const R hB = R(0.75) * B * (sgm - R(2) * v) + K1;
-            const R hC = R(0.75) * C * (sgm - R(2) * u) + K1;
-            const R om = -cwf * ir5 * ir2;  // 1/X = (S/X) / S
-            R fA = om * hA * (B * C);
-            R fB = om * hB * (A * C);
-            R fC = om * hC * AB;
-            if (kSmooth) {  // atm.f90:754-790, switching-function terms
-              fA = sw * fA - dE * dswa * swb * swc;
-              fB = sw * fB - dE * dswb * swa * swc;
-              fC = sw * fC - dE * dswc * swa * swb;
-              dE *= sw;
-            }
+            const R fA = tt.fA, fB = tt.fB, fC = tt.fC;
             di += double(dE * (a1.z + b1.z));
             // dE/dv_a = fA v_a + fC (v_a - v_b), dE/dv_b = fB v_b + fC (v_b - v_a)
             const R cx = fC * (a0.x - b0.x), cy = fC * (a0.y - b0.y), cz = fC * (a0.z - b0.z);
@@ -1329,8 +1609,6 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
             atomicAdd(&accb[1 * kTile + bb], double(fB * b0.y - cy));
             atomicAdd(&accb[2 * kTile + bb], double(fB * b0.z - cz));
             atomicAdd(&accb[3 * kTile + bb], double(dE * (b1.w + q.z)));
-          } else if (kSmooth) {
-            dE *= sw;
           }
           ei -= double(dE);
           if (kPairs) {
@@ -1350,6 +1628,10 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
       const double Gx = accB[0 * kTile + l], Gy = accB[1 * kTile + l], Gz = accB[2 * kTile + l];
       const double D = accB[3 * kTile + l];
       for (int c = 0; c < kAcc; ++c) accB[c * kTile + l] = 0.0;
+      if (kDense) {
+        b_vector(l, vbx, vby, vbz);
+        katl = Q * kTile + l < m ? TB.rank[l] : -1;
+      }
       flush_tile(Gx, Gy, Gz, D, vbx, vby, vbz, katl, TB.rank[l], slot_acc + g.atom_begin, gi, sg);
     }
     if (kPairs && !diag) {  // pair {i, b-slot atom}
@@ -1378,7 +1660,7 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   }
   if (!work_counter) break;
   // block_add ended with a barrier: every wavefront is done with the LDS
-  if (threadIdx.x == 0) next_item = static_cast<long long>(atomicAdd(work_counter, 1ull));
+  if (threadIdx.x == 0) next_item = draw();
   __syncthreads();
   k_item = next_item;
   __syncthreads();  // next_item is rewritten only after every thread has read it
@@ -1388,29 +1670,31 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
 // At least three wavefronts per SIMD in FP64 (the E+grad instantiation
 // otherwise takes 184 VGPRs, two wavefronts, and runs 14 % slower; with the
 // hint it takes 168 and spills a few dozen bytes) and four in FP32.
-template <typename R, bool kGrad, bool kSmooth, int kW, bool kPart>
+template <typename R, bool kGrad, bool kSmooth, int kW, bool kPart, bool kDense>
 __global__ __launch_bounds__(kW * kWave) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void atm_kernel(DevBatch b, const long long* __restrict__ item_off,
+                                                         const int2* __restrict__ items,
                                                          const long long* __restrict__ offset,
                                                          const Slot<R>* __restrict__ slots,
                                                          const R4<R>* __restrict__ pair, double* __restrict__ e_atom,
                                                          double* __restrict__ dedcn, double* __restrict__ grad,
                                                          double* __restrict__ sig_atom,
                                                          double4* __restrict__ slot_acc,
-                                                         unsigned long long* __restrict__ work_counter) {
-  atm_body<R, kGrad, kSmooth, kW, false, kPart>(b, item_off, offset, slots, pair, e_atom, dedcn, grad, sig_atom,
-                                                slot_acc, work_counter, nullptr);
+                                                         unsigned long long* __restrict__ work_counter, int queues) {
+  atm_body<R, kGrad, kSmooth, kW, false, kPart, kDense>(b, item_off, items, offset, slots, pair, e_atom, dedcn, grad, sig_atom,
+                                                slot_acc, work_counter, nullptr, queues);
 }
 
 // Pairwise three-body energies (one block of four wavefronts per work item).
 template <typename R, bool kSmooth>
 __global__ __launch_bounds__(4 * kWave) void atm_pairs_kernel(DevBatch b, const long long* __restrict__ item_off,
+                                                              const int2* __restrict__ items,
                                                               const long long* __restrict__ offset,
                                                               const Slot<R>* __restrict__ slots,
                                                               const R4<R>* __restrict__ pair,
                                                               double* __restrict__ e_atom,
                                                               double* __restrict__ pair3s) {
-  atm_body<R, false, kSmooth, 4, true>(b, item_off, offset, slots, pair, e_atom, nullptr, nullptr, nullptr, nullptr,
-                                       nullptr, pair3s);
+  atm_body<R, false, kSmooth, 4, true>(b, item_off, items, offset, slots, pair, e_atom, nullptr, nullptr, nullptr, nullptr,
+                                       nullptr, pair3s, 1);
 }
 
 // Pair energies in atom order from the storage-order sums of atm_pairs_kernel:
@@ -3022,8 +3306,19 @@ void launch_atm_count(const DevBatch& b, const void* pair, bool mixed, long long
                        count, (const long long*)nullptr, (Slot<double>*)nullptr, 0LL, acc);
 }
 
-void launch_list_scan(const long long* count, int n, long long* offset, long long* item_off, hipStream_t st) {
-  hipLaunchKernelGGL(list_scan_kernel, dim3(1), dim3(kScanBlock), 0, st, count, n, offset, item_off);
+bool list_scan_writes_items(const DevBatch& b) { return b.natoms <= kScanBlock; }
+
+void launch_list_scan(const DevBatch& b, const long long* count, long long* offset, long long* item_off, int2* items,
+                      hipStream_t st) {
+  if (items && !list_scan_writes_items(b)) throw std::invalid_argument("item table of a list scan of several blocks");
+  hipLaunchKernelGGL(list_scan_kernel, dim3(blocks_for(b.natoms, kScanBlock)), dim3(kScanBlock), 0, st, b, count, offset,
+                     item_off, items);
+}
+
+void launch_item_table(const DevBatch& b, const long long* count, const long long* item_off, int2* items,
+                       hipStream_t st) {
+  hipLaunchKernelGGL(item_table_kernel, dim3(blocks_for(b.ntiles, kWavesPerBlock)), dim3(kBlock), 0, st, b, count,
+                     item_off, items);
 }
 
 void launch_atm_fill(const DevBatch& b, const void* pair, bool mixed, const long long* offset, void* slots,
@@ -3074,10 +3369,10 @@ void launch_atm_guard(const DevBatch& b, const long long* offset, long long capa
 
 
 namespace {
-__global__ void zero_counter(unsigned long long* c) { *c = 0ull; }
+__global__ void zero_counter(unsigned long long* c) { c[threadIdx.x * kCounterStride] = 0ull; }
 
-template <typename R, bool kGrad, bool kSmooth, int kW, bool kPart>
-void launch_atm_t(const DevBatch& b, const long long* item_off, long long max_items, const long long* offset,
+template <typename R, bool kGrad, bool kSmooth, int kW, bool kPart, bool kDense>
+void launch_atm_t(const DevBatch& b, const long long* item_off, const int2* items, long long max_items, const long long* offset,
                   const void* slots, const DevWork& w, const AtmShape& shape, unsigned long long* counter,
                   hipStream_t st) {
   long long grid = max_items;
@@ -3085,71 +3380,70 @@ void launch_atm_t(const DevBatch& b, const long long* item_off, long long max_it
   if (shape.blocks_per_cu > 0) {
     grid = std::min<long long>(max_items, static_cast<long long>(shape.blocks_per_cu) * shape.num_cus);
     wc = counter;
-    hipLaunchKernelGGL(zero_counter, dim3(1), dim3(1), 0, st, wc);
+    hipLaunchKernelGGL(zero_counter, dim3(1), dim3(kXcd), 0, st, wc);
   }
   // w.atm_acc was cleared by the list count pass of this evaluation
   if (kGrad && !w.atm_acc) throw std::invalid_argument("three-body gradient launch without its per-atom sums");
-  hipLaunchKernelGGL((atm_kernel<R, kGrad, kSmooth, kW, kPart>), dim3(static_cast<unsigned>(grid)), dim3(kW * kWave), 0,
-                     st, b, item_off, offset, static_cast<const Slot<R>*>(slots),
-                     static_cast<const R4<R>*>(w.pair), w.e_atom, w.dedcn, w.grad, w.sig_atom, w.atm_acc, wc);
+  hipLaunchKernelGGL((atm_kernel<R, kGrad, kSmooth, kW, kPart, kDense>), dim3(static_cast<unsigned>(grid)), dim3(kW * kWave), 0,
+                     st, b, item_off, items, offset, static_cast<const Slot<R>*>(slots),
+                     static_cast<const R4<R>*>(w.pair), w.e_atom, w.dedcn, w.grad, w.sig_atom, w.atm_acc, wc,
+                     b.xcd_queues ? kXcd : 1);
   if (kGrad)
     hipLaunchKernelGGL(atm_acc_kernel, dim3(blocks_for(b.natoms, kBlock)), dim3(kBlock), 0, st, b, w.atm_acc,
                        w.grad, w.dedcn);
 }
 
-template <int kW, bool kPart>
-void launch_atm_w(const DevBatch& b, bool mixed, bool grad, bool smooth, const long long* item_off,
+template <int kW, bool kPart, bool kDense>
+void launch_atm_w(const DevBatch& b, bool mixed, bool grad, bool smooth, const long long* item_off, const int2* items,
                   long long max_items, const long long* offset, const void* slots, const DevWork& w,
                   const AtmShape& shape, unsigned long long* counter, hipStream_t st) {
-  using L = void (*)(const DevBatch&, const long long*, long long, const long long*, const void*, const DevWork&,
+  using L = void (*)(const DevBatch&, const long long*, const int2*, long long, const long long*, const void*, const DevWork&,
                      const AtmShape&, unsigned long long*, hipStream_t);
   static const L table[8] = {
-      launch_atm_t<double, false, false, kW, kPart>, launch_atm_t<double, false, true, kW, kPart>,
-      launch_atm_t<double, true, false, kW, kPart>,  launch_atm_t<double, true, true, kW, kPart>,
-      launch_atm_t<float, false, false, kW, kPart>,  launch_atm_t<float, false, true, kW, kPart>,
-      launch_atm_t<float, true, false, kW, kPart>,   launch_atm_t<float, true, true, kW, kPart>};
-  table[(mixed ? 4 : 0) + (grad ? 2 : 0) + (smooth ? 1 : 0)](b, item_off, max_items, offset, slots, w, shape,
+      launch_atm_t<double, false, false, kW, kPart, kDense>, launch_atm_t<double, false, true, kW, kPart, kDense>,
+      launch_atm_t<double, true, false, kW, kPart, kDense>,  launch_atm_t<double, true, true, kW, kPart, kDense>,
+      launch_atm_t<float, false, false, kW, kPart, kDense>,  launch_atm_t<float, false, true, kW, kPart, kDense>,
+      launch_atm_t<float, true, false, kW, kPart, kDense>,   launch_atm_t<float, true, true, kW, kPart, kDense>};
+  table[(mixed ? 4 : 0) + (grad ? 2 : 0) + (smooth ? 1 : 0)](b, item_off, items, max_items, offset, slots, w, shape,
                                                              counter, st);
 }
 }  // namespace
 
 void launch_atm(const DevBatch& b, bool mixed, bool grad, bool smooth, bool partitioned, const AtmShape& shape,
-                const long long* item_off, long long max_items, const long long* offset, const void* slots,
-                const DevWork& w, unsigned long long* counter, hipStream_t st) {
+                const long long* item_off, const int2* items, long long max_items, const long long* offset,
+                const void* slots, const DevWork& w, unsigned long long* counter, hipStream_t st) {
   if (max_items <= 0) return;
   if (shape.blocks_per_cu > 0 && (!counter || shape.num_cus <= 0))
     throw std::invalid_argument("persistent three-body launch needs a work counter and the CU count");
-  if (partitioned)  // its own instantiation (four wavefronts), so the others keep their registers
-    launch_atm_w<4, true>(b, mixed, grad, smooth, item_off, max_items, offset, slots, w, shape, counter, st);
-  else if (shape.waves == 2)
-    launch_atm_w<2, false>(b, mixed, grad, smooth, item_off, max_items, offset, slots, w, shape, counter, st);
-  else if (shape.waves == 4)
-    launch_atm_w<4, false>(b, mixed, grad, smooth, item_off, max_items, offset, slots, w, shape, counter, st);
-  else if (shape.waves == 1)
-    launch_atm_w<1, false>(b, mixed, grad, smooth, item_off, max_items, offset, slots, w, shape, counter, st);
-  else
-    throw std::invalid_argument("three-body launch: wavefronts per block must be 1, 2 or 4");
+  using L = decltype(&launch_atm_w<4, true, false>);
+  L launch = nullptr;
+  if (partitioned) launch = launch_atm_w<4, true, false>;  // its own instantiation (four wavefronts)
+  else if (shape.waves == 2) launch = b.rank_own ? launch_atm_w<2, false, true> : launch_atm_w<2, false, false>;
+  else if (shape.waves == 4) launch = b.rank_own ? launch_atm_w<4, false, true> : launch_atm_w<4, false, false>;
+  else if (shape.waves == 1) launch = b.rank_own ? launch_atm_w<1, false, true> : launch_atm_w<1, false, false>;
+  else throw std::invalid_argument("three-body launch: wavefronts per block must be 1, 2 or 4");
+  launch(b, mixed, grad, smooth, item_off, items, max_items, offset, slots, w, shape, counter, st);
 }
 
 namespace {
 template <typename R, bool kSmooth>
-void launch_atm_pairs_t(const DevBatch& b, const long long* item_off, long long max_items, const long long* offset,
+void launch_atm_pairs_t(const DevBatch& b, const long long* item_off, const int2* items, long long max_items, const long long* offset,
                         const void* slots, const DevWork& w, double* pair3s, hipStream_t st) {
   hipLaunchKernelGGL((atm_pairs_kernel<R, kSmooth>), dim3(static_cast<unsigned>(max_items)), dim3(4 * kWave), 0, st,
-                     b, item_off, offset, static_cast<const Slot<R>*>(slots), static_cast<const R4<R>*>(w.pair),
+                     b, item_off, items, offset, static_cast<const Slot<R>*>(slots), static_cast<const R4<R>*>(w.pair),
                      w.e_atom, pair3s);
 }
 }  // namespace
 
-void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, long long max_items,
-                      const long long* offset, const void* slots, const DevWork& w, double* pair3s, hipStream_t st) {
+void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, const int2* items,
+                      long long max_items, const long long* offset, const void* slots, const DevWork& w, double* pair3s, hipStream_t st) {
   if (max_items <= 0) return;
   if (mixed) {
-    if (smooth) launch_atm_pairs_t<float, true>(b, item_off, max_items, offset, slots, w, pair3s, st);
-    else launch_atm_pairs_t<float, false>(b, item_off, max_items, offset, slots, w, pair3s, st);
+    if (smooth) launch_atm_pairs_t<float, true>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
+    else launch_atm_pairs_t<float, false>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
   } else {
-    if (smooth) launch_atm_pairs_t<double, true>(b, item_off, max_items, offset, slots, w, pair3s, st);
-    else launch_atm_pairs_t<double, false>(b, item_off, max_items, offset, slots, w, pair3s, st);
+    if (smooth) launch_atm_pairs_t<double, true>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
+    else launch_atm_pairs_t<double, false>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
   }
 }
 

@@ -37,6 +37,8 @@ struct DevBatch {
   const int* order;     // [N] atom at position atom_begin + r of that order
   const double4* posr;  // [N] positions in that order, posr[x] = pos[order[x]] (refreshed with pos)
   int ntiles;
+  int xcd_queues;       // persistent three-body launch: a work queue per XCD
+  int rank_own;         // large molecules: three-body lists by storage order (energy evaluations)
   const int2* tiles;    // [ntiles] first position and count of each 64-position tile of that order
   const double4* tbox;  // [2 ntiles] lower and upper corner of each tile's positions (refreshed with pos)
 };
@@ -87,7 +89,19 @@ void launch_atm_count(const DevBatch& b, const void* pair, bool mixed, long long
                       hipStream_t stream);
 // offset[0..n] and item_off[0..n]: exclusive scans of the list sizes and of
 // their 64-slot tile counts (one block).
-void launch_list_scan(const long long* count, int n, long long* offset, long long* item_off, hipStream_t stream);
+// items (batches small enough for it, else null): the item table is written
+// by the same launch
+bool list_scan_writes_items(const DevBatch& b);
+void launch_list_scan(const DevBatch& b, const long long* count, long long* offset, long long* item_off, int2* items,
+                      hipStream_t stream);
+// items[0 .. item_off[natoms]): the work items in the order the three-body
+// kernels take them (nothing when item_off[natoms] is 0)
+void launch_item_table(const DevBatch& b, const long long* count, const long long* item_off, int2* items,
+                       hipStream_t stream);
+// work counters of a persistent three-body launch: one per XCD, each in a
+// cache line of its own
+constexpr int kXcd = 8;
+constexpr int kCounterStride = 16;
 // Writes nothing when the lists hold more than `capacity` slots.
 void launch_atm_fill(const DevBatch& b, const void* pair, bool mixed, const long long* offset, void* slots,
                      long long capacity, hipStream_t stream);
@@ -114,12 +128,13 @@ struct AtmShape {
 // memory for the work counter of a persistent shape.
 // partitioned: some system has a work partition of more than one part.
 void launch_atm(const DevBatch& b, bool mixed, bool grad, bool smooth, bool partitioned, const AtmShape& shape,
-                const long long* item_off, long long max_items, const long long* offset, const void* slots,
-                const DevWork& w, unsigned long long* counter, hipStream_t stream);
+                const long long* item_off, const int2* items, long long max_items, const long long* offset,
+                const void* slots,                const DevWork& w, unsigned long long* counter, hipStream_t stream);
 // Pairwise three-body energies: adds the pair sums of every triple term to
 // pair3s (per system an n x n block in storage order, zeroed by the caller);
 // pair3_finalize writes the symmetric pair energies in atom order to out.
-void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, long long max_items,
+void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, const int2* items,
+                      long long max_items,
                       const long long* offset, const void* slots, const DevWork& w, double* pair3s,
                       hipStream_t stream);
 void launch_pair3_finalize(const DevBatch& b, const double* pair3s, double* out, hipStream_t stream);
