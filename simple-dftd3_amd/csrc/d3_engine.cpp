@@ -198,15 +198,18 @@ class KernelTimer {
 struct Prepared {
   DevBatch db{};
   long long pair_total = 0;    // sum over systems of n^2
-  bool any_atm = false;        // some system has s9 != 0
+  bool any_atm = false;        // some system has a three-body term by lists
+  PairSumItems ps;             // work items of the systems with a three-body term by pair sums
+  long long tri_total = 0;     // sum over these systems of n^2
   bool smooth = false;         // some three-body system has a nonzero width3
   bool periodic_atm = false;   // some three-body system has lattice images
   bool partitioned = false;    // some system evaluates one part of a work partition
-  bool any_cull = false;       // some system is a molecule of more than 8 tiles
+  bool any_cull = false;       // some system with lists is a molecule of more than 8 tiles
   bool fixed_order = false;    // one system of at most 8 tiles: storage order = atom order, no sort
-  long long slot_bound = 0;    // sum over three-body systems of (il + 1) * images
-  long long atm_atoms = 0;     // atoms of the systems with a three-body term
+  long long slot_bound = 0;    // sum over the systems with lists of (il + 1) * images
+  long long atm_atoms = 0;     // atoms of these systems
   long long item_bound = 0;    // work items of those bounds
+  long long shape_items = 0;   // work items if every three-body system had lists (launch shape of a plan)
   bool ewald = false;          // the (single) system sums its two-body term in reciprocal space
   EwaldBatch eb{};             // its vectors, expansion and species chunks (nk = 0: no two-body term)
   bool spme = false;           // ... on a particle mesh instead of the vectors
@@ -354,9 +357,30 @@ AtmShape per_call_shape(bool mixed, bool periodic, long long items) {
   return a;
 }
 
+// Three-body term by pair sums instead of lists: whole molecules (no lattice
+// images, no work partition) up to this many atoms.  The pair sums visit every
+// triple of atoms, three times with the gradient, at a third to a fifth of the
+// lists' cost a visit; the lists only the triples within the cutoff, so they
+// win once most atoms of a molecule are out of each other's range.  Ellipsoids
+// 1:1:2 at 0.1 atoms per cubic Angstrom, whole evaluations, ms, pair sums /
+// lists; FP64 gradient: 500 atoms 0.23 / 0.44, 1,000 0.64 / 1.08, 2,000 2.57 /
+// 3.91, 3,000 6.67 / 7.75, 4,000 12.6 / 12.5; FP64 energy: 1,000 0.31 / 0.78,
+// 4,000 4.83 / 8.56; mixed gradient: 1,000 0.62 / 0.91, 1,500 1.40 / 1.56,
+// 2,000 2.6 / 2.6 (a sphere 3.1 / 3.0); mixed energy: 4,000 4.75 / 4.88.
+constexpr int kPairSumAtoms = 3500, kPairSumAtomsMixedGrad = 1750;
+int pair_sum_atoms(bool mixed, bool grad) { return mixed && grad ? kPairSumAtomsMixedGrad : kPairSumAtoms; }
+// Tiles of 16 positions a side from this many tile pairs of the batch on, else
+// of 8, which spread a small batch over more wavefronts (gradient, ms, tiles of
+// 8 / 16: 300 atoms 0.155 / 0.158, 500 0.232 / 0.238, 600 (741 tile pairs)
+// 0.321 / 0.291, 1,000 0.80 / 0.67).
+constexpr size_t kPairSumWide = 650;
+// Above this many bytes of records and sums the allocation-free entry point
+// keeps the lists, so that the batches that fit its work area stay the same.
+constexpr long long kPairSumArenaBytes = 16LL << 20;
+
 struct Workspace {
   DeviceBuffer meta, pos, rank, order, sort_tmp, cn, gw, dgw, pair, e_atom, dedcn, grad, sig, atm_acc, cnt, off,
-      item_off, items, slots, gw_rank, sp_rank, pos_rank, tbox, counts, counter, flag, pair3s, hbuf, e_out, ew_tab, ew_c6l, ew_lc6l, ew_ldc6l, ew_part,
+      item_off, items, slots, tri, psum, band, gw_rank, sp_rank, pos_rank, tbox, counts, counter, flag, pair3s, hbuf, e_out, ew_tab, ew_c6l, ew_lc6l, ew_ldc6l, ew_part,
       ew_phi, ew_f, ew_s, sp_base, sp_theta, sp_dtheta, sp_q, sp_qh, sp_th, sp_k, sp_dm, sp_dmir;
   // batched real <-> half-complex 3D transforms of the particle mesh (one per
   // species), kept while the mesh and the species count stay the same
@@ -393,7 +417,7 @@ struct Workspace {
   Arena* arena = nullptr;
   std::vector<DeviceBuffer*> buffers() {
     return {&meta, &pos, &rank, &order, &sort_tmp, &cn, &gw, &dgw, &pair, &e_atom, &dedcn, &grad, &sig, &atm_acc, &cnt, &off,
-            &item_off, &items, &slots, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
+            &item_off, &items, &slots, &tri, &psum, &band, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
             &e_out, &ew_tab, &ew_c6l, &ew_lc6l, &ew_ldc6l, &ew_part, &ew_phi, &ew_f, &ew_s, &sp_base, &sp_theta,
             &sp_dtheta, &sp_q, &sp_qh, &sp_th, &sp_k, &sp_dm, &sp_dmir};
   }
@@ -417,8 +441,9 @@ struct Workspace {
   // Host planning of a batch: species of the batch, per-species tables,
   // lattice images per system and cutoff, pair-block offsets; one metadata
   // upload (stream-ordered).
+  // Molecules of up to max_pair_sum atoms take the pair-sum route.
   Prepared upload(const std::vector<SystemDesc>& systems, const int* numbers, hipStream_t stream,
-                  const int* ghost_host);
+                  const int* ghost_host, int max_pair_sum);
   // Packs the positions; with order_atoms also (re)computes the spatial order
   // of the atoms (the storage order of pair records and three-body lists).
   void pack(const Prepared& pb, const double* positions_dev, hipStream_t stream, bool order_atoms) {
@@ -455,7 +480,7 @@ void Engine::set_kernel_timing(bool enable) {
 std::pair<double, long long> Engine::kernel_time(const std::string& name) const { return ws_->timer.get(name); }
 
 Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* numbers, hipStream_t stream,
-                           const int* ghost_host) {
+                           const int* ghost_host, int max_pair_sum) {
   Prepared pb;
   const int nsys = static_cast<int>(systems.size());
   int natoms = 0;
@@ -536,6 +561,16 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   std::vector<double4> img;
   std::vector<int2> tiles;  // 64-position tiles of every system's spatial order
   long long pair_total = 0, slot_bound = 0, item_bound = 0, atm_atoms = 0;
+  std::vector<int> ps_systems;  // pair-sum route
+  auto pair_sum_route = [&](const SystemDesc& sd) {
+    return !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2]) && sd.nparts == 1 && sd.natoms <= max_pair_sum;
+  };
+  if (arena) {
+    long long bytes = 0;
+    for (const auto& sd : systems)
+      if (pair_sum_route(sd)) bytes += static_cast<long long>(sd.natoms) * sd.natoms * (sizeof(double4) + sizeof(double2));
+    if (bytes > kPairSumArenaBytes) max_pair_sum = 0;
+  }
   bool any_atm = false, smooth = false, periodic_atm = false;
   for (int k = 0, a = 0; k < nsys; ++k) {
     const SystemDesc& sd = systems[k];
@@ -571,21 +606,54 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
     // tile culling for molecules of more than 8 tiles (in smaller ones every
     // tile is usually within the cutoffs and the box tests only cost)
     g.cull = !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2]) && sd.natoms > 8 * kTile;
-    pb.any_cull = pb.any_cull || g.cull;
+    g.tri_begin = -1;
     for (int t = 0; t * kTile < sd.natoms; ++t)
       tiles.push_back(make_int2(g.atom_begin + t * kTile, std::min(kTile, sd.natoms - t * kTile)));
     if (std::fabs(sd.param.s9) >= kEps) {
+      const bool ps = pair_sum_route(sd);
+      long long items = 0;
+      for (long long il = 0; il < sd.natoms; ++il) items += ((il + 1) * g.img3_count + kTile - 1) / kTile;
+      pb.shape_items += items;
+      if (ps) {
+        g.tri_begin = pb.tri_total;
+        pb.tri_total += static_cast<long long>(sd.natoms) * sd.natoms;
+        ps_systems.push_back(k);
+        continue;
+      }
       any_atm = true;
+      pb.any_cull = pb.any_cull || g.cull;
       smooth |= sd.param.width3 > 0.0;
       if (g.img3_count > 1) periodic_atm = true;
       atm_atoms += sd.natoms;
+      item_bound += items;
       // slot j <= i of atom i: at most (il + 1) images each
       for (long long il = 0; il < sd.natoms; ++il) {
         const long long m = (il + 1) * g.img3_count;
         slot_bound += m;
-        item_bound += (m + kTile - 1) / kTile;
       }
     }
+  }
+  // Tile pairs of the pair-sum route, the largest systems (the longest sums) first
+  std::vector<int2> ps_items;
+  if (!ps_systems.empty()) {
+    std::stable_sort(ps_systems.begin(), ps_systems.end(),
+                     [&](int x, int y) { return systems[x].natoms > systems[y].natoms; });
+    auto tile_pairs = [&](int side) {
+      size_t c = 0;
+      for (int k : ps_systems) {
+        const size_t t = (systems[k].natoms + side - 1) / side;
+        c += t * (t + 1) / 2;
+      }
+      return c;
+    };
+    pb.ps.side = tile_pairs(16) >= kPairSumWide ? 16 : 8;
+    ps_items.reserve(tile_pairs(pb.ps.side));
+    for (int k : ps_systems) {
+      const int t = (systems[k].natoms + pb.ps.side - 1) / pb.ps.side;
+      for (int I = 0; I < t; ++I)
+        for (int J = I; J < t; ++J) ps_items.push_back(make_int2(k, I | J << 16));
+    }
+    pb.ps.count = static_cast<int>(ps_items.size());
   }
   // Reciprocal-space set-up (damping.f90:306-385, ewald.f90:113-121).
   ReciprocalTiles rt;
@@ -662,7 +730,7 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
                o_geom = stage(sb, geom),
                o_par = stage(sb, par), o_img = stage(sb, img), o_rcov = stage(sb, rcov), o_r4 = stage(sb, r4r2),
                o_nref = stage(sb, nref), o_refcn = stage(sb, refcn), o_c6r = stage(sb, c6ref),
-               o_rvdw = stage(sb, rvdw), o_ptiles = stage(sb, tiles);
+               o_rvdw = stage(sb, rvdw), o_ptiles = stage(sb, tiles), o_ps = stage(sb, ps_items);
   // a single small system (the usual call of the drop-in interface) keeps
   // the atom order as its storage order: in one or a few tiles the spatial
   // order gains nothing and its sort would run with every evaluation
@@ -713,6 +781,8 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   db.ntiles = static_cast<int>(tiles.size());
   db.tiles = reinterpret_cast<const int2*>(dmeta + o_ptiles);
   db.tbox = tbox.as<double4>(2 * tiles.size());
+  db.band = pb.ps.count > 0 ? band.as<int>(nsys) : nullptr;
+  pb.ps.items = reinterpret_cast<const int2*>(dmeta + o_ps);
   pb.pair_total = pair_total;
   pb.any_atm = any_atm;
   pb.smooth = smooth;
@@ -802,6 +872,8 @@ DevWork Workspace::work(const Prepared& pb, bool mixed, bool grad, const BatchOu
   w.atm_acc = grad && pb.any_atm ? atm_acc.as<double4>(natoms) : nullptr;
   w.gwr = gw_rank.as<double>(size_t(natoms) * 2 * db.mref);
   w.spr = sp_rank.as<int>(natoms);
+  w.tri = pb.ps.count > 0 ? tri.as<double4>(pb.tri_total) : nullptr;
+  w.psum = grad && pb.ps.count > 0 ? psum.as<double2>(pb.tri_total) : nullptr;
   return w;
 }
 
@@ -832,7 +904,7 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
   const DevWork w = work(pb, mixed, grad, out, debug);
   timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, stream); });
   timed("weights", stream, [&] { launch_weights(db, w.cn, w.gw, w.dgw, stream); });
-  timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, stream); });
+  timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, w.tri, stream); });
   timed("disp2", stream, [&] { launch_disp2(db, mixed, grad, w, nullptr, stream); });
   if (pb.ewald && pb.spme) {
     // fourier/spme.f90:78-328, term by term of the expansion
@@ -932,6 +1004,7 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
     timed("atm", stream,
           [&] { launch_atm(db, mixed, grad, smooth, pb.partitioned, sh, io, it, max_items, o, s, w, wc, stream); });
   }
+  if (pb.ps.count > 0) timed("atm", stream, [&] { launch_atm_pairsum(db, mixed, grad, pb.ps, w, nullptr, stream); });
   if (grad) timed("cn_chain", stream, [&] { launch_cn_chain(db, mixed, w, stream); });
   timed("reduce", stream, [&] { launch_reduce(db, w, out.energy, grad ? out.sigma : nullptr, stream); });
   hip_check(hipGetLastError(), "kernel launch");
@@ -942,8 +1015,9 @@ void Engine::run(const std::vector<SystemDesc>& systems, const int* numbers, con
                  RunStats* stats, const int* ghost_host) {
   if (systems.empty()) return;
   Workspace& m = *ws_;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host);
   const bool grad = out.gradient || out.sigma;
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host,
+                               stats ? 0 : pair_sum_atoms(precision == kMixed, grad));
   m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, out, debug, stats, -1, 0, kPerCallShape,
              stream);
   if (m.timer.enabled) m.timer.collect();
@@ -974,8 +1048,8 @@ void run_noalloc(const std::vector<SystemDesc>& systems, const int* numbers, con
   }
   Workspace& m = st->ws;
   m.reset_arena();
-  const Prepared pb = m.upload(systems, numbers, stream, nullptr);
   const bool grad = out.gradient || out.sigma;
+  const Prepared pb = m.upload(systems, numbers, stream, nullptr, pair_sum_atoms(precision == kMixed, grad));
   // the gradient is summed in the work area and copied out at the end, so
   // that a batch rejected for its size leaves every output untouched
   BatchOutput inner = out;
@@ -997,7 +1071,7 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
     if (sd.lowrank && sd.periodic[0] && sd.periodic[1] && sd.periodic[2])
       throw Error("Pairwise analysis is only available for the real space summation");
   Workspace& m = *ws_;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host);
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, kPairSumAtoms);
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   const bool mixed = precision == kMixed;
@@ -1005,11 +1079,11 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
   const DevWork w = m.work(pb, mixed, false, BatchOutput{}, nullptr);
   m.timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, stream); });
   m.timed("weights", stream, [&] { launch_weights(db, w.cn, w.gw, nullptr, stream); });
-  m.timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, nullptr, w.gwr, w.spr, w.pair, stream); });
+  m.timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, nullptr, w.gwr, w.spr, w.pair, w.tri, stream); });
   m.timed("disp2", stream, [&] { launch_disp2(db, mixed, false, w, pair2, stream); });
   const size_t bytes = sizeof(double) * static_cast<size_t>(pb.pair_total);
   if (!pb.any_atm) {
-    hip_check(hipMemsetAsync(pair3, 0, bytes, stream), "hipMemsetAsync");
+    if (pb.tri_total < pb.pair_total) hip_check(hipMemsetAsync(pair3, 0, bytes, stream), "hipMemsetAsync");
   } else {
     double* S = m.pair3s.as<double>(static_cast<size_t>(pb.pair_total));
     hip_check(hipMemsetAsync(S, 0, bytes, stream), "hipMemsetAsync");
@@ -1030,6 +1104,7 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
       launch_pair3_finalize(db, S, pair3, stream);
     });
   }
+  if (pb.ps.count > 0) m.timed("atm", stream, [&] { launch_atm_pairsum(db, mixed, false, pb.ps, w, pair3, stream); });
   hip_check(hipGetLastError(), "kernel launch");
   if (m.timer.enabled) m.timer.collect();
 }
@@ -1043,7 +1118,7 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
   for (const auto& sd : systems)  // disp.f90:113-119
     if (sd.lowrank) throw Error("Hessian is only available for the real space summation");
   Workspace& m = *ws_;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host);
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, 0);
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   double* e = energy ? energy : m.e_out.as<double>(static_cast<size_t>(db.nsys));
@@ -1089,7 +1164,7 @@ void Engine::count_terms(const std::vector<SystemDesc>& systems, const int* numb
   std::vector<SystemDesc> sys = systems;
   for (auto& s : sys)
     if (std::fabs(s.param.s9) < kEps) s.param.s9 = 1.0;  // triples are counted whatever s9 is
-  const Prepared pb = m.upload(sys, numbers, stream, nullptr);
+  const Prepared pb = m.upload(sys, numbers, stream, nullptr, 0);
   m.pack(pb, positions_dev, stream, true);
   const int natoms = pb.db.natoms;
   unsigned long long* dc = m.counts.as<unsigned long long>(size_t(pb.db.nsys) * 3);
@@ -1145,7 +1220,7 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
     State& s = *st_;
     s.mixed = precision == kMixed;
     s.grad = grad;
-    s.pb = s.ws.upload(systems, numbers_host, stream, ghost_host);
+    s.pb = s.ws.upload(systems, numbers_host, stream, ghost_host, pair_sum_atoms(s.mixed, grad));
     s.shape.num_cus = device_cu_count();
     const int natoms = s.pb.db.natoms;
     hip_check(hipMemsetAsync(s.ws.flag.as<int>(1), 0, sizeof(int), stream), "hipMemsetAsync");
@@ -1158,7 +1233,7 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
         const DevWork w = s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
         launch_cn(s.pb.db, s.mixed, w.cn, stream);
         launch_weights(s.pb.db, w.cn, w.gw, w.dgw, stream);
-        launch_pair(s.pb.db, s.mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, stream);
+        launch_pair(s.pb.db, s.mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, w.tri, stream);
         s.ws.list_offsets(s.pb.db, w.pair, s.mixed, w.atm_acc, nullptr, stream);
         long long total = 0;
         hip_check(hipMemcpyAsync(&total, s.ws.off.as<long long>(natoms + 1) + natoms, sizeof total,
@@ -1169,14 +1244,16 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
       }
       s.capacity = cap;
       s.max_items = std::min(s.pb.item_bound, cap / kTile + natoms);
-      const AtmShape a = per_call_shape(s.mixed, s.pb.periodic_atm, s.max_items);  // until set_shape or autotune
-      s.shape.waves = a.waves;
-      s.shape.blocks_per_cu = a.blocks_per_cu;
       // size every buffer now, so that an evaluation allocates nothing
       (void)s.ws.slots.get(std::max<long long>(cap, 1) * slot_record_bytes(s.mixed));
       (void)s.ws.items.as<int2>(std::max<long long>(s.max_items, 1));
       (void)s.ws.counter.as<unsigned long long>(kXcd * kCounterStride);
     }
+    // until set_shape or autotune
+    const AtmShape a =
+        per_call_shape(s.mixed, s.pb.periodic_atm, s.pb.any_atm ? s.max_items : s.pb.shape_items);
+    s.shape.waves = a.waves;
+    s.shape.blocks_per_cu = a.blocks_per_cu;
     (void)s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
     hip_check(hipStreamSynchronize(stream), "plan sync");
   } catch (...) {

@@ -18,6 +18,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "d3_hess3.hpp"
 #include "d3_kernels.hpp"
@@ -328,6 +329,7 @@ __global__ void weights_kernel(DevBatch b, const double* __restrict__ cn, double
                                double* __restrict__ dgw) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= b.natoms) return;
+  if (b.band && i < b.nsys) b.band[i] = 0;  // (a system has at least one atom)
   const double wf = 4.0, wf2 = 2.0 * wf;
   const int s = b.sp[i];
   const int nr = b.nref[s];
@@ -385,11 +387,15 @@ __global__ __launch_bounds__(kBlock) void rank_weights_kernel(DevBatch b, const 
   spr[x] = b.sp[j] | (b.ghost && b.ghost[j] ? kGhostBit : 0);
 }
 
+__device__ __forceinline__ double pow_m8_3(double x);
+
+// With tri the block also writes the row of the three-body records of a
+// system of the pair-sum route (see atm_pairsum_kernel).
 template <typename R>
 __global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* __restrict__ gw,
                                                       const double* __restrict__ dgw,
                                                       const double* __restrict__ gwr, const int* __restrict__ spr,
-                                                      R4<R>* __restrict__ pair) {
+                                                      R4<R>* __restrict__ pair, double4* __restrict__ tri) {
   const int i = blockIdx.x;
   const int s = b.sys[i];
   const SysGeom g = b.geom[s];
@@ -425,7 +431,12 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* 
   for (int t = threadIdx.x; t < b.nsp; t += blockDim.x) r0p_s[t] = pow(kRs9 * b.rvdw[t * b.nsp + spi], alp3);
   __syncthreads();
   const bool gi_ghost = b.ghost && b.ghost[i];
-  R4<R>* row = pair + g.c6_begin + static_cast<long long>(b.rank[i]) * n;
+  const int ri = b.rank[i];
+  R4<R>* row = pair + g.c6_begin + static_cast<long long>(ri) * n;
+  double4* tri_row = g.tri_begin >= 0 ? tri + g.tri_begin + static_cast<long long>(ri) * n : nullptr;
+  const double4 xi = b.pos[i];
+  const double cut3 = b.par[s].cut3, width3 = b.par[s].width3;
+  const bool alp14 = b.par[s].alp == 14.0;
   const long long nat = b.natoms;
   for (int jr = threadIdx.x; jr < n; jr += blockDim.x) {
     const int x = g.atom_begin + jr;  // position of partner j in the spatial order
@@ -444,7 +455,27 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* 
       }
     }
     const double ic = cc > 0.0 ? 1.0 / cc : 0.0;
-    row[jr] = make_r4<R>(R(sqrt(cc)), R(di * ic), R(dj * ic), R(r0p_s[spj]));
+    const double sc6 = sqrt(cc);
+    row[jr] = make_r4<R>(R(sc6), R(di * ic), R(dj * ic), R(r0p_s[spj]));
+    if (!tri_row) continue;
+    double4 t = make_double4(1.0, 0.0, 0.0, 0.0);  // no pair: no term
+    double v0, v1, v2;
+    const double r2 = atm_vec(b.posr[x], make_double4(0.0, 0.0, 0.0, 0.0), xi, v0, v1, v2);
+    const double cut2 = cut3 * cut3;
+    if (jr != ri && r2 <= cut2 * (1.0 + kBand) && r2 >= kEps && cc >= kEps) {
+      const double r1 = sqrt(r2);
+      double sw, dswdr;
+      smooth_cutoff(r1, cut3, width3, sw, dswdr);
+      t.x = r2;
+      t.y = sw * sc6 / (r2 * r1);
+      t.z = r0p_s[spj] * (alp14 ? pow_m8_3(r2) : pow(r2, -0.5 * alp3));
+      t.w = t.y / r2;
+      if (r2 > cut2 * (1.0 - kBand)) {  // see atm_pairsum_kernel
+        t.z = -t.z;
+        b.band[s] = 1;
+      }
+    }
+    tri_row[jr] = t;
   }
 }
 
@@ -790,7 +821,7 @@ __global__ __launch_bounds__(kBlock) void atm_list_kernel(DevBatch b, const R4<R
   const int s = b.sys[i];
   const SysGeom g = b.geom[s];
   const SysParam p = b.par[s];
-  if (fabs(p.s9) < kEps) {
+  if (fabs(p.s9) < kEps || g.tri_begin >= 0) {  // (the pair-sum route has no lists)
     if (!kFill && lane == 0) count[i] = 0;
     return;
   }
@@ -1695,6 +1726,268 @@ __global__ __launch_bounds__(4 * kWave) void atm_pairs_kernel(DevBatch b, const 
                                                               double* __restrict__ pair3s) {
   atm_body<R, false, kSmooth, 4, true>(b, item_off, items, offset, slots, pair, e_atom, nullptr, nullptr, nullptr, nullptr,
                                        nullptr, pair3s, 1);
+}
+
+// ------------------------------------------- three-body term by pair sums
+// Systems without lattice images (rule: pair_sum_route in the engine).  In
+// such a system every pair of atoms has one distance, so all that a triple
+// needs of a pair can be tabulated per pair (pair_kernel):
+//   A = r^2, h = sqrt(C6) sw / r^3, g = (r0/r)^((alp+2)/3), k = h / A
+// (h = g = k = 0, A = 1 where there is no pair), and with
+//   X_abc = h_ac h_bc + 3/8 (A^2 - (B - C)^2) (B + C - A) / A  k_ac k_bc,
+//   f_abc = 1 / (1 + 6 g_ab g_ac g_bc),   A = r_ab^2, B = r_ac^2, C = r_bc^2,
+// the energy of a triple is s9 h_ab X_abc f_abc (atm.f90:736-748).  A lane
+// owns pairs (a, b) and sums over all c: the sum S of X f is the pair's share
+// in its triples' energies (dE/dCN), the sums S, Y, Z give dE/dA_ab
+//   A dE/dA = s9 h [ (alp/6 - 3/2) S + 3/8 Y / A - alp/6 Z ],   alp + 2 -> alp,
+//   Y = sum f k_ac k_bc (A (2 A t3 - m) - m t3), m = A^2 - (B-C)^2, t3 = B+C-A,
+//   Z = sum X f^2,
+// and gradient and virial follow from the pair sums at O(n^2) cost
+// (pair_sum_finish_kernel).  A triple is visited from each of its three
+// pairs, but a visit is 21 FP64 operations and one reciprocal, without a
+// distance test, a power, a gather or an LDS atomic; the energy alone visits
+// c > b only.  Everything is FP64 whatever the precision: FP32 issues at the
+// same rate.
+//
+// A block owns a tile of (8 kT)^2 pairs, kT x kT per lane; its wavefronts
+// take the chunks of kC atoms c in turn, and their sums meet in the LDS.  The
+// records (c, a-tile) and (c, b-tile) of a chunk are 4 KB, staged by each
+// wavefront for itself one chunk ahead; atoms c beyond the cutoff of all of
+// a-tile or all of b-tile are skipped (their h are all zero).  The lists of
+// such systems spent most of their time on the distance tests, the LDS
+// atomics and the gathers: 1,501-atom molecule, FP64 energy, whole call 1.82
+// -> 0.64 ms; planned batch of 1,024 molecules, FP64 gradient, 5.75 -> 3.30;
+// 200-atom molecule from host arrays 0.24 -> 0.17; the kernel is bound by
+// FP64 issue.
+//
+// Which triples the reference takes is decided from the atom of the largest
+// index (atm.f90:706-724), so a distance within kBand of the cutoff can fall
+// on either side by the rounding of another atom's vectors: such pairs have
+// g < 0, and in a system that has one (band[s]) triple_in_range decides every
+// triple with such a pair.
+enum PairSumMode { kPsEnergy, kPsGrad, kPsPairs };
+template <int kMode, int kT>
+__global__ __launch_bounds__(kBlock) void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items,
+                                                             const double4* __restrict__ tri,
+                                                             double2* __restrict__ psum, double* __restrict__ e_atom,
+                                                             double* __restrict__ pair3) {
+  constexpr int kSide = 8 * kT, kRecs = 2 * kSide, kC = 128 / kRecs, kOwn = kT * kT;
+  constexpr int kSums = kMode == kPsGrad ? 3 : 1;
+  __shared__ double2 stage[kWavesPerBlock][2][2 * kRecs * kC];
+  __shared__ double red[kWavesPerBlock];
+  const int2 it = items[blockIdx.x];
+  const int s = it.x, I = it.y & 0xffff, J = it.y >> 16;
+  const SysGeom g = b.geom[s];
+  const SysParam& p = b.par[s];
+  const int n = g.natoms;
+  const double4* __restrict__ rec = tri + g.tri_begin;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = wave_lane();
+  const int la = l >> 3, lb = l & 7;
+  double A[kOwn], c38[kOwn], G6[kOwn], h[kOwn], S[kOwn], Y[kOwn], Z[kOwn];
+  bool any = false, own_band[kOwn];
+#pragma unroll
+  for (int o = 0; o < kOwn; ++o) {
+    const int a = I * kSide + la + 8 * (o / kT), bb = J * kSide + lb + 8 * (o % kT);
+    const double4 q = a < n && bb < n ? rec[static_cast<long long>(a) * n + bb] : make_double4(1.0, 0.0, 0.0, 0.0);
+    A[o] = q.x;
+    c38[o] = 0.375 / q.x;
+    h[o] = kMode == kPsEnergy && a >= bb ? 0.0 : q.y;
+    G6[o] = 6.0 * fabs(q.z);
+    own_band[o] = q.z < 0.0;
+    any |= h[o] != 0.0;
+    S[o] = Y[o] = Z[o] = 0.0;
+  }
+  // (the wavefronts of the block hold the same pairs)
+  const bool live = __ballot(any) != 0ull;
+  if (kMode == kPsEnergy && !live) return;
+
+  const int nchunks = (n + kC - 1) / kC;
+  int ch = (kMode == kPsEnergy ? J * (kSide / kC) : 0) + w;
+  // 16-byte unit u = 64 k + l of a chunk: atom c = u / (2 kRecs), record
+  // r = u / 2 mod kRecs (a-tile, then b-tile), half u mod 2
+  double2 pre[4];
+  const int r = (l >> 1) & (kRecs - 1);
+  const int rx = min(r < kSide ? I * kSide + r : J * kSide + r - kSide, n - 1);
+  auto fetch = [&](int chunk) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int c = chunk * kC + (kWave * k + l) / (2 * kRecs);
+      pre[k] = make_double2(0.0, 0.0);
+      if (c < n) pre[k] = reinterpret_cast<const double2*>(rec + static_cast<long long>(c) * n + rx)[l & 1];
+    }
+  };
+  auto run = [&](auto banded) {
+    constexpr bool kBanded = decltype(banded)::value;
+    int buf = 0;
+    if (ch < nchunks) fetch(ch);
+    for (; ch < nchunks; ch += kWavesPerBlock, buf ^= 1) {
+      unsigned act = 0;  // atoms of the chunk with a term
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        stage[w][buf][kWave * k + l] = pre[k];
+        const unsigned long long nz = __ballot((l & 1) == 0 && pre[k].y != 0.0);
+        if (kT == 2) {
+          if ((nz & 0xffffffffull) && (nz >> 32)) act |= 1u << k;
+        } else {
+          if ((nz & 0xffffull) && (nz & 0xffff0000ull)) act |= 1u << (2 * k);
+          if (((nz >> 32) & 0xffffull) && (nz >> 48)) act |= 2u << (2 * k);
+        }
+      }
+      const int chunk = ch;
+      if (ch + kWavesPerBlock < nchunks) fetch(ch + kWavesPerBlock);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      // energy: c > b within the b-tile
+      const bool within = kMode == kPsEnergy && chunk * kC < (J + 1) * kSide;
+      while (act) {
+        const int c = __builtin_ctz(act);
+        act &= act - 1;
+        const double4* row = reinterpret_cast<const double4*>(stage[w][buf]) + c * kRecs;
+        double4 ra[kT], rb[kT];
+#pragma unroll
+        for (int u = 0; u < kT; ++u) {
+          ra[u] = row[la + 8 * u];
+          rb[u] = row[kSide + lb + 8 * u];
+        }
+#pragma unroll
+        for (int o = 0; o < kOwn; ++o) {
+          double4 x = ra[o / kT], y = rb[o % kT];
+          bool ok = true;
+          if (kMode == kPsEnergy && within) ok = chunk * kC + c > J * kSide + lb + 8 * (o % kT);
+          if (kBanded) {
+            if ((x.z < 0.0 || y.z < 0.0 || own_band[o]) && ok && h[o] != 0.0 && x.y != 0.0 && y.y != 0.0) {
+              const int* __restrict__ ord = b.order + g.atom_begin;
+              ok = triple_in_range(b.pos, ord[I * kSide + la + 8 * (o / kT)], ord[J * kSide + lb + 8 * (o % kT)],
+                                   ord[chunk * kC + c], p.cut3 * p.cut3);
+            }
+            x.z = fabs(x.z);
+            y.z = fabs(y.z);
+          }
+          double hh = x.y * y.y, kk = x.w * y.w;
+          if (kBanded || (kMode == kPsEnergy && within)) {
+            hh = ok ? hh : 0.0;
+            kk = ok ? kk : 0.0;
+          }
+          const double f = rcp_fast(fma(G6[o], x.z * y.z, 1.0));
+          const double d = x.x - y.x, t3 = (x.x + y.x) - A[o];
+          const double m = fma(-d, d, A[o] * A[o]);
+          const double P = m * t3;
+          const double Xf = fma(c38[o], P * kk, hh) * f;
+          S[o] += Xf;
+          if (kMode == kPsGrad) {
+            const double y1 = fma(A[o], fma(A[o] + A[o], t3, -m), -P);
+            Y[o] = fma(kk * y1, f, Y[o]);
+            Z[o] = fma(Xf, f, Z[o]);
+          }
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  if (live) {
+    if (b.band[s]) run(std::true_type{});
+    else run(std::false_type{});
+  }
+  // the wavefronts' sums: value v of pair o and lane l at sums[w][v][o][l],
+  // then wavefront o (of the first kOwn) finishes pair o of every lane
+  __syncthreads();
+  double* __restrict__ sums = reinterpret_cast<double*>(&stage[0][0][0]);
+  static_assert(sizeof stage >= sizeof(double) * kWavesPerBlock * kSums * kOwn * kWave, "sums fit the stage");
+#pragma unroll
+  for (int o = 0; o < kOwn; ++o) {
+    sums[((w * kSums + 0) * kOwn + o) * kWave + l] = S[o];
+    if (kMode == kPsGrad) {
+      sums[((w * kSums + 1) * kOwn + o) * kWave + l] = Y[o];
+      sums[((w * kSums + 2) * kOwn + o) * kWave + l] = Z[o];
+    }
+  }
+  __syncthreads();
+  double e = 0.0;
+  if (w < kOwn) {
+    double t[kSums];
+#pragma unroll
+    for (int v = 0; v < kSums; ++v) {
+      t[v] = 0.0;
+#pragma unroll
+      for (int q = 0; q < kWavesPerBlock; ++q) t[v] += sums[((q * kSums + v) * kOwn + w) * kWave + l];
+    }
+    // w is uniform: the pair's constants without an indexed register file
+    double Ao = A[0], ho = h[0];
+#pragma unroll
+    for (int o = 1; o < kOwn; ++o) {
+      Ao = w == o ? A[o] : Ao;
+      ho = w == o ? h[o] : ho;
+    }
+    const int a = I * kSide + la + 8 * (w / kT), bb = J * kSide + lb + 8 * (w % kT);
+    const double E = p.s9 * ho * t[0];  // energy of all triples of the pair
+    if (kMode == kPsEnergy) e = E;
+    if (a <= bb && bb < n) {  // (a diagonal tile holds both orders of its pairs)
+      if (kMode == kPsGrad) {
+        const double a6 = (p.alp + 2.0) / 6.0, iA = 1.0 / Ao;
+        const double F = 2.0 * p.s9 * ho * iA * ((a6 - 1.5) * t[0] + 0.375 * iA * t[kSums - 2] - a6 * t[kSums - 1]);
+        psum[g.tri_begin + static_cast<long long>(a) * n + bb] = make_double2(E, F);
+        psum[g.tri_begin + static_cast<long long>(bb) * n + a] = make_double2(E, F);
+      }
+      if (kMode == kPsPairs) {  // atm.f90:829-950: a sixth of every term on each ordered pair of its atoms
+        const long long ia = b.order[g.atom_begin + a] - g.atom_begin, ib = b.order[g.atom_begin + bb] - g.atom_begin;
+        pair3[g.c6_begin + ia * n + ib] = E / 6.0;
+        pair3[g.c6_begin + ib * n + ia] = E / 6.0;
+      }
+    }
+  }
+  if (kMode == kPsEnergy) block_add(e_atom + b.order[g.atom_begin + I * kSide], e, red);
+}
+
+// Energy, dE/dCN, gradient and virial of the pair sums {E_ab, 2 dE/dA_ab},
+// wavefront per atom of a system of the pair-sum route: each triple energy
+// is in the sums of six ordered pairs; dE/dCN_a = 1/2 sum_b E_ab
+// (dC6_ab/dCN_a)/C6_ab; the derivative of the switching function, whose
+// factor is in h, is added here.
+template <typename R>
+__global__ __launch_bounds__(kBlock) void pair_sum_finish_kernel(DevBatch b, const R4<R>* __restrict__ pair,
+                                                                 const double2* __restrict__ psum,
+                                                                 double* __restrict__ e_atom,
+                                                                 double* __restrict__ dedcn,
+                                                                 double* __restrict__ grad,
+                                                                 double* __restrict__ sig_atom) {
+  const int i = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  if (i >= b.natoms) return;
+  const int s = b.sys[i];
+  const SysGeom g = b.geom[s];
+  if (g.tri_begin < 0) return;
+  const SysParam& p = b.par[s];
+  const int n = g.natoms;
+  const long long row = static_cast<long long>(b.rank[i]) * n;
+  const double4 xi = b.pos[i];
+  const bool smooth = p.width3 > 0.0;
+  double v[11] = {0.0};
+  for (int x = wave_lane(); x < n; x += kWave) {
+    const double2 q = psum[g.tri_begin + row + x];
+    const double qi = double(pair[g.c6_begin + row + x].y);
+    const double4 xj = b.posr[g.atom_begin + x];
+    const double u0 = xi.x - xj.x, u1 = xi.y - xj.y, u2 = xi.z - xj.z;
+    double F = q.y;
+    if (smooth && q.x != 0.0) {
+      const double r1 = sqrt(u0 * u0 + u1 * u1 + u2 * u2);
+      double sw, dswdr;
+      smooth_cutoff(r1, p.cut3, p.width3, sw, dswdr);
+      if (sw > 0.0) F += q.x * dswdr / (sw * r1);
+    }
+    v[0] += q.x;
+    v[1] += q.x * qi;
+    v[2] += F * u0; v[3] += F * u1; v[4] += F * u2;
+    const double hf = 0.5 * F;
+    v[5] += hf * u0 * u0; v[6] += hf * u1 * u1; v[7] += hf * u2 * u2;
+    v[8] += hf * u0 * u1; v[9] += hf * u0 * u2; v[10] += hf * u1 * u2;
+  }
+#pragma unroll
+  for (int c = 0; c < 11; ++c) v[c] = wave_sum(v[c]);
+  if (wave_lane() == 0) {
+    e_atom[i] += v[0] / 6.0;
+    dedcn[i] += 0.5 * v[1];
+    for (int c = 0; c < 3; ++c) grad[3 * i + c] += v[2 + c];
+    for (int c = 0; c < 6; ++c) sig_atom[6 * i + c] += v[5 + c];
+  }
 }
 
 // Pair energies in atom order from the storage-order sums of atm_pairs_kernel:
@@ -3263,16 +3556,16 @@ void launch_rank_pos(const DevBatch& b, hipStream_t st) {
 }
 
 void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, double* gwr, int* spr,
-                 void* pair, hipStream_t st) {
+                 void* pair, double4* tri, hipStream_t st) {
   hipLaunchKernelGGL(rank_weights_kernel, dim3(blocks_for(b.natoms, kBlock)), dim3(kBlock), 0, st, b, gw, dgw, gwr,
                      spr);
   const size_t lds = sizeof(double) * static_cast<size_t>(b.nsp) * (2 * kMaxRef + 1);  // h, dh, r0p
   if (mixed)
     hipLaunchKernelGGL(pair_kernel<float>, dim3(b.natoms), dim3(kBlock), lds, st, b, gw, dgw, gwr, spr,
-                       static_cast<float4*>(pair));
+                       static_cast<float4*>(pair), tri);
   else
     hipLaunchKernelGGL(pair_kernel<double>, dim3(b.natoms), dim3(kBlock), lds, st, b, gw, dgw, gwr, spr,
-                       static_cast<double4*>(pair));
+                       static_cast<double4*>(pair), tri);
 }
 
 template <typename R, bool kGrad, bool kPairs>
@@ -3445,6 +3738,27 @@ void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long lon
     if (smooth) launch_atm_pairs_t<double, true>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
     else launch_atm_pairs_t<double, false>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
   }
+}
+
+void launch_atm_pairsum(const DevBatch& b, bool mixed, bool grad, const PairSumItems& t, const DevWork& w,
+                        double* pair3, hipStream_t st) {
+  if (t.count <= 0) return;
+  using K = void (*)(DevBatch, const int2*, const double4*, double2*, double*, double*);
+  const K kernel = t.side == 16 ? (pair3  ? atm_pairsum_kernel<kPsPairs, 2>
+                                   : grad ? atm_pairsum_kernel<kPsGrad, 2>
+                                          : atm_pairsum_kernel<kPsEnergy, 2>)
+                                : (pair3  ? atm_pairsum_kernel<kPsPairs, 1>
+                                   : grad ? atm_pairsum_kernel<kPsGrad, 1>
+                                          : atm_pairsum_kernel<kPsEnergy, 1>);
+  hipLaunchKernelGGL(kernel, dim3(t.count), dim3(kBlock), 0, st, b, t.items, w.tri, w.psum, w.e_atom, pair3);
+  if (!grad || pair3) return;
+  const dim3 grid(blocks_for(b.natoms, kWavesPerBlock)), blk(kBlock);
+  if (mixed)
+    hipLaunchKernelGGL(pair_sum_finish_kernel<float>, grid, blk, 0, st, b, static_cast<const float4*>(w.pair), w.psum,
+                       w.e_atom, w.dedcn, w.grad, w.sig_atom);
+  else
+    hipLaunchKernelGGL(pair_sum_finish_kernel<double>, grid, blk, 0, st, b, static_cast<const double4*>(w.pair),
+                       w.psum, w.e_atom, w.dedcn, w.grad, w.sig_atom);
 }
 
 void launch_pair3_finalize(const DevBatch& b, const double* pair3s, double* out, hipStream_t st) {

@@ -40,6 +40,7 @@ struct DevBatch {
   int xcd_queues;       // persistent three-body launch: a work queue per XCD
   int rank_own;         // large molecules: three-body lists by storage order (energy evaluations)
   const int2* tiles;    // [ntiles] first position and count of each 64-position tile of that order
+  int* band;            // [nsys] a pair of the system is within kBand of the three-body cutoff (pair-sum route)
   const double4* tbox;  // [2 ntiles] lower and upper corner of each tile's positions (refreshed with pos)
 };
 
@@ -57,6 +58,18 @@ struct DevWork {
   double4* atm_acc; // [N] three-body slot sums per atom in spatial order (G xyz, D), E+grad only
   double* gwr;      // [2 mref][N] weights and dw/dCN in spatial order (pair records)
   int* spr;         // [N] species | ghost flag in spatial order
+  // pair-sum route of the three-body term (systems with SysGeom::tri_begin
+  // >= 0): per system n x n records and, with gradient, pair sums
+  double4* tri;
+  double2* psum;
+};
+
+// Work items of the pair-sum route: {system, I | J << 16}, tiles I <= J of
+// `side` (8 or 16) positions of the system's spatial order.
+struct PairSumItems {
+  const int2* items = nullptr;
+  int count = 0;
+  int side = 16;
 };
 
 // Size in bytes of one pair record and one three-body slot.
@@ -79,7 +92,7 @@ void launch_rank_pos(const DevBatch& b, hipStream_t stream);
 // gwr [(dgw ? 2 : 1) * mref][natoms] and spr [natoms]: scratch for the
 // weights in spatial order.
 void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, double* gwr, int* spr,
-                 void* pair, hipStream_t stream);
+                 void* pair, double4* tri, hipStream_t stream);
 // pair2 (energy only, may be null): per system an n x n block (offset
 // c6_begin, atom order) of pairwise two-body energies.
 void launch_disp2(const DevBatch& b, bool mixed, bool grad, const DevWork& w, double* pair2, hipStream_t stream);
@@ -137,6 +150,11 @@ void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long lon
                       long long max_items,
                       const long long* offset, const void* slots, const DevWork& w, double* pair3s,
                       hipStream_t stream);
+// The three-body term of the systems of the pair-sum route: energy (and
+// gradient, dE/dCN, virial) added to the accumulators of w, or, with pair3,
+// their n x n pair energies (atom order, offset c6_begin) written to it.
+void launch_atm_pairsum(const DevBatch& b, bool mixed, bool grad, const PairSumItems& t, const DevWork& w,
+                        double* pair3, hipStream_t stream);
 void launch_pair3_finalize(const DevBatch& b, const double* pair3s, double* out, hipStream_t stream);
 // Analytic Hessian (FP64) of a batch; per system, atom order within the
 // system, offsets from c6_begin: c6, dc6, d2c6, d2c6ij and dEdcndcn n x n at
