@@ -1118,7 +1118,12 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
   for (const auto& sd : systems)  // disp.f90:113-119
     if (sd.lowrank) throw Error("Hessian is only available for the real space summation");
   Workspace& m = *ws_;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, 0);
+  // three-body term by pair sums for molecules without a switching width
+  // (the visits are the gradient's, three per triple, at any size cheaper than
+  // the lists' global atomics)
+  bool smooth = false;
+  for (const auto& sd : systems) smooth = smooth || sd.param.width3 > 0.0;
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, smooth ? 0 : kPairSumAtoms);
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   double* e = energy ? energy : m.e_out.as<double>(static_cast<size_t>(db.nsys));
@@ -1127,11 +1132,15 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
   RunStats stats;
   m.evaluate(pb, positions_dev, true, false, false, pb.smooth, out, nullptr, &stats, -1, 0, kPerCallShape, stream);
   const size_t nn = static_cast<size_t>(pb.pair_total), nm = static_cast<size_t>(natoms) * db.mref;
-  const size_t words = 3 * nm + 4 * nn + 3 * nn + natoms + 3 * nn + nn + 3 * nn;
+  const size_t ps_entries = static_cast<size_t>(pb.ps.count > 0 ? pb.tri_total : 0);
+  const size_t words = 3 * nm + 4 * nn + 3 * nn + natoms + 3 * nn + nn + 3 * nn + ps_entries * hess_pairsum_doubles();
   double* base = m.hbuf.as<double>(words);
   HessWork h{};
   h.cn = m.cn.as<double>(natoms);
-  h.gw = base;
+  h.rec = reinterpret_cast<double4*>(base);  // (first: aligned for 32-byte records)
+  h.rho = base + 4 * ps_entries;
+  h.planes = h.rho + ps_entries;
+  h.gw = base + ps_entries * hess_pairsum_doubles();
   h.gwd = h.gw + nm;
   h.gwd2 = h.gwd + nm;
   h.c6 = h.gwd2 + nm;
@@ -1150,7 +1159,7 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
   for (const auto& sd : systems) max_natoms = std::max(max_natoms, sd.natoms);
   const long long total = pb.any_atm ? stats.atm_list_entries : 0;
   m.timed("hessian", stream, [&] {
-    launch_hessian(db, h, m.off.as<long long>(natoms + 1), total > 0 ? m.slots.get(0) : nullptr, total, max_natoms,
+    launch_hessian(db, h, m.off.as<long long>(natoms + 1), total > 0 ? m.slots.get(0) : nullptr, total, pb.ps, max_natoms,
                    stream);
   });
   hip_check(hipGetLastError(), "kernel launch");

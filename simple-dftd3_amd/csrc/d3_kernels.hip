@@ -2634,6 +2634,245 @@ __global__ __launch_bounds__(kBlock) void hess3_kernel(DevBatch b, const long lo
   }
 }
 
+// ------------------------------------------ three-body Hessian by pair sums
+// Molecules of the pair-sum route (see atm_pairsum_kernel) without a switching
+// width.  The records of the pairs in atom order, row c, column a:
+// rec = {A, h, g (negative within kBand of the cutoff), 1 / A} and
+// rho = (dC6_ac / dCN_a) / C6_ac.
+__global__ __launch_bounds__(kBlock) void hess_rec_kernel(DevBatch b, const double* __restrict__ c6,
+                                                          const double* __restrict__ dc6, double4* __restrict__ rec,
+                                                          double* __restrict__ rho) {
+  const int i = blockIdx.x;
+  const int s = b.sys[i];
+  const SysGeom g = b.geom[s];
+  if (g.tri_begin < 0) return;
+  const SysParam& p = b.par[s];
+  const int n = g.natoms, c = i - g.atom_begin;
+  const double cut2 = p.cut3 * p.cut3, alp3 = (p.alp + 2.0) / 3.0;
+  const double4 xi = b.pos[i];
+  const int spi = b.sp[i];
+  for (int a = threadIdx.x; a < n; a += blockDim.x) {
+    const long long o = static_cast<long long>(c) * n + a;
+    const double c6ca = c6[g.c6_begin + o];
+    double4 t = make_double4(1.0, 0.0, 0.0, 1.0);
+    double q = 0.0, v0, v1, v2;
+    const double r2 = atm_vec(b.pos[g.atom_begin + a], make_double4(0.0, 0.0, 0.0, 0.0), xi, v0, v1, v2);
+    if (a != c && r2 <= cut2 * (1.0 + kBand) && r2 >= kEps && c6ca >= kEps) {
+      const double r0 = kRs9 * b.rvdw[b.sp[g.atom_begin + a] * b.nsp + spi];
+      t.x = r2;
+      t.y = sqrt(c6ca) / (r2 * sqrt(r2));
+      t.z = pow(r0 * r0 / r2, 0.5 * alp3);
+      if (r2 > cut2 * (1.0 - kBand)) t.z = -t.z;
+      t.w = 1.0 / r2;
+      q = dc6[g.c6_begin + static_cast<long long>(a) * n + c] / c6ca;
+    }
+    rec[g.tri_begin + o] = t;
+    rho[g.tri_begin + o] = q;
+  }
+}
+
+// A lane owns a pair (a, b) and sums over all c.  With D_X = X d/dX, X one of
+// A = r_ab^2, B = r_ac^2, C = r_bc^2, N = P / (ABC), P = (A^2 - (B-C)^2)(B+C-A),
+// G = 1 + 3/8 N, f = 1 / (1 + t), u = 1 - f, beta = (alp + 2) / 6 and
+// kappa = beta u - 3/2, the energy of a triple is E = s9 H G f, H = h h h, and
+//   D_X E = s9 H f (G kappa + D_X G),
+//   D_X D_Y E = s9 H f (G (kappa^2 - beta^2 f u) + kappa (D_X G + D_Y G) + D_X D_Y G).
+// The off-diagonal block of the pair (atm.f90:38-429 in these variables) is
+//   H_ab = -2 E_A - 4 E_AA r r^T + 4 r (E_AC r_bc)^T - 4 (E_AB r_ac) r^T
+//          + 4 E_BC r_ac r_bc^T,   r = r_ab = x_a - x_b,
+// and the diagonal blocks follow from translation, H_aa = -sum_b H_ab.  With
+// rho_ac = (dC6_ac/dCN_a)/C6_ac, d ln E / dCN_a = (rho_ab + rho_ac) / 2, so the
+// derivatives by coordination numbers are sums of the same kind.  The pair's
+// 18 values for each order go to `out` (planes of n x n: H_ab 9, d2E/dR_a dCN_b
+// 3, d2E/dCN_a dCN_b, and the pair's part of d2E/dR_a dCN_a 3, d2E/dCN_a^2,
+// dE/dCN_a), which hess3_finish_kernel sums over b: no atomics, where the list
+// kernel adds about 100 values a triple with global atomics (200-atom
+// molecule, energy and Hessian: 6.15 ms with it, 0.27 ms).  Each triple is
+// visited from its three pairs, about 170 FP64 operations a visit.
+constexpr int kHessPlanes = 18, kHessSums = 35;
+__global__ __launch_bounds__(kBlock) void hess3_pairsum_kernel(DevBatch b, const int2* __restrict__ items, int side,
+                                                               const double4* __restrict__ rec,
+                                                               const double* __restrict__ rho,
+                                                               const double* __restrict__ c6,
+                                                               const double* __restrict__ d2c6,
+                                                               const double* __restrict__ d2c6ij,
+                                                               double* __restrict__ out) {
+  __shared__ double red[kHessSums][kWave];
+  const int2 it = items[blockIdx.x];
+  const int s = it.x, I = it.y & 0xffff, J = it.y >> 16;
+  const SysGeom g = b.geom[s];
+  const SysParam& p = b.par[s];
+  const int n = g.natoms;
+  const double4* __restrict__ R = rec + g.tri_begin;
+  const double* __restrict__ Q = rho + g.tri_begin;
+  const double4* __restrict__ pos = b.pos + g.atom_begin;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = wave_lane();
+  const double beta = (p.alp + 2.0) / 6.0, cut2 = p.cut3 * p.cut3;
+  const bool banded = b.band[s] != 0;
+  const int subs = side / 8;
+  for (int t = 0; t < subs * subs; ++t) {
+    const int a0 = I * side + 8 * (t / subs), b0 = J * side + 8 * (t % subs);
+    if (a0 > b0 || b0 >= n) continue;  // (uniform) the other order, or past the end
+    const int a = a0 + (l >> 3), bb = b0 + (l & 7);
+    const bool own = a < bb && bb < n;
+    const int ac = min(a, n - 1), bc = min(bb, n - 1);
+    const double4 q = own ? R[static_cast<long long>(ac) * n + bc] : make_double4(1.0, 0.0, 0.0, 1.0);
+    const double4 xa = pos[ac], xb = pos[bc];
+    const double A = q.x, iA = q.w, G6 = 6.0 * fabs(q.z);
+    double v[kHessSums];
+#pragma unroll
+    for (int k = 0; k < kHessSums; ++k) v[k] = 0.0;
+    for (int k = threadIdx.x; k < kHessSums * kWave; k += kBlock) (&red[0][0])[k] = 0.0;
+    __syncthreads();
+    if (__ballot(q.y != 0.0) != 0ull) {
+      for (int c = w; c < n; c += kWavesPerBlock) {
+        const long long row = static_cast<long long>(c) * n;
+        const double4 rb = R[row + ac], rc = R[row + bc], xc = pos[c];
+        const double qa = Q[row + ac], qb = Q[row + bc];
+        double hh = rb.y * rc.y;
+        if (banded && hh * q.y != 0.0 && (rb.z < 0.0 || rc.z < 0.0 || q.z < 0.0) &&
+            !triple_in_range(b.pos, g.atom_begin + a, g.atom_begin + bb, g.atom_begin + c, cut2))
+          hh = 0.0;
+        const double B = rb.x, C = rc.x, iB = rb.w, iC = rc.w;
+        const double tt = G6 * fabs(rb.z * rc.z);
+        const double f = rcp_fast(1.0 + tt), u = tt * f;
+        const double d = B - C, e = B + C, t3 = e - A;
+        const double P = fma(-d, d, A * A) * t3;
+        const double ab = A - B, ca = A - C;
+        const double PA = fma(A, 2.0 * e - 3.0 * A, d * d);
+        const double PB = fma(B, 2.0 * (A + C) - 3.0 * B, ca * ca);
+        const double PC = fma(C, 2.0 * (A + B) - 3.0 * C, ab * ab);
+        const double iBC = iB * iC;
+        const double N = P * iBC * iA;
+        const double nA = PA * iBC, nB = PB * (iA * iC), nC = PC * (iA * iB);
+        const double nAA = fma(A * (2.0 * e - 6.0 * A), iBC, nA);
+        const double nAB = 2.0 * (ab + (B + B - C)) * iC, nAC = 2.0 * (ca + (C + C - B)) * iB, nBC = 2.0 * t3 * iA;
+        const double G = fma(0.375, N, 1.0);
+        const double GA = 0.375 * (nA - N), GB = 0.375 * (nB - N), GC = 0.375 * (nC - N);
+        const double GAA = 0.375 * (nAA - nA - nA + N), GAB = 0.375 * (nAB - nA - nB + N);
+        const double GAC = 0.375 * (nAC - nA - nC + N), GBC = 0.375 * (nBC - nB - nC + N);
+        const double kap = fma(beta, u, -1.5);
+        const double Gk = G * kap, Gk2 = G * fma(kap, kap, -beta * beta * f * u);
+        const double wt = hh * f;
+        const double E = wt * G;
+        const double DA = wt * (Gk + GA), EB = wt * (Gk + GB) * iB, EC = wt * (Gk + GC) * iC;
+        const double DAA = wt * (Gk2 + 2.0 * kap * GA + GAA);
+        const double EAB = wt * (Gk2 + kap * (GA + GB) + GAB) * iB;
+        const double EAC = wt * (Gk2 + kap * (GA + GC) + GAC) * iC;
+        const double EBC = wt * (Gk2 + kap * (GB + GC) + GBC) * iBC;
+        const double ra[3] = {xa.x - xc.x, xa.y - xc.y, xa.z - xc.z};
+        const double rv[3] = {xb.x - xc.x, xb.y - xc.y, xb.z - xc.z};
+        v[0] += E;
+        v[1] = fma(E, qa, v[1]);
+        v[2] = fma(E, qb, v[2]);
+        v[3] = fma(E * qa, qb, v[3]);
+        v[4] += DA;
+        v[5] = fma(DA, qa, v[5]);
+        v[6] = fma(DA, qb, v[6]);
+        v[7] += DAA;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double ba = EB * ra[k], cv = EC * rv[k], bx = EBC * ra[k];
+          v[8 + k] = fma(EAB, ra[k], v[8 + k]);
+          v[11 + k] = fma(EAC, rv[k], v[11 + k]);
+          v[14 + k] += ba;
+          v[17 + k] = fma(ba, qb, v[17 + k]);
+          v[20 + k] += cv;
+          v[23 + k] = fma(cv, qa, v[23 + k]);
+#pragma unroll
+          for (int m = 0; m < 3; ++m) v[26 + 3 * k + m] = fma(bx, rv[m], v[26 + 3 * k + m]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kHessSums; ++k) atomicAdd(&red[k][l], v[k]);
+    }
+    __syncthreads();
+    // wavefronts 0 and 1: the values of (a, b) and of (b, a)
+    if (w < 2 && own) {
+#pragma unroll
+      for (int k = 0; k < kHessSums; ++k) v[k] = red[k][l];
+      const double pre = p.s9 * q.y;
+      const double r[3] = {xa.x - xb.x, xa.y - xb.y, xa.z - xb.z};
+      const long long nn = static_cast<long long>(n) * n;
+      const int x = w == 0 ? a : bb, y = w == 0 ? bb : a;
+      const long long o = static_cast<long long>(x) * n + y;
+      double* __restrict__ dst = out + kHessPlanes * g.tri_begin + o;
+      const double eaa = 4.0 * iA * iA * (v[7] - v[4]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {  // entry (k of a, m of b)
+          double h = 4.0 * v[26 + 3 * k + m] - eaa * r[k] * r[m] + 4.0 * iA * (r[k] * v[11 + m] - v[8 + k] * r[m]);
+          if (k == m) h -= 2.0 * iA * v[4];
+          dst[nn * (w == 0 ? 3 * k + m : 3 * m + k)] = pre * h;
+        }
+      const double c6ab = c6[g.c6_begin + o];
+      const double qab = Q[static_cast<long long>(bb) * n + a], qba = Q[static_cast<long long>(a) * n + bb];
+      const double qx = w == 0 ? qab : qba, qy = w == 0 ? qba : qab;  // rho of x and of y in the pair
+      const double sx = w == 0 ? v[1] : v[2];                          // sum E rho_xc
+      const double dax = w == 0 ? v[5] : v[6], day = w == 0 ? v[6] : v[5];
+      const double sign = w == 0 ? 1.0 : -1.0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double rk = sign * r[k] * iA;
+        const double e1 = w == 0 ? v[14 + k] : v[20 + k], e2 = w == 0 ? v[17 + k] : v[23 + k];
+        dst[nn * (9 + k)] = pre * (rk * (qy * v[4] + day) + qy * e1 + e2);
+        dst[nn * (13 + k)] = pre * rk * (qx * v[4] + dax);
+      }
+      const double mix = c6ab >= kEps ? d2c6ij[g.c6_begin + o] / c6ab : 0.0;
+      const double sec = c6ab >= kEps ? d2c6[g.c6_begin + o] / c6ab : 0.0;
+      dst[nn * 12] = pre * (0.25 * (qab * qba * v[0] + qab * v[2] + qba * v[1] + v[3]) + 0.5 * (mix - qab * qba) * v[0]);
+      dst[nn * 16] = pre * (0.25 * qx * (qx * v[0] + sx) + 0.5 * (sec - qx * qx) * v[0]);
+      dst[nn * 17] = pre * 0.5 * qx * v[0];
+    }
+    __syncthreads();
+  }
+}
+
+// Adds the pair values of hess3_pairsum_kernel: the off-diagonal entries of
+// atom a's rows, and the sums over b to its diagonal ones (wavefront per atom).
+__global__ __launch_bounds__(kBlock) void hess3_finish_kernel(DevBatch b, const double* __restrict__ in,
+                                                              double* __restrict__ hess, double* __restrict__ dedcn,
+                                                              double* __restrict__ dEdcndr,
+                                                              double* __restrict__ dEdcndcn) {
+  const int lane = wave_lane();
+  const int i = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  if (i >= b.natoms) return;
+  const SysGeom g = b.geom[b.sys[i]];
+  if (g.tri_begin < 0) return;
+  const int n = g.natoms, a = i - g.atom_begin;
+  const long long nn = static_cast<long long>(n) * n, ndim = 3 * n;
+  const double* __restrict__ src = in + kHessPlanes * g.tri_begin + static_cast<long long>(a) * n;
+  double* __restrict__ H = hess + 9 * g.c6_begin + 3 * a * ndim;
+  double* __restrict__ D = dEdcndr + 3 * g.c6_begin + 3LL * a * n;
+  double* __restrict__ X = dEdcndcn + g.c6_begin + static_cast<long long>(a) * n;
+  double sum[14] = {0.0};
+  for (int y = lane; y < n; y += kWave) {
+    if (y == a) continue;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      const double v = src[nn * k + y];
+      H[(k / 3) * ndim + 3 * y + k % 3] += v;
+      sum[k] -= v;
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      D[static_cast<long long>(k) * n + y] += src[nn * (9 + k) + y];
+      sum[9 + k] += src[nn * (13 + k) + y];
+    }
+    X[y] += src[nn * 12 + y];
+    sum[12] += src[nn * 16 + y];
+    sum[13] += src[nn * 17 + y];
+  }
+#pragma unroll
+  for (int k = 0; k < 14; ++k) sum[k] = wave_sum(sum[k]);
+  if (lane != 0) return;
+  for (int k = 0; k < 9; ++k) H[(k / 3) * ndim + 3 * a + k % 3] += sum[k];
+  for (int k = 0; k < 3; ++k) D[static_cast<long long>(k) * n + a] += sum[9 + k];
+  X[a] += sum[12];
+  dedcn[i] += sum[13];
+}
+
 // ncoord.f90:236-306 add_coordination_number_hessian (wavefront per atom i,
 // lanes over j != i): dE/dCN times the second derivatives of the CN.
 __global__ __launch_bounds__(kBlock) void hess_cn_kernel(DevBatch b, const double* __restrict__ dedcn,
@@ -3877,8 +4116,10 @@ void launch_count_triples(const DevBatch& b, bool mixed, const long long* offset
                        static_cast<const Slot<double>*>(slots), counts);
 }
 
+size_t hess_pairsum_doubles() { return 4 + 1 + kHessPlanes; }
+
 void launch_hessian(const DevBatch& b, const HessWork& h, const long long* offset, const void* slots,
-                    long long total_slots, int max_natoms, hipStream_t st) {
+                    long long total_slots, const PairSumItems& ps, int max_natoms, hipStream_t st) {
   const dim3 wgrid(blocks_for(b.natoms, kWavesPerBlock)), blk(kBlock);
   hipLaunchKernelGGL(hess_weights_kernel, dim3(blocks_for(b.natoms, kBlock)), dim3(kBlock), 0, st, b, h.cn, h.gw,
                      h.gwd, h.gwd2);
@@ -3891,6 +4132,12 @@ void launch_hessian(const DevBatch& b, const HessWork& h, const long long* offse
     hipLaunchKernelGGL(hess3_kernel, dim3(blocks_for(total_slots, kWavesPerBlock)), dim3(kBlock), 0, st, b, offset,
                        static_cast<const Slot<double>*>(slots), h.c6, h.dc6, h.d2c6, h.d2c6ij, h.hess, h.dedcn,
                        h.dEdcndr, h.dEdcndcn);
+  if (ps.count > 0) {
+    hipLaunchKernelGGL(hess_rec_kernel, dim3(b.natoms), blk, 0, st, b, h.c6, h.dc6, h.rec, h.rho);
+    hipLaunchKernelGGL(hess3_pairsum_kernel, dim3(ps.count), blk, 0, st, b, ps.items, ps.side, h.rec, h.rho, h.c6,
+                       h.d2c6, h.d2c6ij, h.planes);
+    hipLaunchKernelGGL(hess3_finish_kernel, wgrid, blk, 0, st, b, h.planes, h.hess, h.dedcn, h.dEdcndr, h.dEdcndcn);
+  }
   hipLaunchKernelGGL(hess_cn_kernel, wgrid, blk, 0, st, b, h.dedcn, h.hess);
   const int ndim = 3 * max_natoms;
   hipLaunchKernelGGL(hess_tmp_kernel, dim3(blocks_for(ndim, kHT), blocks_for(max_natoms, kHT), b.nsys),

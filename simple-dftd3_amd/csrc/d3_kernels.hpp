@@ -167,9 +167,15 @@ struct HessWork {
   double *gw, *gwd, *gwd2;
   double *c6, *dc6, *d2c6, *d2c6ij;
   double *dr, *dedcn, *dEdcndr, *dEdcndcn, *tmp, *hess;
+  // three-body term by pair sums: n x n records and planes of pair values of
+  // each of its systems (offset SysGeom::tri_begin times the doubles of each)
+  double4* rec;
+  double *rho, *planes;
 };
+// Doubles per n x n entry of rec, rho and planes together.
+size_t hess_pairsum_doubles();
 void launch_hessian(const DevBatch& b, const HessWork& h, const long long* offset, const void* slots,
-                    long long total_slots, int max_natoms, hipStream_t stream);
+                    long long total_slots, const PairSumItems& ps, int max_natoms, hipStream_t stream);
 // Reciprocal-space two-body term of one 3D-periodic system with a low-rank
 // model (fourier/ewald.f90:47-252): one vector of each +-k pair within the
 // cutoff, in tiles {h, k, l0, count} of up to kWave vectors h b1 + k b2 +
