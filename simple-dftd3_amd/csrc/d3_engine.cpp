@@ -1099,8 +1099,19 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
       launch_item_table(db, m.cnt.as<long long>(natoms), io, it, stream);
       launch_atm_fill(db, w.pair, mixed, o, sl, total, stream);
     });
+    // images of an atom within the three-body cutoff, the least over the
+    // 3D-periodic systems with a three-body term (other cells: one)
+    double images = 1.0e9;
+    for (const auto& sd : systems) {
+      if (std::fabs(sd.param.s9) < kEps || !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2])) continue;
+      const double* a = sd.lattice;
+      const double vol = std::fabs(a[0] * (a[4] * a[8] - a[5] * a[7]) - a[1] * (a[3] * a[8] - a[5] * a[6]) +
+                                   a[2] * (a[3] * a[7] - a[4] * a[6]));
+      const bool bulk = sd.periodic[0] && sd.periodic[1] && sd.periodic[2] && vol > 0.0;
+      images = std::min(images, bulk ? 4.0 / 3.0 * M_PI * std::pow(sd.param.cut3, 3) / vol : 1.0);
+    }
     m.timed("atm", stream, [&] {
-      launch_atm_pairs(db, mixed, pb.smooth, io, it, total / kTile + natoms, o, sl, w, S, stream);
+      launch_atm_pairs(db, mixed, pb.smooth, io, it, total / kTile + natoms, o, sl, w, S, images, stream);
       launch_pair3_finalize(db, S, pair3, stream);
     });
   }

@@ -1000,11 +1000,16 @@ __global__ __launch_bounds__(kBlock) void item_table_kernel(DevBatch b, const lo
 constexpr int kQueue = 128;  // entries of the accepted-pair ring of a wavefront
 
 // Slot data of one 64-slot tile in LDS.
-template <typename R>
+template <typename R, bool kLean = false>
 struct TileSlots {
   R4<R> g0[kTile];                          // vx, vy, vz, r2
   R4<R> g1[kTile];                          // pdmp, sc6h, qi, qx
   int rank[kTile];                          // storage index of the slot's atom (0 past the list's end)
+};
+template <typename R>  // pairwise energies
+struct TileSlots<R, true> {
+  R4<R> g1[kTile];                          // pdmp, sc6h, r2, 0
+  int rank[kTile];
 };
 // Accepted slot pair (a, b) of a tile pair, written at test step st:
 // lo = a | (a + st) << 8 (b = (a + st) mod 64), C = r_jk^2.  The term phase
@@ -1028,15 +1033,19 @@ constexpr int kAcc = 4;
 // Loads slot idx of the list of atom i into position l of a tile and its
 // FP64 vector into (vx, vy, vz); returns the slot's atom (-1 past the end of
 // the list).  Without a tile (T == nullptr) only the vector is loaded.
-template <typename R>
-__device__ __forceinline__ int load_tile(TileSlots<R>* T, const Slot<R>* __restrict__ slots, long long base, int idx,
+template <typename R, bool kLean = false>
+__device__ __forceinline__ int load_tile(TileSlots<R, kLean>* T, const Slot<R>* __restrict__ slots, long long base, int idx,
                                          int m, int l, double& vx, double& vy, double& vz) {
   if (idx < m) {
     const Slot<R> s = slots[base + idx];
     vx = s.vx; vy = s.vy; vz = s.vz;
     if (T) {
-      T->g0[l] = make_r4<R>(R(s.vx), R(s.vy), R(s.vz), s.r2);
-      T->g1[l] = make_r4<R>(s.pdmp, s.sc6h, s.qi, s.qx);
+      if constexpr (kLean) {
+        T->g1[l] = make_r4<R>(s.pdmp, s.sc6h, s.r2, R(0));
+      } else {
+        T->g0[l] = make_r4<R>(R(s.vx), R(s.vy), R(s.vz), s.r2);
+        T->g1[l] = make_r4<R>(s.pdmp, s.sc6h, s.qi, s.qx);
+      }
       T->rank[l] = s.rank;
     }
     return s.atom;
@@ -1045,7 +1054,7 @@ __device__ __forceinline__ int load_tile(TileSlots<R>* T, const Slot<R>* __restr
   vx = 1e30; vy = 1e30; vz = 1e30;
   if (T) {
     const R far = sizeof(R) == 8 ? R(1e30) : R(0);
-    T->g0[l] = make_r4<R>(far, far, far, R(0));
+    if constexpr (!kLean) T->g0[l] = make_r4<R>(far, far, far, R(0));
     T->g1[l] = make_r4<R>(R(0), R(0), R(0), R(0));
     T->rank[l] = 0;
   }
@@ -1285,13 +1294,33 @@ __device__ __forceinline__ TripleTerm<R> triple_term(R A, R B, R C, const R4<R>&
 // in pair3s, an n x n block per system in storage order (rank_x, rank_y),
 // each unordered pair in one of its two orders: {j, k} at the queue entry's
 // pair-record index, {i, s} per slot s at (rank_i, rank_s) when the slot is
-// flushed.  The pair energy of (x, y) is then pair3s(rx, ry) + pair3s(ry, rx)
+// flushed.  The {j, k} terms of a tile pair are first summed in the LDS per
+// pair of atoms (the slots of an atom's images are a run of the tile), then
+// added to pair3s in rows of consecutive entries: a global atomic for every
+// term, to a random line, was most of the cost (pair energies, FP64, whole call:
+// cells of 1,000 atoms 45.8 -> 7.7 ms, of 2,000 atoms 78 -> 24 ms).  The number of cells is chosen from the images per
+// atom (launch_atm_pairs); a tile pair of more pairs of atoms adds its terms
+// directly.  One wavefront per block, so that the cells are private to it.  The pair energy of (x, y) is then pair3s(rx, ry) + pair3s(ry, rx)
 // (pair3_finalize_kernel).
 // A tile pair of which kDenseShare or more of the kSample * 64 sampled slot
 // pairs are within the cutoff is evaluated densely.
 constexpr int kSample = 8;
 constexpr int kDenseShare = kSample * kWave * 6 / 10;
 constexpr int kAccPairs = 1;  // per-slot sums of the pairwise mode: sum t
+
+// The runs of equal atoms k (k < 0: no slot) among the lanes' slots: the run
+// of this lane's slot; count receives the number of runs and run_rank[q] the
+// storage index r of run q's atom.
+__device__ __forceinline__ int tile_runs(int k, int r, int& count, int* run_rank) {
+  const int l = wave_lane();
+  const int kprev = __shfl_up(k, 1, kWave);
+  const bool head = k >= 0 && (l == 0 || kprev != k);
+  const unsigned long long heads = __ballot(head);
+  const int q = __popcll(heads & (~0ull >> (kWave - 1 - l))) - 1;
+  if (head) run_rank[q] = r;
+  count = __popcll(heads);
+  return q;
+}
 
 // Lane l receives the value of lane (l + 1) mod 64 (DPP wave_rol:1; every
 // lane has a source, so the move's old value is never used).
@@ -1316,13 +1345,14 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
                                          double* __restrict__ dedcn, double* __restrict__ grad,
                                          double* __restrict__ sig_atom, double4* __restrict__ slot_acc,
                                          unsigned long long* __restrict__ work_counter, double* __restrict__ pair3s,
-                                         int queues) {
+                                         int queues, int ncells = 0) {
   static_assert(!(kDense && (kPairs || kPart)), "dense tile pairs: energy kernels only");
   static_assert(!(kGrad && kPairs), "the pairwise mode is energy only");
+  static_assert(!kPairs || kW == 1, "the pairwise mode sums in cells of one wavefront");
   constexpr int kNAcc = kGrad ? kAcc : (kPairs ? kAccPairs : 0);
   constexpr int kAccLen = kNAcc > 0 ? kNAcc * kTile : 1;
-  __shared__ TileSlots<R> tileA;
-  __shared__ TileSlots<R> tileB[kW];
+  __shared__ TileSlots<R, kPairs> tileA;
+  __shared__ TileSlots<R, kPairs> tileB[kW];
   // per-slot sums in double (FP32 LDS atomics, ds_add_f32, measured five
   // times slower than FP64 ones in this kernel): the A tile's for the whole
   // item, each wavefront's B tile for one tile pair
@@ -1334,6 +1364,12 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   // FP64 vectors of the tiles' slots (dense FP32 instantiations)
   __shared__ double avec[3][kDense ? kTile : 1];
   __shared__ double bvec[kDense && sizeof(R) == 4 ? kW : 1][3][kDense ? kTile : 1];
+  // pairwise mode: sums per pair of atoms of a tile pair, the run of every
+  // slot of the A and B tile and the runs' storage indices
+  extern __shared__ double cells[];  // [ncells]
+  __shared__ int run_of[2][kPairs ? kTile : 1], run_rank[2][kPairs ? kTile : 1];
+  if (kPairs)
+    for (int e = threadIdx.x; e < ncells; e += kW * kWave) cells[e] = 0.0;
   // the atoms of the A tile and of each wavefront's B tile (work partition only)
   __shared__ int part_atom[kPart ? (kW + 1) * kTile : 1];
   const long long total = item_off[b.natoms];
@@ -1390,7 +1426,7 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   int jat = -1;  // atom of a-slot l
   double ax, ay, az;  // FP64 vector of a-slot l (every wavefront holds them)
   if (w == 0) {
-    jat = load_tile(&tileA, slots, L0, P * kTile + l, m, l, ax, ay, az);
+    jat = load_tile<R, kPairs>(&tileA, slots, L0, P * kTile + l, m, l, ax, ay, az);
     if (kPart) part_atom[l] = jat < 0 ? i : jat;
     if (kDense && sizeof(R) == 4) {
       avec[0][l] = ax;
@@ -1399,7 +1435,7 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
     }
     for (int c = 0; c < kNAcc; ++c) accA[c * kTile + l] = 0.0;
   } else {
-    load_tile<R>(nullptr, slots, L0, P * kTile + l, m, l, ax, ay, az);
+    load_tile<R, false>(nullptr, slots, L0, P * kTile + l, m, l, ax, ay, az);
   }
   for (int c = 0; c < kNAcc; ++c) accB[c * kTile + l] = 0.0;
   __syncthreads();
@@ -1416,6 +1452,8 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
   const int ri = b.rank[i];  // storage index of atom i: slots with this rank are its images
   const unsigned lane_tag = static_cast<unsigned>(l) * 257u;  // entry word a | a << 8
   const long long irow = kPairs ? static_cast<long long>(ri) * n : 0;  // pairs {i, s} in pair3s
+  int runs_a = 0;
+  if (kPairs) run_of[0][l] = tile_runs(jat, arank, runs_a, run_rank[0]);
 
   double ei = 0.0, di = 0.0;
   double gi[3] = {0.0, 0.0, 0.0};
@@ -1424,11 +1462,11 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
 
   for (int Q = P + w; Q < nb; Q += kW) {
     const bool diag = Q == P;
-    TileSlots<R>& TB = diag ? tileA : tileB[w];
+    TileSlots<R, kPairs>& TB = diag ? tileA : tileB[w];
     double* __restrict__ accb = diag ? accA : accB;  // b-slots of a diagonal tile are a-slots
     int katl = -1;                          // atom of b-slot l of this tile
     double vbx = 0.0, vby = 0.0, vbz = 0.0;  // and its FP64 vector
-    if (!diag) katl = load_tile(&TB, slots, L0, Q * kTile + l, m, l, vbx, vby, vbz);
+    if (!diag) katl = load_tile<R, kPairs>(&TB, slots, L0, Q * kTile + l, m, l, vbx, vby, vbz);
     // FP64 vectors of the tile's slots in LDS (dense instantiations): FP64
     // tiles hold them (1e30 past the list's end), FP32 tiles have bvec beside
     if (kDense && sizeof(R) == 4 && !diag) {
@@ -1442,7 +1480,7 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
         x = v[0][k];
         y = v[1][k];
         z = v[2][k];
-      } else {
+      } else if constexpr (!kPairs) {
         const R4<R> v = TB.g0[k];
         x = double(v.x);
         y = double(v.y);
@@ -1450,6 +1488,10 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
       }
     };
     if (kPart && !diag) part_atom[(w + 1) * kTile + l] = katl < 0 ? i : katl;
+    int runs_b = runs_a;
+    const int tb = kPairs && !diag ? 1 : 0;
+    if (kPairs && !diag) run_of[1][l] = tile_runs(katl, TB.rank[l], runs_b, run_rank[1]);
+    const bool in_cells = kPairs && runs_a * runs_b <= ncells;
     const int* __restrict__ batom = part_atom + (kPart && !diag ? (w + 1) * kTile : 0);
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
@@ -1460,7 +1502,7 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
     // the pairs of tiles with a slot in the band are all decided exactly
     const bool exact = by_rank && (a_band || (!diag && __ballot(katl >= 0 && vbx * vbx + vby * vby + vbz * vbz >
                                                                                  cut2_lo) != 0ull));
-    if (kDense && !diag && !exact) {
+    if constexpr (kDense) if (!diag && !exact) {
       // the share of a sample of the slot pairs that pass the distance test
       int near = 0;
       const R4<R> c0 = tileA.g0[l];
@@ -1622,8 +1664,15 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
               static_cast<unsigned>(kb);
           const R4<R> q = prow[rec];
           const R C = e.C;
-          const R4<R> a0 = tileA.g0[a], a1 = tileA.g1[a];
-          const R4<R> b0 = TB.g0[bb], b1 = TB.g1[bb];
+          const R4<R> a1 = tileA.g1[a], b1 = TB.g1[bb];
+          R4<R> a0{}, b0{};
+          if constexpr (kPairs) {
+            a0.w = a1.z;
+            b0.w = b1.z;
+          } else {
+            a0 = tileA.g0[a];
+            b0 = TB.g0[bb];
+          }
           const TripleTerm<R> tt = triple_term<R, kGrad, kSmooth>(a0.w, b0.w, C, a1, b1, q, pair_power(C),
                                                                   ka == ri && kb == ri, ns9, alp2, cutr, width);
           const R dE = tt.dE;
@@ -1646,7 +1695,8 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
             const double t = double(dE) * (-1.0 / 6.0);
             atomicAdd(&accA[a], t);
             atomicAdd(&accb[bb], t);
-            atomicAdd(pair3s + g.c6_begin + rec, t);
+            if (in_cells) atomicAdd(&cells[run_of[0][a] * runs_b + run_of[tb][bb]], t);
+            else atomicAdd(pair3s + g.c6_begin + rec, t);
           }
         }
       }
@@ -1664,6 +1714,15 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
         katl = Q * kTile + l < m ? TB.rank[l] : -1;
       }
       flush_tile(Gx, Gy, Gz, D, vbx, vby, vbz, katl, TB.rank[l], slot_acc + g.atom_begin, gi, sg);
+    }
+    if (in_cells) {
+      for (int e = l; e < runs_a * runs_b; e += kWave) {
+        const double t = cells[e];
+        if (t == 0.0) continue;
+        cells[e] = 0.0;
+        const int ra = e / runs_b;
+        atomicAdd(pair3s + g.c6_begin + static_cast<long long>(run_rank[0][ra]) * n + run_rank[tb][e - ra * runs_b], t);
+      }
     }
     if (kPairs && !diag) {  // pair {i, b-slot atom}
       double t[1] = {accB[l]};
@@ -1715,17 +1774,17 @@ __global__ __launch_bounds__(kW * kWave) __attribute__((amdgpu_waves_per_eu(size
                                                 slot_acc, work_counter, nullptr, queues);
 }
 
-// Pairwise three-body energies (one block of four wavefronts per work item).
+// Pairwise three-body energies (one wavefront per work item).
 template <typename R, bool kSmooth>
-__global__ __launch_bounds__(4 * kWave) void atm_pairs_kernel(DevBatch b, const long long* __restrict__ item_off,
+__global__ __launch_bounds__(kWave) void atm_pairs_kernel(DevBatch b, const long long* __restrict__ item_off,
                                                               const int2* __restrict__ items,
                                                               const long long* __restrict__ offset,
                                                               const Slot<R>* __restrict__ slots,
                                                               const R4<R>* __restrict__ pair,
                                                               double* __restrict__ e_atom,
-                                                              double* __restrict__ pair3s) {
-  atm_body<R, false, kSmooth, 4, true>(b, item_off, items, offset, slots, pair, e_atom, nullptr, nullptr, nullptr, nullptr,
-                                       nullptr, pair3s, 1);
+                                                              double* __restrict__ pair3s, int ncells) {
+  atm_body<R, false, kSmooth, 1, true>(b, item_off, items, offset, slots, pair, e_atom, nullptr, nullptr, nullptr, nullptr,
+                                       nullptr, pair3s, 1, ncells);
 }
 
 // ------------------------------------------- three-body term by pair sums
@@ -3960,22 +4019,30 @@ void launch_atm(const DevBatch& b, bool mixed, bool grad, bool smooth, bool part
 namespace {
 template <typename R, bool kSmooth>
 void launch_atm_pairs_t(const DevBatch& b, const long long* item_off, const int2* items, long long max_items, const long long* offset,
-                        const void* slots, const DevWork& w, double* pair3s, hipStream_t st) {
-  hipLaunchKernelGGL((atm_pairs_kernel<R, kSmooth>), dim3(static_cast<unsigned>(max_items)), dim3(4 * kWave), 0, st,
+                        const void* slots, const DevWork& w, double* pair3s, int cells, hipStream_t st) {
+  hipLaunchKernelGGL((atm_pairs_kernel<R, kSmooth>), dim3(static_cast<unsigned>(max_items)), dim3(kWave),
+                     sizeof(double) * cells, st,
                      b, item_off, items, offset, static_cast<const Slot<R>*>(slots), static_cast<const R4<R>*>(w.pair),
-                     w.e_atom, pair3s);
+                     w.e_atom, pair3s, cells);
 }
 }  // namespace
 
 void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, const int2* items,
-                      long long max_items, const long long* offset, const void* slots, const DevWork& w, double* pair3s, hipStream_t st) {
+                      long long max_items, const long long* offset, const void* slots, const DevWork& w, double* pair3s,
+                      double images, hipStream_t st) {
   if (max_items <= 0) return;
+  // Expected runs of a tile, 64 / images, and some for the spread over the
+  // tiles: as few cells as possible, since they set how many wavefronts a CU
+  // holds (1,000-atom cell, 3.6 images an atom: 1,536 cells and whole tiles in
+  // the LDS 12.2 ms, 640 cells 9.8, these 625 cells and lean tiles 7.7).
+  const int runs = static_cast<int>(std::min(double(kTile), kTile / std::max(images, 1.0) + 7.0));
+  const int cells = runs * runs;
   if (mixed) {
-    if (smooth) launch_atm_pairs_t<float, true>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
-    else launch_atm_pairs_t<float, false>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
+    if (smooth) launch_atm_pairs_t<float, true>(b, item_off, items, max_items, offset, slots, w, pair3s, cells, st);
+    else launch_atm_pairs_t<float, false>(b, item_off, items, max_items, offset, slots, w, pair3s, cells, st);
   } else {
-    if (smooth) launch_atm_pairs_t<double, true>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
-    else launch_atm_pairs_t<double, false>(b, item_off, items, max_items, offset, slots, w, pair3s, st);
+    if (smooth) launch_atm_pairs_t<double, true>(b, item_off, items, max_items, offset, slots, w, pair3s, cells, st);
+    else launch_atm_pairs_t<double, false>(b, item_off, items, max_items, offset, slots, w, pair3s, cells, st);
   }
 }
 

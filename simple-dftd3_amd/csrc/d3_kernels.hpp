@@ -143,12 +143,14 @@ struct AtmShape {
 void launch_atm(const DevBatch& b, bool mixed, bool grad, bool smooth, bool partitioned, const AtmShape& shape,
                 const long long* item_off, const int2* items, long long max_items, const long long* offset,
                 const void* slots,                const DevWork& w, unsigned long long* counter, hipStream_t stream);
+// images: about how many images of an atom a list holds (the least of the
+// systems), by which the LDS cells per tile pair are sized.
 // Pairwise three-body energies: adds the pair sums of every triple term to
 // pair3s (per system an n x n block in storage order, zeroed by the caller);
 // pair3_finalize writes the symmetric pair energies in atom order to out.
 void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, const int2* items,
                       long long max_items,
-                      const long long* offset, const void* slots, const DevWork& w, double* pair3s,
+                      const long long* offset, const void* slots, const DevWork& w, double* pair3s, double images,
                       hipStream_t stream);
 // The three-body term of the systems of the pair-sum route: energy (and
 // gradient, dE/dCN, virial) added to the accumulators of w, or, with pair3,
