@@ -32,7 +32,7 @@ METRIC = "E+grad pair-terms/s & molecules/s: mixed vs FP64 on GPU, |dE|<=1e-8 Eh
 OPS_PER_TRIPLE = 233    # ATM E+grad+sigma (atm.f90:733-806)
 OPS_PER_PAIR_BJ = 63    # two-body BJ E+grad+sigma (rational.f90:462-497)
 OPS_PER_TRIPLE_E = 60   # ATM energy only (atm.f90:500-621), the arithmetic of a pairwise triple term
-KERNEL_GROUPS = ("pack", "order", "cn", "weights", "c6", "disp2", "atm_list", "atm", "cn_chain", "reduce")
+KERNEL_GROUPS = ("pack", "order", "cn", "c6", "disp2", "atm_list", "atm", "cn_chain", "reduce")
 PEAK_TFLOPS = {"fp64": 78.6, "mixed": 157.3}  # MI355X vector FP64 / FP32
 # HBM bytes per launch of the mixed ATM kernel on the 2,000-atom cell,
 # measured by two rocprofv3 --pmc runs of this script (FETCH_SIZE, then

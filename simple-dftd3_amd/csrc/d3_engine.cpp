@@ -3,7 +3,7 @@
 // kernels of d3_kernels.hip on one stream.
 //
 // Order of one evaluation (disp.f90:56-185):
-//   pack -> cn -> weights -> pair (C6 and derivatives) -> disp2 ->
+//   pack -> cn and weights -> pair (C6 and derivatives) -> disp2 ->
 //   [reciprocal space: lowrank -> ewald_sf -> ewald_f -> ewald_atom, or on a
 //    particle mesh: lowrank -> spme_setup -> per term (spread -> FFT -> conv ->
 //    FFT -> gather)] ->
@@ -447,16 +447,20 @@ struct Workspace {
   // Packs the positions; with order_atoms also (re)computes the spatial order
   // of the atoms (the storage order of pair records and three-body lists).
   void pack(const Prepared& pb, const double* positions_dev, hipStream_t stream, bool order_atoms) {
+    if (pb.fixed_order) {
+      timed("pack", stream, [&] { launch_rank_pos(pb.db, positions_dev, stream); });
+      return;
+    }
     timed("pack", stream,
           [&] { launch_pack(positions_dev, pb.db.natoms, const_cast<double4*>(pb.db.pos), stream); });
-    if (order_atoms && !pb.fixed_order) {
+    if (order_atoms) {
       const size_t bytes = spatial_order_temp_bytes(pb.db.natoms);
       void* t = sort_tmp.get(bytes);
       timed("order", stream, [&] {
         launch_spatial_order(pb.db, t, bytes, const_cast<int*>(pb.db.rank), const_cast<int*>(pb.db.order), stream);
       });
     }
-    timed("pack", stream, [&] { launch_rank_pos(pb.db, stream); });
+    timed("pack", stream, [&] { launch_rank_pos(pb.db, nullptr, stream); });
   }
   DevWork work(const Prepared& pb, bool mixed, bool grad, const BatchOutput& out, const BatchDebug* debug);
   // count -> scans of the list sizes and of their work items (three-body lists of every atom)
@@ -902,8 +906,7 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
   const int natoms = db.natoms;
   pack(pb, positions_dev, stream, order_atoms);
   const DevWork w = work(pb, mixed, grad, out, debug);
-  timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, stream); });
-  timed("weights", stream, [&] { launch_weights(db, w.cn, w.gw, w.dgw, stream); });
+  timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, w.gw, w.dgw, w.gwr, w.spr, stream); });
   timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, w.tri, stream); });
   timed("disp2", stream, [&] { launch_disp2(db, mixed, grad, w, nullptr, stream); });
   if (pb.ewald && pb.spme) {
@@ -1077,8 +1080,7 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
   const bool mixed = precision == kMixed;
   m.pack(pb, positions_dev, stream, true);
   const DevWork w = m.work(pb, mixed, false, BatchOutput{}, nullptr);
-  m.timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, stream); });
-  m.timed("weights", stream, [&] { launch_weights(db, w.cn, w.gw, nullptr, stream); });
+  m.timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, w.gw, nullptr, w.gwr, w.spr, stream); });
   m.timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, nullptr, w.gwr, w.spr, w.pair, w.tri, stream); });
   m.timed("disp2", stream, [&] { launch_disp2(db, mixed, false, w, pair2, stream); });
   const size_t bytes = sizeof(double) * static_cast<size_t>(pb.pair_total);
@@ -1251,8 +1253,7 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
       if (s.pb.periodic_atm) {
         // lists of the initial coordinates, with headroom for later ones
         const DevWork w = s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
-        launch_cn(s.pb.db, s.mixed, w.cn, stream);
-        launch_weights(s.pb.db, w.cn, w.gw, w.dgw, stream);
+        launch_cn(s.pb.db, s.mixed, w.cn, w.gw, w.dgw, w.gwr, w.spr, stream);
         launch_pair(s.pb.db, s.mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, w.tri, stream);
         s.ws.list_offsets(s.pb.db, w.pair, s.mixed, w.atm_acc, nullptr, stream);
         long long total = 0;

@@ -166,7 +166,7 @@ class Engine {
   // Per-kernel timing with HIP events on the launch stream (resets totals).
   void set_kernel_timing(bool enable);
   // Total milliseconds and number of launches of a kernel group since the
-  // timing was enabled: pack, order, cn, weights, c6, disp2, lowrank,
+  // timing was enabled: pack, order, cn (with the weights), c6, disp2, lowrank,
   // ewald_sf, ewald_f, ewald_atom, atm_list, atm, cn_chain, reduce, hessian.
   std::pair<double, long long> kernel_time(const std::string& name) const;
 

@@ -283,9 +283,20 @@ __global__ void spatial_rank_kernel(DevBatch b, const int* __restrict__ order, i
 
 // ------------------------------------------------------- coordination number
 // ncoord.f90:86-144, one wavefront per atom i over all partners j and images
-// (each ordered pair once; the reference's triangle counts it for both atoms).
+// (each ordered pair once; the reference's triangle counts it for both atoms),
+// then, in the same wavefront, the atom's reference weights, model.f90:228-287
+// weight_references with wf = 4 (model.f90:80): always FP64 (weights down to
+// 1e-41 and the NaN fallback need it), one reference per lane of a group of 8.
+// They are written by atom (gw, dgw) and, for the lanes of pair_kernel, which
+// walk a row in spatial order and read consecutive addresses, by position x of
+// that order, reference-major: gwr[r][x], gwr[mref + r][x] (dw/dCN), and the
+// species with the ghost flag, spr[x].  Kernels of their own for the weights
+// and for that layout were two launches of 3 to 4 us in every evaluation.
+constexpr int kGhostBit = 1 << 20;
 template <typename R>
-__global__ __launch_bounds__(kBlock) void cn_kernel(DevBatch b, double* __restrict__ cn) {
+__global__ __launch_bounds__(kBlock) void cn_kernel(DevBatch b, double* __restrict__ cn, double* __restrict__ gw,
+                                                    double* __restrict__ dgw, double* __restrict__ gwr,
+                                                    int* __restrict__ spr) {
   const int lane = wave_lane();
   const int i = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (i >= b.natoms) return;
@@ -320,45 +331,43 @@ __global__ __launch_bounds__(kBlock) void cn_kernel(DevBatch b, double* __restri
     for (int j = g.atom_begin + lane; j < g.atom_begin + g.natoms; j += kWave) partner(j, b.pos[j]);
   }
   acc = wave_sum(acc);
-  if (lane == 0) cn[i] = acc;
-}
-
-// ------------------------------------------------------------ weights
-// model.f90:228-287 weight_references with wf = 4 (model.f90:80), FP64.
-__global__ void weights_kernel(DevBatch b, const double* __restrict__ cn, double* __restrict__ gw,
-                               double* __restrict__ dgw) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= b.natoms) return;
-  if (b.band && i < b.nsys) b.band[i] = 0;  // (a system has at least one atom)
-  const double wf = 4.0, wf2 = 2.0 * wf;
-  const int s = b.sp[i];
-  const int nr = b.nref[s];
-  const double* rcn = b.refcn + s * kMaxRef;
-  const double c = cn[i];
-  double gwt[kMaxRef];
-  double norm = 0.0, dnorm = 0.0, maxcn = -1.0e300;
-  for (int r = 0; r < nr; ++r) {
-    const double d = c - rcn[r];
-    const double w = exp(-wf * (d * d));
-    gwt[r] = w;
-    norm += w;
-    dnorm += wf2 * (rcn[r] - c) * w;
-    maxcn = fmax(maxcn, rcn[r]);
+  if (lane == 0) {
+    cn[i] = acc;
+    if (b.band && i == g.atom_begin) b.band[s] = 0;
+  }
+  static_assert(kMaxRef <= 8, "one reference per lane of a group of 8");
+  constexpr double wf = 4.0, wf2 = 2.0 * wf;
+  const int spi = b.sp[i], nr = b.nref[spi], r = lane & 7;
+  const double ref = r < nr ? b.refcn[spi * kMaxRef + r] : 0.0;
+  const double d = acc - ref;
+  const double expw = r < nr ? exp(-wf * (d * d)) : 0.0;
+  const double expd = wf2 * (ref - acc) * expw;
+  double norm = expw, dnorm = expd, maxcn = r < nr ? ref : -1.0e300;
+#pragma unroll
+  for (int off = 4; off > 0; off >>= 1) {
+    norm += __shfl_xor(norm, off, kWave);
+    dnorm += __shfl_xor(dnorm, off, kWave);
+    maxcn = fmax(maxcn, __shfl_xor(maxcn, off, kWave));
   }
   norm = 1.0 / norm;
-  for (int r = 0; r < b.mref; ++r) {
+  const int x = g.atom_begin + b.rank[i];
+  if (lane < b.mref) {
     double gwk = 0.0, dgwk = 0.0;
     if (r < nr) {
-      const double expw = gwt[r];
-      const double expd = wf2 * (rcn[r] - c) * expw;
       gwk = expw * norm;
-      if (isnan(gwk) || isinf(gwk)) gwk = (maxcn == rcn[r]) ? 1.0 : 0.0;  // model.f90:260-266
+      if (isnan(gwk) || isinf(gwk)) gwk = (maxcn == ref) ? 1.0 : 0.0;  // model.f90:260-266
       dgwk = expd * norm - expw * dnorm * (norm * norm);
       if (isnan(dgwk) || isinf(dgwk)) dgwk = 0.0;  // model.f90:269-273
     }
-    gw[i * b.mref + r] = gwk;
-    if (dgw) dgw[i * b.mref + r] = dgwk;
+    const long long nat = b.natoms;
+    gw[static_cast<long long>(i) * b.mref + r] = gwk;
+    gwr[r * nat + x] = gwk;
+    if (dgw) {
+      dgw[static_cast<long long>(i) * b.mref + r] = dgwk;
+      gwr[(b.mref + r) * nat + x] = dgwk;
+    }
   }
+  if (lane == 0) spr[x] = spi | (b.ghost && b.ghost[i] ? kGhostBit : 0);
 }
 
 // ---------------------------------------------------------- pair records
@@ -367,26 +376,6 @@ __global__ void weights_kernel(DevBatch b, const double* __restrict__ cn, double
 // (dC6_ij/dCN_j)/C6_ij, (4/3 rvdw_ij)^(alp/3)} (the last two feed the ATM
 // term, atm.f90:667-668,811-816).  One block per row i of the system block;
 // rows and columns are laid out in the spatial order of the atoms.
-// The weights, dw/dCN, species and ghost flags of the atoms at position x of
-// the batch's spatial order, reference-major: gwr[r][x], gwr[mref + r][x]
-// (with dw/dCN) and spr[x] = species | kGhostBit for a ghost atom, so that
-// the lanes of pair_kernel, which walk a row in that order, read consecutive
-// addresses.
-constexpr int kGhostBit = 1 << 20;
-__global__ __launch_bounds__(kBlock) void rank_weights_kernel(DevBatch b, const double* __restrict__ gw,
-                                                              const double* __restrict__ dgw,
-                                                              double* __restrict__ gwr, int* __restrict__ spr) {
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
-  if (x >= b.natoms) return;
-  const int j = b.order[x];
-  const int mref = b.mref, nat = b.natoms;
-  for (int r = 0; r < mref; ++r) {
-    gwr[static_cast<long long>(r) * nat + x] = gw[j * mref + r];
-    if (dgw) gwr[static_cast<long long>(mref + r) * nat + x] = dgw[j * mref + r];
-  }
-  spr[x] = b.sp[j] | (b.ghost && b.ghost[j] ? kGhostBit : 0);
-}
-
 __device__ __forceinline__ double pow_m8_3(double x);
 
 // With tri the block also writes the row of the three-body records of a
@@ -3789,14 +3778,11 @@ void launch_spatial_order(const DevBatch& b, void* temp, size_t temp_bytes, int*
   hipLaunchKernelGGL(spatial_rank_kernel, dim3(blocks_for(n, kBlock)), dim3(kBlock), 0, st, b, order, rank);
 }
 
-void launch_cn(const DevBatch& b, bool mixed, double* cn, hipStream_t st) {
+void launch_cn(const DevBatch& b, bool mixed, double* cn, double* gw, double* dgw, double* gwr, int* spr,
+               hipStream_t st) {
   const dim3 grid(blocks_for(b.natoms, kWavesPerBlock)), blk(kBlock);
-  if (mixed) hipLaunchKernelGGL(cn_kernel<float>, grid, blk, 0, st, b, cn);
-  else hipLaunchKernelGGL(cn_kernel<double>, grid, blk, 0, st, b, cn);
-}
-
-void launch_weights(const DevBatch& b, const double* cn, double* gw, double* dgw, hipStream_t st) {
-  hipLaunchKernelGGL(weights_kernel, dim3(blocks_for(b.natoms, kBlock)), dim3(kBlock), 0, st, b, cn, gw, dgw);
+  if (mixed) hipLaunchKernelGGL(cn_kernel<float>, grid, blk, 0, st, b, cn, gw, dgw, gwr, spr);
+  else hipLaunchKernelGGL(cn_kernel<double>, grid, blk, 0, st, b, cn, gw, dgw, gwr, spr);
 }
 
 namespace {
@@ -3804,14 +3790,23 @@ namespace {
 // The positions in spatial order, posr[x] = pos[order[x]], and the bounding
 // box of every 64-position tile of that order (wavefront per tile; the tiles
 // cover every position).
-__global__ __launch_bounds__(kBlock) void tile_box_kernel(DevBatch b, double4* __restrict__ posr,
+// With xyz (storage order = atom order) it also packs the caller's positions
+// into pos, instead of a kernel before it.
+__global__ __launch_bounds__(kBlock) void tile_box_kernel(DevBatch b, const double* __restrict__ xyz,
+                                                          double4* __restrict__ pos, double4* __restrict__ posr,
                                                           double4* __restrict__ tbox) {
   const int lane = wave_lane();
   const int t = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
   if (t >= b.ntiles) return;
   const int2 tile = b.tiles[t];
   const int x = tile.x + min(lane, tile.y - 1);  // lanes past the tile repeat its last position
-  const double4 p = b.pos[b.order[x]];
+  double4 p;
+  if (xyz) {
+    p = make_double4(xyz[3LL * x], xyz[3LL * x + 1], xyz[3LL * x + 2], 0.0);
+    if (lane < tile.y) pos[x] = p;
+  } else {
+    p = b.pos[b.order[x]];
+  }
   if (lane < tile.y) posr[x] = p;
   double lo[3] = {p.x, p.y, p.z}, hi[3] = {p.x, p.y, p.z};
 #pragma unroll
@@ -3847,16 +3842,14 @@ void* noalloc_area(int device, hipError_t* hip_err) {
   return p;
 }
 
-void launch_rank_pos(const DevBatch& b, hipStream_t st) {
+void launch_rank_pos(const DevBatch& b, const double* xyz, hipStream_t st) {
   if (b.ntiles > 0)
-    hipLaunchKernelGGL(tile_box_kernel, dim3(blocks_for(b.ntiles, kWavesPerBlock)), dim3(kBlock), 0, st, b,
-                       const_cast<double4*>(b.posr), const_cast<double4*>(b.tbox));
+    hipLaunchKernelGGL(tile_box_kernel, dim3(blocks_for(b.ntiles, kWavesPerBlock)), dim3(kBlock), 0, st, b, xyz,
+                       const_cast<double4*>(b.pos), const_cast<double4*>(b.posr), const_cast<double4*>(b.tbox));
 }
 
-void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, double* gwr, int* spr,
+void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, const double* gwr, const int* spr,
                  void* pair, double4* tri, hipStream_t st) {
-  hipLaunchKernelGGL(rank_weights_kernel, dim3(blocks_for(b.natoms, kBlock)), dim3(kBlock), 0, st, b, gw, dgw, gwr,
-                     spr);
   const size_t lds = sizeof(double) * static_cast<size_t>(b.nsp) * (2 * kMaxRef + 1);  // h, dh, r0p
   if (mixed)
     hipLaunchKernelGGL(pair_kernel<float>, dim3(b.natoms), dim3(kBlock), lds, st, b, gw, dgw, gwr, spr,

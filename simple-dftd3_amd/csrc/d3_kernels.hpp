@@ -84,14 +84,16 @@ void launch_pack(const double* xyz, int n, double4* pos, hipStream_t stream);
 size_t spatial_order_temp_bytes(int n);
 void launch_spatial_order(const DevBatch& b, void* temp, size_t temp_bytes, int* rank, int* order,
                           hipStream_t stream);
-void launch_cn(const DevBatch& b, bool mixed, double* cn, hipStream_t stream);
-void launch_weights(const DevBatch& b, const double* cn, double* gw, double* dgw, hipStream_t stream);
+// Coordination numbers and reference weights: by atom (gw, dgw [natoms][mref])
+// and in spatial order (gwr [2 mref][natoms], spr [natoms]); dgw may be null.
+void launch_cn(const DevBatch& b, bool mixed, double* cn, double* gw, double* dgw, double* gwr, int* spr,
+               hipStream_t stream);
 // posr[x] = pos[order[x]] for every position x of the batch's spatial order,
-// and the bounding box of every 64-position tile of that order (tbox).
-void launch_rank_pos(const DevBatch& b, hipStream_t stream);
-// gwr [(dgw ? 2 : 1) * mref][natoms] and spr [natoms]: scratch for the
-// weights in spatial order.
-void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, double* gwr, int* spr,
+// and the bounding box of every 64-position tile of that order (tbox).  With
+// xyz, the caller's positions of a batch whose storage order is the atom
+// order, it first packs them into pos.
+void launch_rank_pos(const DevBatch& b, const double* xyz, hipStream_t stream);
+void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, const double* gwr, const int* spr,
                  void* pair, double4* tri, hipStream_t stream);
 // pair2 (energy only, may be null): per system an n x n block (offset
 // c6_begin, atom order) of pairwise two-body energies.
