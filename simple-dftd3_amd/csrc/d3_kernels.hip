@@ -1830,11 +1830,14 @@ __global__ __launch_bounds__(kWave) void atm_pairs_kernel(DevBatch b, const long
 // g < 0, and in a system that has one (band[s]) triple_in_range decides every
 // triple with such a pair.
 enum PairSumMode { kPsEnergy, kPsGrad, kPsPairs };
+//
+// Three wavefronts per SIMD with the gradient, four without: four with the
+// gradient spill (planned batch of 1,024 molecules 2.93 and 3.17 ms;
+// 1,501-atom molecule, energy, three and four 0.613 and 0.594 ms).
 template <int kMode, int kT>
-__global__ __launch_bounds__(kBlock) void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items,
-                                                             const double4* __restrict__ tri,
-                                                             double2* __restrict__ psum, double* __restrict__ e_atom,
-                                                             double* __restrict__ pair3) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode == kPsGrad ? 3 : 4)))
+void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items, const double4* __restrict__ tri,
+                        double2* __restrict__ psum, double* __restrict__ e_atom, double* __restrict__ pair3) {
   constexpr int kSide = 8 * kT, kRecs = 2 * kSide, kC = 128 / kRecs, kOwn = kT * kT;
   constexpr int kSums = kMode == kPsGrad ? 3 : 1;
   __shared__ double2 stage[kWavesPerBlock][2][2 * kRecs * kC];
@@ -1847,22 +1850,20 @@ __global__ __launch_bounds__(kBlock) void atm_pairsum_kernel(DevBatch b, const i
   const double4* __restrict__ rec = tri + g.tri_begin;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = wave_lane();
   const int la = l >> 3, lb = l & 7;
-  double A[kOwn], c38[kOwn], G6[kOwn], h[kOwn], S[kOwn], Y[kOwn], Z[kOwn];
-  bool any = false, own_band[kOwn];
+  double A[kOwn], c38[kOwn], G6[kOwn], S[kOwn], Y[kOwn], Z[kOwn];
+  unsigned own = 0;  // bit o: pair o has terms; bit 8 + o: it is near the cutoff
 #pragma unroll
   for (int o = 0; o < kOwn; ++o) {
     const int a = I * kSide + la + 8 * (o / kT), bb = J * kSide + lb + 8 * (o % kT);
     const double4 q = a < n && bb < n ? rec[static_cast<long long>(a) * n + bb] : make_double4(1.0, 0.0, 0.0, 0.0);
     A[o] = q.x;
     c38[o] = 0.375 / q.x;
-    h[o] = kMode == kPsEnergy && a >= bb ? 0.0 : q.y;
     G6[o] = 6.0 * fabs(q.z);
-    own_band[o] = q.z < 0.0;
-    any |= h[o] != 0.0;
+    if (q.y != 0.0 && !(kMode == kPsEnergy && a >= bb)) own |= (q.z < 0.0 ? 0x101u : 1u) << o;
     S[o] = Y[o] = Z[o] = 0.0;
   }
   // (the wavefronts of the block hold the same pairs)
-  const bool live = __ballot(any) != 0ull;
+  const bool live = __ballot(own != 0u) != 0ull;
   if (kMode == kPsEnergy && !live) return;
 
   const int nchunks = (n + kC - 1) / kC;
@@ -1919,7 +1920,7 @@ __global__ __launch_bounds__(kBlock) void atm_pairsum_kernel(DevBatch b, const i
           bool ok = true;
           if (kMode == kPsEnergy && within) ok = chunk * kC + c > J * kSide + lb + 8 * (o % kT);
           if (kBanded) {
-            if ((x.z < 0.0 || y.z < 0.0 || own_band[o]) && ok && h[o] != 0.0 && x.y != 0.0 && y.y != 0.0) {
+            if ((x.z < 0.0 || y.z < 0.0 || (own >> (8 + o) & 1u)) && (own >> o & 1u) && ok && x.y != 0.0 && y.y != 0.0) {
               const int* __restrict__ ord = b.order + g.atom_begin;
               ok = triple_in_range(b.pos, ord[I * kSide + la + 8 * (o / kT)], ord[J * kSide + lb + 8 * (o % kT)],
                                    ord[chunk * kC + c], p.cut3 * p.cut3);
@@ -1976,13 +1977,11 @@ __global__ __launch_bounds__(kBlock) void atm_pairsum_kernel(DevBatch b, const i
       for (int q = 0; q < kWavesPerBlock; ++q) t[v] += sums[((q * kSums + v) * kOwn + w) * kWave + l];
     }
     // w is uniform: the pair's constants without an indexed register file
-    double Ao = A[0], ho = h[0];
+    double Ao = A[0];
 #pragma unroll
-    for (int o = 1; o < kOwn; ++o) {
-      Ao = w == o ? A[o] : Ao;
-      ho = w == o ? h[o] : ho;
-    }
+    for (int o = 1; o < kOwn; ++o) Ao = w == o ? A[o] : Ao;
     const int a = I * kSide + la + 8 * (w / kT), bb = J * kSide + lb + 8 * (w % kT);
+    const double ho = own >> w & 1u ? rec[static_cast<long long>(a) * n + bb].y : 0.0;
     const double E = p.s9 * ho * t[0];  // energy of all triples of the pair
     if (kMode == kPsEnergy) e = E;
     if (a <= bb && bb < n) {  // (a diagonal tile holds both orders of its pairs)
