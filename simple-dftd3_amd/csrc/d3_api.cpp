@@ -46,14 +46,17 @@ struct _dftd3_model {
   int precision = d3::kFP64;
   std::unique_ptr<d3::Engine> engine;
   hipStream_t stream = nullptr;
-  // device buffers of the host-pointer entry point
-  double* d_xyz = nullptr;
+  // buffers of the host-pointer entry points: pinned host memory for the
+  // positions, which the packing kernel reads in place, and the results
+  // (every call ends with a stream synchronisation, so the next may write it)
+  double* h_xyz = nullptr;
+  double* h_out = nullptr;
   double* d_out = nullptr;  // energy | sigma[9] | gradient[nat][3]
   size_t cap_atoms = 0;
   double* d_pairs = nullptr;  // pairwise energies pair2 | pair3, or the Hessian
   size_t cap_pairs = 0;       // doubles allocated at d_pairs
   ~_dftd3_model() {
-    if (d_xyz) (void)hipFree(d_xyz);
+    if (h_xyz) (void)hipHostFree(h_xyz);
     if (d_out) (void)hipFree(d_out);
     if (d_pairs) (void)hipFree(d_pairs);
     if (stream) (void)hipStreamDestroy(stream);
@@ -173,13 +176,18 @@ const ParamRecord* find_record(const ParamRecord* table, int n, const char* id) 
 
 void ensure_model_buffers(_dftd3_model* m, int nat) {
   if (!m->stream) d3::hip_check(hipStreamCreate(&m->stream), "hipStreamCreate");
-  if (static_cast<size_t>(nat) > m->cap_atoms || !m->d_xyz) {
-    if (m->d_xyz) d3::hip_check(hipFree(m->d_xyz), "hipFree");
+  if (static_cast<size_t>(nat) > m->cap_atoms || !m->h_xyz) {
+    if (m->h_xyz) d3::hip_check(hipHostFree(m->h_xyz), "hipHostFree");
     if (m->d_out) d3::hip_check(hipFree(m->d_out), "hipFree");
-    m->d_xyz = nullptr;
+    m->h_xyz = nullptr;
     m->d_out = nullptr;
-    d3::hip_check(hipMalloc(&m->d_xyz, sizeof(double) * 3 * std::max(nat, 1)), "hipMalloc");
-    d3::hip_check(hipMalloc(&m->d_out, sizeof(double) * (10 + 3 * std::max(nat, 1))), "hipMalloc");
+    m->cap_atoms = 0;
+    const size_t xyz = 3 * static_cast<size_t>(std::max(nat, 1));
+    d3::hip_check(hipHostMalloc(reinterpret_cast<void**>(&m->h_xyz), sizeof(double) * (2 * xyz + 10),
+                                hipHostMallocDefault),
+                  "hipHostMalloc");
+    m->h_out = m->h_xyz + xyz;
+    d3::hip_check(hipMalloc(&m->d_out, sizeof(double) * (10 + xyz)), "hipMalloc");
     m->cap_atoms = nat;
   }
 }
@@ -572,25 +580,23 @@ void dftd3_get_dispersion(dftd3_error error, dftd3_structure mol, dftd3_model di
     sys[0].part = disp->part;  // api.f90:1099
     sys[0].nparts = disp->nparts;
     const bool grad = gradient || sigma;
-    d3::hip_check(hipMemcpyAsync(disp->d_xyz, mol->xyz.data(), sizeof(double) * 3 * nat, hipMemcpyHostToDevice,
-                                 disp->stream),
-                  "upload positions");
+    std::memcpy(disp->h_xyz, mol->xyz.data(), sizeof(double) * 3 * nat);
     d3::BatchOutput out;
     out.energy = disp->d_out;
     out.sigma = grad ? disp->d_out + 1 : nullptr;
     out.gradient = grad ? disp->d_out + 10 : nullptr;
     bool any_ghost = false;
     for (int g : disp->ghost) any_ghost |= g != 0;
-    disp->engine->run(sys, mol->num.data(), disp->d_xyz, disp->precision, out, disp->stream, nullptr, nullptr,
+    disp->engine->run(sys, mol->num.data(), disp->h_xyz, disp->precision, out, disp->stream, nullptr, nullptr,
                       any_ghost ? disp->ghost.data() : nullptr);
-    std::vector<double> host(grad ? 10 + 3 * nat : 1);
-    d3::hip_check(hipMemcpyAsync(host.data(), disp->d_out, sizeof(double) * host.size(), hipMemcpyDeviceToHost,
-                                 disp->stream),
+    const double* host = disp->h_out;
+    d3::hip_check(hipMemcpyAsync(disp->h_out, disp->d_out, sizeof(double) * (grad ? 10 + 3 * nat : 1),
+                                 hipMemcpyDeviceToHost, disp->stream),
                   "download results");
     d3::hip_check(hipStreamSynchronize(disp->stream), "hipStreamSynchronize");
     if (energy) *energy = host[0];
-    if (sigma) std::memcpy(sigma, host.data() + 1, sizeof(double) * 9);
-    if (gradient) std::memcpy(gradient, host.data() + 10, sizeof(double) * 3 * nat);
+    if (sigma) std::memcpy(sigma, host + 1, sizeof(double) * 9);
+    if (gradient) std::memcpy(gradient, host + 10, sizeof(double) * 3 * nat);
   });
 }
 
@@ -615,12 +621,10 @@ void dftd3_get_pairwise_dispersion(dftd3_error error, dftd3_structure mol, dftd3
     std::memcpy(sys[0].periodic, mol->periodic, sizeof mol->periodic);
     sys[0].param = make_sys_param(param, disp->cutoff);
     sys[0].lowrank = disp->lowrank.get();
-    d3::hip_check(hipMemcpyAsync(disp->d_xyz, mol->xyz.data(), sizeof(double) * 3 * nat, hipMemcpyHostToDevice,
-                                 disp->stream),
-                  "upload positions");
+    std::memcpy(disp->h_xyz, mol->xyz.data(), sizeof(double) * 3 * nat);
     bool any_ghost = false;
     for (int g : disp->ghost) any_ghost |= g != 0;
-    disp->engine->run_pairwise(sys, mol->num.data(), disp->d_xyz, disp->precision, disp->d_pairs,
+    disp->engine->run_pairwise(sys, mol->num.data(), disp->h_xyz, disp->precision, disp->d_pairs,
                                disp->d_pairs + nn, disp->stream, any_ghost ? disp->ghost.data() : nullptr);
     d3::hip_check(hipMemcpyAsync(pair_energy2, disp->d_pairs, sizeof(double) * nn, hipMemcpyDeviceToHost,
                                  disp->stream),
@@ -655,12 +659,10 @@ void dftd3_get_dispersion_hessian(dftd3_error error, dftd3_structure mol, dftd3_
     sys[0].lowrank = disp->lowrank.get();
     sys[0].part = disp->part;  // api.f90:1170
     sys[0].nparts = disp->nparts;
-    d3::hip_check(hipMemcpyAsync(disp->d_xyz, mol->xyz.data(), sizeof(double) * 3 * nat, hipMemcpyHostToDevice,
-                                 disp->stream),
-                  "upload positions");
+    std::memcpy(disp->h_xyz, mol->xyz.data(), sizeof(double) * 3 * nat);
     bool any_ghost = false;
     for (int g : disp->ghost) any_ghost |= g != 0;
-    disp->engine->run_hessian(sys, mol->num.data(), disp->d_xyz, disp->d_out, disp->d_pairs, disp->stream,
+    disp->engine->run_hessian(sys, mol->num.data(), disp->h_xyz, disp->d_out, disp->d_pairs, disp->stream,
                               any_ghost ? disp->ghost.data() : nullptr);
     double e = 0.0;
     d3::hip_check(hipMemcpyAsync(&e, disp->d_out, sizeof(double), hipMemcpyDeviceToHost, disp->stream),
