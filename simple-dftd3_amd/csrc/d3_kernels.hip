@@ -2985,60 +2985,89 @@ __global__ __launch_bounds__(kBlock) void hess_cn_kernel(DevBatch b, const doubl
       for (int c = 0; c < 3; ++c) hrow[static_cast<long long>(a) * ndim + 3 * il + c] += hii[3 * a + c];
 }
 
-// tmp[k][y] = sum_l dEdcndcn[k][l] dr[y][l] (n x 3n per system; grid.z = system).
-constexpr int kHT = 16;  // tile edge of the dense products
-__global__ __launch_bounds__(kHT * kHT) void hess_tmp_kernel(DevBatch b, const double* __restrict__ dEdcndcn,
-                                                             const double* __restrict__ dr, double* __restrict__ tmp) {
-  const SysGeom g = b.geom[blockIdx.z];
-  const int n = g.natoms, ndim = 3 * n;
-  const int k = blockIdx.y * kHT + threadIdx.y, y = blockIdx.x * kHT + threadIdx.x;
-  __shared__ double A[kHT][kHT + 1], B[kHT][kHT + 1];
-  const double* C = dEdcndcn + g.c6_begin;
-  const double* D = dr + 3 * g.c6_begin;
-  double acc = 0.0;
-  for (int l0 = 0; l0 < n; l0 += kHT) {
-    const int la = l0 + threadIdx.x;
-    A[threadIdx.y][threadIdx.x] = (k < n && la < n) ? C[static_cast<long long>(k) * n + la] : 0.0;
-    const int yb = blockIdx.x * kHT + threadIdx.y;
-    B[threadIdx.y][threadIdx.x] = (yb < ndim && la < n) ? D[static_cast<long long>(yb) * n + la] : 0.0;
-    __syncthreads();
-    for (int q = 0; q < kHT; ++q) acc += A[threadIdx.y][q] * B[threadIdx.x][q];
-    __syncthreads();
+// The Hessian's part through the coordination numbers (disp.f90:303-306),
+// H += A D^T + D A^T + D X D^T with A = d2E/dRdCN, D = dCN/dR (3n x n, row-major)
+// and X = d2E/dCN^2 (n x n, symmetric), as H += B D^T + D B^T, B = A + D X / 2,
+// by FP64 matrix instructions.  A block owns a 16 x 16 tile of the result (of
+// the upper triangle of H), its wavefronts take 16 columns k in turn.  Lane l
+// holds columns k + 4 (l / 16) .. + 3 of row l mod 16 of both factors, so a
+// wavefront reads whole lines, and the four instructions of a step take one of
+// these columns each (the sum over k is in no particular order).  With one
+// value a thread and scalar products from the LDS the products took 74 us of a
+// 200-atom molecule's 259, now 25 of 214.
+constexpr int kHT = 16;  // tile edge
+using Mfma4 = __attribute__((__vector_size__(4 * sizeof(double)))) double;
+
+// acc += rows x0 .. x0 + 15 of P times rows y0 .. y0 + 15 of Q, transposed
+// (columns of this wavefront; rows past the last are clamped, their results
+// unused).
+__device__ __forceinline__ void mfma_rows(Mfma4& acc, const double* __restrict__ P, int x0, int nx,
+                                          const double* __restrict__ Q, int y0, int ny, int n, int w) {
+  const int l = wave_lane();
+  const double* __restrict__ p = P + static_cast<long long>(min(x0 + (l & 15), nx - 1)) * n;
+  const double* __restrict__ q = Q + static_cast<long long>(min(y0 + (l & 15), ny - 1)) * n;
+  for (int k0 = 16 * w + 4 * (l >> 4); k0 - 4 * (l >> 4) < n; k0 += 16 * kWavesPerBlock) {
+    double a[4], c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool in = k0 + k < n;
+      a[k] = in ? p[k0 + k] : 0.0;
+      c[k] = in ? q[k0 + k] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[k], c[k], acc, 0, 0, 0);
   }
-  if (k < n && y < ndim) tmp[3 * g.c6_begin + static_cast<long long>(k) * ndim + y] = acc;
 }
 
-// hess[x][y] += sum_k dEdcndr[x][k] dr[y][k] + dr[x][k] dEdcndr[y][k] + dr[x][k] tmp[k][y]
-// (disp.f90:303-306; grid.z = system).
-__global__ __launch_bounds__(kHT * kHT) void hess_assemble_kernel(DevBatch b, const double* __restrict__ dEdcndr,
-                                                                  const double* __restrict__ dr,
-                                                                  const double* __restrict__ tmp,
-                                                                  double* __restrict__ hess) {
+// The sum of the wavefronts' tiles, one element per thread: row 4 (t / 64) +
+// (t mod 64) / 16, column t mod 16 (value r of lane l is row 4 r + l / 16).
+__device__ __forceinline__ double mfma_tile_sum(const Mfma4& acc, double (*red)[kBlock]) {
+  const int w = threadIdx.x >> 6, l = wave_lane();
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[w][r * kWave + l] = acc[r];
+  __syncthreads();
+  double v = 0.0;
+  for (int q = 0; q < kWavesPerBlock; ++q) v += red[q][threadIdx.x];
+  return v;
+}
+
+// B = A + D X / 2 (grid: tiles of the columns, of the rows, systems).
+__global__ __launch_bounds__(kBlock) void hess_b_kernel(DevBatch b, const double* __restrict__ dEdcndr,
+                                                        const double* __restrict__ dr,
+                                                        const double* __restrict__ dEdcndcn, double* __restrict__ B) {
+  __shared__ double red[kWavesPerBlock][kBlock];
   const SysGeom g = b.geom[blockIdx.z];
-  const int n = g.natoms, ndim = 3 * n;
-  const int x = blockIdx.y * kHT + threadIdx.y, y = blockIdx.x * kHT + threadIdx.x;
-  __shared__ double Ax[kHT][kHT + 1], Dx[kHT][kHT + 1], Ay[kHT][kHT + 1], Dy[kHT][kHT + 1], Tk[kHT][kHT + 1];
-  const double* A = dEdcndr + 3 * g.c6_begin;
-  const double* D = dr + 3 * g.c6_begin;
-  const double* T = tmp + 3 * g.c6_begin;
-  double acc = 0.0;
-  for (int k0 = 0; k0 < n; k0 += kHT) {
-    const int kk = k0 + threadIdx.x;
-    const int xr = blockIdx.y * kHT + threadIdx.y, yr = blockIdx.x * kHT + threadIdx.y;
-    const bool kok = kk < n;
-    Ax[threadIdx.y][threadIdx.x] = (xr < ndim && kok) ? A[static_cast<long long>(xr) * n + kk] : 0.0;
-    Dx[threadIdx.y][threadIdx.x] = (xr < ndim && kok) ? D[static_cast<long long>(xr) * n + kk] : 0.0;
-    Ay[threadIdx.y][threadIdx.x] = (yr < ndim && kok) ? A[static_cast<long long>(yr) * n + kk] : 0.0;
-    Dy[threadIdx.y][threadIdx.x] = (yr < ndim && kok) ? D[static_cast<long long>(yr) * n + kk] : 0.0;
-    const int kt = k0 + threadIdx.y, yt = blockIdx.x * kHT + threadIdx.x;
-    Tk[threadIdx.y][threadIdx.x] = (kt < n && yt < ndim) ? T[static_cast<long long>(kt) * ndim + yt] : 0.0;
-    __syncthreads();
-    for (int q = 0; q < kHT; ++q)
-      acc += Ax[threadIdx.y][q] * Dy[threadIdx.x][q] + Dx[threadIdx.y][q] * Ay[threadIdx.x][q] +
-             Dx[threadIdx.y][q] * Tk[q][threadIdx.x];
-    __syncthreads();
+  const int n = g.natoms, ndim = 3 * n, x0 = blockIdx.y * kHT, y0 = blockIdx.x * kHT;
+  if (x0 >= ndim || y0 >= n) return;
+  Mfma4 acc = {0.0, 0.0, 0.0, 0.0};
+  mfma_rows(acc, dr + 3 * g.c6_begin, x0, ndim, dEdcndcn + g.c6_begin, y0, n, n, threadIdx.x >> 6);
+  const double v = mfma_tile_sum(acc, red);
+  const int x = x0 + 4 * (threadIdx.x >> 6) + ((threadIdx.x & 63) >> 4), y = y0 + (threadIdx.x & 15);
+  if (x < ndim && y < n) {
+    const long long o = 3 * g.c6_begin + static_cast<long long>(x) * n + y;
+    B[o] = dEdcndr[o] + 0.5 * v;
   }
-  if (x < ndim && y < ndim) hess[9 * g.c6_begin + static_cast<long long>(x) * ndim + y] += acc;
+}
+
+// H += B D^T + D B^T (grid: tiles of the columns, of the rows, systems).
+__global__ __launch_bounds__(kBlock) void hess_assemble_kernel(DevBatch b, const double* __restrict__ B,
+                                                               const double* __restrict__ dr,
+                                                               double* __restrict__ hess) {
+  __shared__ double red[kWavesPerBlock][kBlock];
+  const SysGeom g = b.geom[blockIdx.z];
+  const int n = g.natoms, ndim = 3 * n, x0 = blockIdx.y * kHT, y0 = blockIdx.x * kHT;
+  if (x0 > y0 || y0 >= ndim) return;
+  const double* __restrict__ Bs = B + 3 * g.c6_begin;
+  const double* __restrict__ D = dr + 3 * g.c6_begin;
+  Mfma4 acc = {0.0, 0.0, 0.0, 0.0};
+  mfma_rows(acc, Bs, x0, ndim, D, y0, ndim, n, threadIdx.x >> 6);
+  mfma_rows(acc, D, x0, ndim, Bs, y0, ndim, n, threadIdx.x >> 6);
+  const double v = mfma_tile_sum(acc, red);
+  const int x = x0 + 4 * (threadIdx.x >> 6) + ((threadIdx.x & 63) >> 4), y = y0 + (threadIdx.x & 15);
+  if (x >= ndim || y >= ndim) return;
+  double* __restrict__ H = hess + 9 * g.c6_begin;
+  H[static_cast<long long>(x) * ndim + y] += v;
+  if (x0 != y0) H[static_cast<long long>(y) * ndim + x] += v;
 }
 
 
@@ -4219,10 +4248,10 @@ void launch_hessian(const DevBatch& b, const HessWork& h, const long long* offse
   }
   hipLaunchKernelGGL(hess_cn_kernel, wgrid, blk, 0, st, b, h.dedcn, h.hess);
   const int ndim = 3 * max_natoms;
-  hipLaunchKernelGGL(hess_tmp_kernel, dim3(blocks_for(ndim, kHT), blocks_for(max_natoms, kHT), b.nsys),
-                     dim3(kHT, kHT), 0, st, b, h.dEdcndcn, h.dr, h.tmp);
-  hipLaunchKernelGGL(hess_assemble_kernel, dim3(blocks_for(ndim, kHT), blocks_for(ndim, kHT), b.nsys),
-                     dim3(kHT, kHT), 0, st, b, h.dEdcndr, h.dr, h.tmp, h.hess);
+  hipLaunchKernelGGL(hess_b_kernel, dim3(blocks_for(max_natoms, kHT), blocks_for(ndim, kHT), b.nsys), blk, 0, st, b,
+                     h.dEdcndr, h.dr, h.dEdcndcn, h.tmp);
+  hipLaunchKernelGGL(hess_assemble_kernel, dim3(blocks_for(ndim, kHT), blocks_for(ndim, kHT), b.nsys), blk, 0, st, b,
+                     h.tmp, h.dr, h.hess);
 }
 
 }  // namespace d3

@@ -162,7 +162,7 @@ void launch_atm_pairsum(const DevBatch& b, bool mixed, bool grad, const PairSumI
 void launch_pair3_finalize(const DevBatch& b, const double* pair3s, double* out, hipStream_t stream);
 // Analytic Hessian (FP64) of a batch; per system, atom order within the
 // system, offsets from c6_begin: c6, dc6, d2c6, d2c6ij and dEdcndcn n x n at
-// c6_begin; dr and dEdcndr 3n x n and tmp n x 3n at 3 c6_begin; hess 3n x 3n
+// c6_begin; dr, dEdcndr and tmp 3n x n at 3 c6_begin; hess 3n x 3n
 // at 9 c6_begin.  hess, dedcn, dEdcndr and dEdcndcn must be zeroed; the
 // FP64 three-body lists (offset, slots; total_slots entries) must be filled
 // and cn computed.  max_natoms: largest system of the batch.
