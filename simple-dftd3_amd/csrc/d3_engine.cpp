@@ -33,6 +33,10 @@ namespace {
 
 constexpr double kEps = 2.220446049250313e-16;
 
+struct ArenaFull : Error {
+  using Error::Error;
+};
+
 // A fixed region of device memory handed out front to back (256-byte
 // aligned); reset() makes all of it free again.  Used by the allocation-free
 // entry point, whose region is the library's static work area.
@@ -47,8 +51,8 @@ class Arena {
   void* take(size_t bytes) {
     const size_t at = (used_ + 255) / 256 * 256;
     if (at > size_ || bytes > size_ - at)
-      throw Error("The batch needs more device memory than the fixed work area of the allocation-free entry point (" +
-                  std::to_string(size_ >> 20) + " MiB)");
+      throw ArenaFull("The batch needs more device memory than the fixed work area of the allocation-free entry point (" +
+                      std::to_string(size_ >> 20) + " MiB)");
     used_ = at + bytes;
     return base_ + at;
   }
@@ -1050,15 +1054,25 @@ void run_noalloc(const std::vector<SystemDesc>& systems, const int* numbers, con
     st->ws.use_arena(&st->arena);
   }
   Workspace& m = st->ws;
-  m.reset_arena();
   const bool grad = out.gradient || out.sigma;
-  const Prepared pb = m.upload(systems, numbers, stream, nullptr, pair_sum_atoms(precision == kMixed, grad));
   // the gradient is summed in the work area and copied out at the end, so
   // that a batch rejected for its size leaves every output untouched
   BatchOutput inner = out;
   inner.gradient = nullptr;
-  m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, inner, nullptr, nullptr, -1, 0,
-             kPerCallShape, stream);
+  Prepared pb;
+  auto attempt = [&](int max_pair_sum) {
+    m.reset_arena();
+    pb = m.upload(systems, numbers, stream, nullptr, max_pair_sum);
+    m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, inner, nullptr, nullptr, -1, 0,
+               kPerCallShape, stream);
+  };
+  // pair sums take 48 bytes a pair of atoms where lists take 40: a batch that
+  // only fits with lists gets them
+  try {
+    attempt(pair_sum_atoms(precision == kMixed, grad));
+  } catch (const ArenaFull&) {
+    attempt(0);
+  }
   if (out.gradient)
     hip_check(hipMemcpyAsync(out.gradient, m.grad.as<double>(size_t(pb.db.natoms) * 3),
                              sizeof(double) * 3 * size_t(pb.db.natoms), hipMemcpyDeviceToDevice, stream),
