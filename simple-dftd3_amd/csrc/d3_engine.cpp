@@ -7,7 +7,7 @@
 //   [reciprocal space: lowrank -> ewald_sf -> ewald_f -> ewald_atom, or on a
 //    particle mesh: lowrank -> spme_setup -> per term (spread -> FFT -> conv ->
 //    FFT -> gather)] ->
-//   atm_list (count, scan, fill) -> atm -> cn_chain -> reduce
+//   atm_list (count, scan, fill) -> atm -> [molecules: pair sums] -> cn_chain -> reduce
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 
@@ -911,8 +911,9 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
   pack(pb, positions_dev, stream, order_atoms);
   const DevWork w = work(pb, mixed, grad, out, debug);
   timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, w.gw, w.dgw, w.gwr, w.spr, stream); });
-  timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, w.tri, stream); });
-  timed("disp2", stream, [&] { launch_disp2(db, mixed, grad, w, nullptr, stream); });
+  timed("c6", stream, [&] { launch_pair(db, mixed, w, true, grad, stream); });
+  if (pb.tri_total < pb.pair_total)
+    timed("disp2", stream, [&] { launch_disp2(db, mixed, grad, w, nullptr, stream); });
   if (pb.ewald && pb.spme) {
     // fourier/spme.f90:78-328, term by term of the expansion
     const EwaldBatch& e = pb.eb;
@@ -1095,7 +1096,7 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
   m.pack(pb, positions_dev, stream, true);
   const DevWork w = m.work(pb, mixed, false, BatchOutput{}, nullptr);
   m.timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, w.gw, nullptr, w.gwr, w.spr, stream); });
-  m.timed("c6", stream, [&] { launch_pair(db, mixed, w.gw, nullptr, w.gwr, w.spr, w.pair, w.tri, stream); });
+  m.timed("c6", stream, [&] { launch_pair(db, mixed, w, false, false, stream); });
   m.timed("disp2", stream, [&] { launch_disp2(db, mixed, false, w, pair2, stream); });
   const size_t bytes = sizeof(double) * static_cast<size_t>(pb.pair_total);
   if (!pb.any_atm) {
@@ -1268,7 +1269,7 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
         // lists of the initial coordinates, with headroom for later ones
         const DevWork w = s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
         launch_cn(s.pb.db, s.mixed, w.cn, w.gw, w.dgw, w.gwr, w.spr, stream);
-        launch_pair(s.pb.db, s.mixed, w.gw, w.dgw, w.gwr, w.spr, w.pair, w.tri, stream);
+        launch_pair(s.pb.db, s.mixed, w, false, grad, stream);
         s.ws.list_offsets(s.pb.db, w.pair, s.mixed, w.atm_acc, nullptr, stream);
         long long total = 0;
         hip_check(hipMemcpyAsync(&total, s.ws.off.as<long long>(natoms + 1) + natoms, sizeof total,

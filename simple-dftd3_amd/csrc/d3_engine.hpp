@@ -180,7 +180,8 @@ class Engine {
 // kernel launches on one stream without host synchronisation or allocation,
 // which can be captured in a HIP graph and replayed.
 //
-// Three-body lists: a batch of molecules gets the exact bound n(n+1)/2 slots
+// Three-body lists (molecules of the pair-sum route have none): a batch of
+// molecules gets the exact bound n(n+1)/2 slots
 // per molecule; a periodic system gets 1.5 times the list size of the
 // coordinates the plan is made with (and at least 64 more slots per atom of a
 // system with a three-body term),

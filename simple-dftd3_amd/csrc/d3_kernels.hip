@@ -370,104 +370,6 @@ __global__ __launch_bounds__(kBlock) void cn_kernel(DevBatch b, double* __restri
   if (lane == 0) spr[x] = spi | (b.ghost && b.ghost[i] ? kGhostBit : 0);
 }
 
-// ---------------------------------------------------------- pair records
-// model.f90:432-462: C6_ij = sum_kl w_ik w_jl C6ref_kl and its derivatives,
-// stored per ordered pair as {sqrt(C6_ij), (dC6_ij/dCN_i)/C6_ij,
-// (dC6_ij/dCN_j)/C6_ij, (4/3 rvdw_ij)^(alp/3)} (the last two feed the ATM
-// term, atm.f90:667-668,811-816).  One block per row i of the system block;
-// rows and columns are laid out in the spatial order of the atoms.
-__device__ __forceinline__ double pow_m8_3(double x);
-
-// With tri the block also writes the row of the three-body records of a
-// system of the pair-sum route (see atm_pairsum_kernel).
-template <typename R>
-__global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* __restrict__ gw,
-                                                      const double* __restrict__ dgw,
-                                                      const double* __restrict__ gwr, const int* __restrict__ spr,
-                                                      R4<R>* __restrict__ pair, double4* __restrict__ tri) {
-  const int i = blockIdx.x;
-  const int s = b.sys[i];
-  const SysGeom g = b.geom[s];
-  const double alp3 = (b.par[s].alp + 2.0) / 3.0;
-  const int n = g.natoms;
-  const int spi = b.sp[i];
-  const int mref = b.mref;
-  const int nri = b.nref[spi];
-  double gi[kMaxRef], dgi[kMaxRef];
-  for (int r = 0; r < kMaxRef; ++r) {
-    gi[r] = r < nri ? gw[i * mref + r] : 0.0;
-    dgi[r] = (r < nri && dgw) ? dgw[i * mref + r] : 0.0;
-  }
-  // per species s of the batch: h[s][r] = sum_ri w_i[ri] C6ref[ri][r] and the
-  // same with dw_i/dCN_i, so that a record costs three nref_j-term dots; and
-  // (4/3 rvdw_is)^(alp/3), in dynamic LDS ((2 kMaxRef + 1) nsp doubles, sized
-  // at the launch).
-  extern __shared__ double pair_lds[];
-  double* __restrict__ h = pair_lds;                   // [nsp][kMaxRef]
-  double* __restrict__ dh = pair_lds + b.nsp * kMaxRef;  // [nsp][kMaxRef]
-  double* __restrict__ r0p_s = dh + b.nsp * kMaxRef;     // [nsp]
-  for (int t = threadIdx.x; t < b.nsp * kMaxRef; t += blockDim.x) {
-    const int sj = t / kMaxRef, rj = t % kMaxRef;
-    const double* ref = b.c6ref + (spi * b.nsp + sj) * (kMaxRef * kMaxRef);
-    double a = 0.0, d = 0.0;
-    for (int ri = 0; ri < nri; ++ri) {
-      a += gi[ri] * ref[ri * kMaxRef + rj];
-      d += dgi[ri] * ref[ri * kMaxRef + rj];
-    }
-    h[t] = a;
-    dh[t] = d;
-  }
-  for (int t = threadIdx.x; t < b.nsp; t += blockDim.x) r0p_s[t] = pow(kRs9 * b.rvdw[t * b.nsp + spi], alp3);
-  __syncthreads();
-  const bool gi_ghost = b.ghost && b.ghost[i];
-  const int ri = b.rank[i];
-  R4<R>* row = pair + g.c6_begin + static_cast<long long>(ri) * n;
-  double4* tri_row = g.tri_begin >= 0 ? tri + g.tri_begin + static_cast<long long>(ri) * n : nullptr;
-  const double4 xi = b.pos[i];
-  const double cut3 = b.par[s].cut3, width3 = b.par[s].width3;
-  const bool alp14 = b.par[s].alp == 14.0;
-  const long long nat = b.natoms;
-  for (int jr = threadIdx.x; jr < n; jr += blockDim.x) {
-    const int x = g.atom_begin + jr;  // position of partner j in the spatial order
-    const int code = spr[x];
-    const int spj = code & (kGhostBit - 1);
-    const int nrj = b.nref[spj];
-    double cc = 0.0, di = 0.0, dj = 0.0;
-    if (!(gi_ghost || (code & kGhostBit))) {  // model.f90:436-440
-      for (int rj = 0; rj < nrj; ++rj) {
-        const double w = gwr[rj * nat + x];
-        cc += w * h[spj * kMaxRef + rj];
-        if (dgw) {
-          di += w * dh[spj * kMaxRef + rj];
-          dj += gwr[(mref + rj) * nat + x] * h[spj * kMaxRef + rj];
-        }
-      }
-    }
-    const double ic = cc > 0.0 ? 1.0 / cc : 0.0;
-    const double sc6 = sqrt(cc);
-    row[jr] = make_r4<R>(R(sc6), R(di * ic), R(dj * ic), R(r0p_s[spj]));
-    if (!tri_row) continue;
-    double4 t = make_double4(1.0, 0.0, 0.0, 0.0);  // no pair: no term
-    double v0, v1, v2;
-    const double r2 = atm_vec(b.posr[x], make_double4(0.0, 0.0, 0.0, 0.0), xi, v0, v1, v2);
-    const double cut2 = cut3 * cut3;
-    if (jr != ri && r2 <= cut2 * (1.0 + kBand) && r2 >= kEps && cc >= kEps) {
-      const double r1 = sqrt(r2);
-      double sw, dswdr;
-      smooth_cutoff(r1, cut3, width3, sw, dswdr);
-      t.x = r2;
-      t.y = sw * sc6 / (r2 * r1);
-      t.z = r0p_s[spj] * (alp14 ? pow_m8_3(r2) : pow(r2, -0.5 * alp3));
-      t.w = t.y / r2;
-      if (r2 > cut2 * (1.0 - kBand)) {  // see atm_pairsum_kernel
-        t.z = -t.z;
-        b.band[s] = 1;
-      }
-    }
-    tri_row[jr] = t;
-  }
-}
-
 // ------------------------------------------------- two-body damping families
 // Per-pair constants of the damping (what the reference hoists out of the
 // image loop) and one pair term without the switching function:
@@ -661,6 +563,180 @@ __device__ __forceinline__ bool two_body_active(const SysParam& p) {
   return !(fabs(p.s6) < kEps && fabs(p.s8) < kEps);
 }
 
+// ---------------------------------------------------------- pair records
+// model.f90:432-462: C6_ij = sum_kl w_ik w_jl C6ref_kl and its derivatives,
+// stored per ordered pair as {sqrt(C6_ij), (dC6_ij/dCN_i)/C6_ij,
+// (dC6_ij/dCN_j)/C6_ij, (4/3 rvdw_ij)^(alp/3)} (the last two feed the ATM
+// term, atm.f90:667-668,811-816).  One block per row i of the system block;
+// rows and columns are laid out in the spatial order of the atoms.
+__device__ __forceinline__ double pow_m8_3(double x);
+
+// With tri the block also writes the row of the three-body records of a
+// system of the pair-sum route (see atm_pairsum_kernel).  With kTwo it also
+// sums the two-body term of such a system, which has one image per pair, where
+// the pair's C6 is at hand (disp2_atom's terms): a separate kernel reads the
+// records again and, for a small molecule, is a launch more (whole calls, FP64:
+// planned batch of 1,024 molecules 2.95 -> 2.78 ms, 1,501-atom energy 0.593 ->
+// 0.562, 200 atoms from host arrays 0.143 -> 0.135).
+enum PairTwoBody { kNoTwoBody, kTwoBodyEnergy, kTwoBodyGrad };
+template <typename R, int kTwo>
+__global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* __restrict__ gw,
+                                                      const double* __restrict__ dgw,
+                                                      const double* __restrict__ gwr, const int* __restrict__ spr,
+                                                      R4<R>* __restrict__ pair, double4* __restrict__ tri,
+                                                      double* __restrict__ e_atom, double* __restrict__ dedcn,
+                                                      double* __restrict__ grad, double* __restrict__ sig_atom) {
+  const int i = blockIdx.x;
+  const int s = b.sys[i];
+  const SysGeom g = b.geom[s];
+  const double alp3 = (b.par[s].alp + 2.0) / 3.0;
+  const int n = g.natoms;
+  const int spi = b.sp[i];
+  const int mref = b.mref;
+  const int nri = b.nref[spi];
+  double gi[kMaxRef], dgi[kMaxRef];
+  for (int r = 0; r < kMaxRef; ++r) {
+    gi[r] = r < nri ? gw[i * mref + r] : 0.0;
+    dgi[r] = (r < nri && dgw) ? dgw[i * mref + r] : 0.0;
+  }
+  // per species s of the batch: h[s][r] = sum_ri w_i[ri] C6ref[ri][r] and the
+  // same with dw_i/dCN_i, so that a record costs three nref_j-term dots; and
+  // (4/3 rvdw_is)^(alp/3), in dynamic LDS ((2 kMaxRef + 1) nsp doubles, sized
+  // at the launch).
+  extern __shared__ double pair_lds[];
+  double* __restrict__ h = pair_lds;                   // [nsp][kMaxRef]
+  double* __restrict__ dh = pair_lds + b.nsp * kMaxRef;  // [nsp][kMaxRef]
+  double* __restrict__ r0p_s = dh + b.nsp * kMaxRef;     // [nsp]
+  for (int t = threadIdx.x; t < b.nsp * kMaxRef; t += blockDim.x) {
+    const int sj = t / kMaxRef, rj = t % kMaxRef;
+    const double* ref = b.c6ref + (spi * b.nsp + sj) * (kMaxRef * kMaxRef);
+    double a = 0.0, d = 0.0;
+    for (int ri = 0; ri < nri; ++ri) {
+      a += gi[ri] * ref[ri * kMaxRef + rj];
+      d += dgi[ri] * ref[ri * kMaxRef + rj];
+    }
+    h[t] = a;
+    dh[t] = d;
+  }
+  for (int t = threadIdx.x; t < b.nsp; t += blockDim.x) r0p_s[t] = pow(kRs9 * b.rvdw[t * b.nsp + spi], alp3);
+  __syncthreads();
+  const bool gi_ghost = b.ghost && b.ghost[i];
+  const int ri = b.rank[i];
+  R4<R>* row = pair + g.c6_begin + static_cast<long long>(ri) * n;
+  double4* tri_row = g.tri_begin >= 0 ? tri + g.tri_begin + static_cast<long long>(ri) * n : nullptr;
+  const double4 xi = b.pos[i];
+  const double cut3 = b.par[s].cut3, width3 = b.par[s].width3;
+  const bool alp14 = b.par[s].alp == 14.0;
+  const long long nat = b.natoms;
+  // two-body sums: e, dE/dCN, gradient, virial
+  constexpr bool kGrad = kTwo == kTwoBodyGrad;
+  constexpr int kSums = kTwo == kNoTwoBody ? 1 : (kGrad ? 11 : 1);
+  double v[kSums] = {0.0};
+  const SysParam& p = b.par[s];
+  const bool two = kTwo != kNoTwoBody && tri_row && two_body_active(p);
+  const double cut2b = p.cut2 * p.cut2;
+  const R r4r2i = R(b.r4r2[spi]);
+  for (int jr = threadIdx.x; jr < n; jr += blockDim.x) {
+    const int x = g.atom_begin + jr;  // position of partner j in the spatial order
+    const int code = spr[x];
+    const int spj = code & (kGhostBit - 1);
+    const int nrj = b.nref[spj];
+    double cc = 0.0, di = 0.0, dj = 0.0;
+    if (!(gi_ghost || (code & kGhostBit))) {  // model.f90:436-440
+      for (int rj = 0; rj < nrj; ++rj) {
+        const double w = gwr[rj * nat + x];
+        cc += w * h[spj * kMaxRef + rj];
+        if (dgw) {
+          di += w * dh[spj * kMaxRef + rj];
+          dj += gwr[(mref + rj) * nat + x] * h[spj * kMaxRef + rj];
+        }
+      }
+    }
+    const double ic = cc > 0.0 ? 1.0 / cc : 0.0;
+    const double sc6 = sqrt(cc);
+    const R4<R> q = make_r4<R>(R(sc6), R(di * ic), R(dj * ic), R(r0p_s[spj]));
+    row[jr] = q;
+    if (!tri_row) continue;
+    if (two) {
+      const int j = b.order[x];
+      const double4 xj = b.posr[x];
+      double u0, u1, u2;
+      const double r2d = pair_vec(xi, xj, make_double4(0.0, 0.0, 0.0, 0.0), j > i, u0, u1, u2);
+      if (!(r2d > cut2b || r2d < kEps)) {
+        const R rrij = R(3) * r4r2i * R(b.r4r2[spj]);
+        const R c6ij = q.x * q.x;
+        const R dc6i = q.y * c6ij;  // dC6_ij/dCN_i
+        const R r2 = R(r2d), r1 = d_sqrt(r2);
+        R sw, dswdr, edisp0, gdisp0 = R(0), dedc6 = R(0);
+        smooth_cutoff(r1, R(p.cut2), R(p.width2), sw, dswdr);
+        auto term = [&](auto kind) {
+          constexpr int kKind = decltype(kind)::value;
+          const DampPair<R> dp =
+              damp_setup<R, kKind>(p, rrij, b.rvdw[spj * b.nsp + spi], c6ij, b.sid[i] + b.sid[j]);
+          edisp0 = damp_term<R, kGrad, kKind>(p, dp, r2, r1, gdisp0, dedc6);
+        };
+        switch (p.kind) {
+          case kRational: term(std::integral_constant<int, kRational>{}); break;
+          case kZero: term(std::integral_constant<int, kZero>{}); break;
+          case kModifiedZero: term(std::integral_constant<int, kModifiedZero>{}); break;
+          case kOptimizedPower: term(std::integral_constant<int, kOptimizedPower>{}); break;
+          case kCSO: term(std::integral_constant<int, kCSO>{}); break;
+          default: term(std::integral_constant<int, kZDamping>{}); break;
+        }
+        const R edisp = sw * edisp0;
+        v[0] += double(-c6ij * edisp * R(0.5));
+        if constexpr (kGrad) {
+          const R gdisp = sw * gdisp0 + dswdr * edisp0 / r1;
+          const R f = -c6ij * gdisp;  // dG = f * vec
+          v[1] -= double(p.kind == kZDamping ? dc6i * sw * dedc6 : dc6i * edisp);
+          const R w0 = R(u0), w1 = R(u1), w2 = R(u2);
+          v[2] += double(f * w0); v[3] += double(f * w1); v[4] += double(f * w2);
+          const R h2 = R(0.5) * f;  // dS = 0.5 dG (x) vec
+          v[5] += double(h2 * w0 * w0); v[6] += double(h2 * w1 * w1); v[7] += double(h2 * w2 * w2);
+          v[8] += double(h2 * w0 * w1); v[9] += double(h2 * w0 * w2); v[10] += double(h2 * w1 * w2);
+        }
+      }
+    }
+    double4 t = make_double4(1.0, 0.0, 0.0, 0.0);  // no pair: no term
+    double d0, d1, d2;
+    const double r2 = atm_vec(b.posr[x], make_double4(0.0, 0.0, 0.0, 0.0), xi, d0, d1, d2);
+    const double cut2 = cut3 * cut3;
+    if (jr != ri && r2 <= cut2 * (1.0 + kBand) && r2 >= kEps && cc >= kEps) {
+      const double r1 = sqrt(r2);
+      double sw, dswdr;
+      smooth_cutoff(r1, cut3, width3, sw, dswdr);
+      t.x = r2;
+      t.y = sw * sc6 / (r2 * r1);
+      t.z = r0p_s[spj] * (alp14 ? pow_m8_3(r2) : pow(r2, -0.5 * alp3));
+      t.w = t.y / r2;
+      if (r2 > cut2 * (1.0 - kBand)) {  // see atm_pairsum_kernel
+        t.z = -t.z;
+        b.band[s] = 1;
+      }
+    }
+    tri_row[jr] = t;
+  }
+  if constexpr (kTwo != kNoTwoBody) {
+    if (!tri_row) return;  // (uniform) disp2_kernel sums this system's term
+    __shared__ double red[kWavesPerBlock][kSums];
+#pragma unroll
+    for (int c = 0; c < kSums; ++c) {
+      v[c] = wave_sum(v[c]);
+      if (wave_lane() == 0) red[threadIdx.x >> 6][c] = v[c];
+    }
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c < kSums) {
+      double t = 0.0;
+      for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) t += red[w][c];
+      if (c == 0) e_atom[i] = t;
+      else if (c == 1) dedcn[i] = t;
+      else if (c < 5) grad[3 * i + c - 2] = t;
+      else sig_atom[6 * i + c - 5] = t;
+    }
+  }
+}
+
 // --------------------------------------------------------------- two-body
 // get_dispersion_derivs of every damping family (rational.f90:378-514,
 // zero.f90:409-553, mzero.f90:361-508, optimizedpower.f90, cso.f90, z.f90),
@@ -785,6 +861,7 @@ void disp2_kernel(DevBatch b, const R4<R>* __restrict__ pair,
   if (i >= b.natoms) return;
   const int s = b.sys[i];
   const SysGeom g = b.geom[s];
+  if (!kPairs && g.tri_begin >= 0) return;  // summed by pair_kernel
   const SysParam p = b.par[s];
   switch (p.kind) {
     case kRational: disp2_atom<R, kGrad, kPairs, kRational>(b, pair, e_atom, dedcn, grad, sig_atom, pair2, i, g, p); break;
@@ -3892,19 +3969,27 @@ void launch_rank_pos(const DevBatch& b, const double* xyz, hipStream_t st) {
                        const_cast<double4*>(b.pos), const_cast<double4*>(b.posr), const_cast<double4*>(b.tbox));
 }
 
-void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, const double* gwr, const int* spr,
-                 void* pair, double4* tri, hipStream_t st) {
+void launch_pair(const DevBatch& b, bool mixed, const DevWork& w, bool two_body, bool grad, hipStream_t st) {
   const size_t lds = sizeof(double) * static_cast<size_t>(b.nsp) * (2 * kMaxRef + 1);  // h, dh, r0p
   // One wavefront per row in large batches of small systems, whose rows do not
   // fill four and whose per-species sums cost as much as the row (1,024
 // molecules, FP64: 680 -> 440 us); else four, for the latency of a row.
   const dim3 blk(b.nsys > 1 && b.natoms >= 4096 && b.natoms / b.nsys <= kBlock ? kWave : kBlock);
-  if (mixed)
-    hipLaunchKernelGGL(pair_kernel<float>, dim3(b.natoms), blk, lds, st, b, gw, dgw, gwr, spr,
-                       static_cast<float4*>(pair), tri);
-  else
-    hipLaunchKernelGGL(pair_kernel<double>, dim3(b.natoms), blk, lds, st, b, gw, dgw, gwr, spr,
-                       static_cast<double4*>(pair), tri);
+  auto launch = [&](auto kernel, auto* pair) {
+    hipLaunchKernelGGL(kernel, dim3(b.natoms), blk, lds, st, b, w.gw, w.dgw, w.gwr, w.spr, pair, w.tri, w.e_atom,
+                       w.dedcn, w.grad, w.sig_atom);
+  };
+  if (mixed) {
+    float4* pair = static_cast<float4*>(w.pair);
+    if (!two_body || !w.tri) launch(pair_kernel<float, kNoTwoBody>, pair);
+    else if (grad) launch(pair_kernel<float, kTwoBodyGrad>, pair);
+    else launch(pair_kernel<float, kTwoBodyEnergy>, pair);
+  } else {
+    double4* pair = static_cast<double4*>(w.pair);
+    if (!two_body || !w.tri) launch(pair_kernel<double, kNoTwoBody>, pair);
+    else if (grad) launch(pair_kernel<double, kTwoBodyGrad>, pair);
+    else launch(pair_kernel<double, kTwoBodyEnergy>, pair);
+  }
 }
 
 template <typename R, bool kGrad, bool kPairs>

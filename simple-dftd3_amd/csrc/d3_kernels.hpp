@@ -93,8 +93,12 @@ void launch_cn(const DevBatch& b, bool mixed, double* cn, double* gw, double* dg
 // xyz, the caller's positions of a batch whose storage order is the atom
 // order, it first packs them into pos.
 void launch_rank_pos(const DevBatch& b, const double* xyz, hipStream_t stream);
-void launch_pair(const DevBatch& b, bool mixed, const double* gw, const double* dgw, const double* gwr, const int* spr,
-                 void* pair, double4* tri, hipStream_t stream);
+// Pair records of every system and (w.tri) the three-body records of the
+// systems of the pair-sum route; with two_body also the two-body term of the
+// latter (energy, and with grad dE/dCN, gradient and virial), written to the
+// accumulators.
+void launch_pair(const DevBatch& b, bool mixed, const DevWork& w, bool two_body, bool grad, hipStream_t stream);
+// The two-body term of the systems that launch_pair leaves out (without pair2).
 // pair2 (energy only, may be null): per system an n x n block (offset
 // c6_begin, atom order) of pairwise two-body energies.
 void launch_disp2(const DevBatch& b, bool mixed, bool grad, const DevWork& w, double* pair2, hipStream_t stream);
