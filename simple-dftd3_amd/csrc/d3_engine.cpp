@@ -378,8 +378,11 @@ int pair_sum_atoms(bool mixed, bool grad) { return mixed && grad ? kPairSumAtoms
 // 8 / 16: 300 atoms 0.155 / 0.158, 500 0.232 / 0.238, 600 (741 tile pairs)
 // 0.321 / 0.291, 1,000 0.80 / 0.67).
 constexpr size_t kPairSumWide = 650;
-// Above this many bytes of records and sums the allocation-free entry point
-// keeps the lists, so that the batches that fit its work area stay the same.
+// Above this many bytes of records and sums a batch keeps the lists, which
+// take less memory (28 or 40 bytes a pair of atoms, the sums 48, the Hessian's
+// 184 more), so that the batches that fit the device stay the same; and with
+// less in the fixed work area of the allocation-free entry point.
+constexpr long long kPairSumBytes = 32LL << 30;
 constexpr long long kPairSumArenaBytes = 16LL << 20;
 
 struct Workspace {
@@ -573,11 +576,11 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   auto pair_sum_route = [&](const SystemDesc& sd) {
     return !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2]) && sd.nparts == 1 && sd.natoms <= max_pair_sum;
   };
-  if (arena) {
+  {
     long long bytes = 0;
     for (const auto& sd : systems)
       if (pair_sum_route(sd)) bytes += static_cast<long long>(sd.natoms) * sd.natoms * (sizeof(double4) + sizeof(double2));
-    if (bytes > kPairSumArenaBytes) max_pair_sum = 0;
+    if (bytes > (arena ? kPairSumArenaBytes : kPairSumBytes)) max_pair_sum = 0;
   }
   bool any_atm = false, smooth = false, periodic_atm = false;
   for (int k = 0, a = 0; k < nsys; ++k) {
@@ -1149,9 +1152,13 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
   // three-body term by pair sums for molecules without a switching width
   // (the visits are the gradient's, three per triple, at any size cheaper than
   // the lists' global atomics)
-  bool smooth = false;
-  for (const auto& sd : systems) smooth = smooth || sd.param.width3 > 0.0;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, smooth ? 0 : kPairSumAtoms);
+  bool lists = false;
+  long long bytes = 0;
+  for (const auto& sd : systems) {
+    lists = lists || sd.param.width3 > 0.0;
+    bytes += static_cast<long long>(sd.natoms) * sd.natoms * static_cast<long long>(sizeof(double) * hess_pairsum_doubles());
+  }
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, lists || bytes > kPairSumBytes ? 0 : kPairSumAtoms);
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   double* e = energy ? energy : m.e_out.as<double>(static_cast<size_t>(db.nsys));
