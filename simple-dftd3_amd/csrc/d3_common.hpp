@@ -67,6 +67,8 @@ struct SysGeom {
   // offset of the system's n x n three-body records (pair-sum route: systems
   // without lattice images up to a size), < 0: three-body lists
   long long tri_begin;
+  // ... and of the rows of DevBatch::reach of its tiles
+  long long reach_begin;
   // 3D-periodic systems: the images of set s (kImgCn, kImg2, kImg3) form the
   // index box |n_d| <= box[s][d] in list order (n_x outer, n_z inner); the
   // rows of frac (b_d / 2 pi) give fractional coordinates and span[s][d] =

@@ -371,7 +371,11 @@ AtmShape per_call_shape(bool mixed, bool periodic, long long items) {
 // 3.91, 3,000 6.67 / 7.75, 4,000 12.6 / 12.5; FP64 energy: 1,000 0.31 / 0.78,
 // 4,000 4.83 / 8.56; mixed gradient: 1,000 0.62 / 0.91, 1,500 1.40 / 1.56,
 // 2,000 2.6 / 2.6 (a sphere 3.1 / 3.0); mixed energy: 4,000 4.75 / 4.88.
+// Extended molecules cost less on both sides; FP64 gradient of 3,500 atoms: a
+// wire of 2 x 2 atoms 0.45 / 0.52, a sheet of one layer 0.84 / 0.90, of three
+// layers 1.99 / 2.46.
 constexpr int kPairSumAtoms = 3500, kPairSumAtomsMixedGrad = 1750;
+static_assert(kPairSumAtoms <= 64 * kTile, "a bit per tile of 64 positions (pair_kernel, atm_pairsum_kernel)");
 int pair_sum_atoms(bool mixed, bool grad) { return mixed && grad ? kPairSumAtomsMixedGrad : kPairSumAtoms; }
 // Tiles of 16 positions a side from this many tile pairs of the batch on, else
 // of 8, which spread a small batch over more wavefronts (gradient, ms, tiles of
@@ -387,7 +391,7 @@ constexpr long long kPairSumArenaBytes = 16LL << 20;
 
 struct Workspace {
   DeviceBuffer meta, pos, rank, order, sort_tmp, cn, gw, dgw, pair, e_atom, dedcn, grad, sig, atm_acc, cnt, off,
-      item_off, items, slots, tri, psum, band, gw_rank, sp_rank, pos_rank, tbox, counts, counter, flag, pair3s, hbuf, e_out, ew_tab, ew_c6l, ew_lc6l, ew_ldc6l, ew_part,
+      item_off, items, slots, tri, psum, band, reach, gw_rank, sp_rank, pos_rank, tbox, counts, counter, flag, pair3s, hbuf, e_out, ew_tab, ew_c6l, ew_lc6l, ew_ldc6l, ew_part,
       ew_phi, ew_f, ew_s, sp_base, sp_theta, sp_dtheta, sp_q, sp_qh, sp_th, sp_k, sp_dm, sp_dmir;
   // batched real <-> half-complex 3D transforms of the particle mesh (one per
   // species), kept while the mesh and the species count stay the same
@@ -424,7 +428,7 @@ struct Workspace {
   Arena* arena = nullptr;
   std::vector<DeviceBuffer*> buffers() {
     return {&meta, &pos, &rank, &order, &sort_tmp, &cn, &gw, &dgw, &pair, &e_atom, &dedcn, &grad, &sig, &atm_acc, &cnt, &off,
-            &item_off, &items, &slots, &tri, &psum, &band, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
+            &item_off, &items, &slots, &tri, &psum, &band, &reach, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
             &e_out, &ew_tab, &ew_c6l, &ew_lc6l, &ew_ldc6l, &ew_part, &ew_phi, &ew_f, &ew_s, &sp_base, &sp_theta,
             &sp_dtheta, &sp_q, &sp_qh, &sp_th, &sp_k, &sp_dm, &sp_dmir};
   }
@@ -618,6 +622,7 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
     // tile is usually within the cutoffs and the box tests only cost)
     g.cull = !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2]) && sd.natoms > 8 * kTile;
     g.tri_begin = -1;
+    g.reach_begin = 0;
     for (int t = 0; t * kTile < sd.natoms; ++t)
       tiles.push_back(make_int2(g.atom_begin + t * kTile, std::min(kTile, sd.natoms - t * kTile)));
     if (std::fabs(sd.param.s9) >= kEps) {
@@ -646,6 +651,7 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   }
   // Tile pairs of the pair-sum route, the largest systems (the longest sums) first
   std::vector<int2> ps_items;
+  long long reach_words = 0;
   if (!ps_systems.empty()) {
     std::stable_sort(ps_systems.begin(), ps_systems.end(),
                      [&](int x, int y) { return systems[x].natoms > systems[y].natoms; });
@@ -661,6 +667,8 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
     ps_items.reserve(tile_pairs(pb.ps.side));
     for (int k : ps_systems) {
       const int t = (systems[k].natoms + pb.ps.side - 1) / pb.ps.side;
+      geom[k].reach_begin = reach_words;
+      reach_words += static_cast<long long>(t) * ((systems[k].natoms + kTile - 1) / kTile);
       for (int I = 0; I < t; ++I)
         for (int J = I; J < t; ++J) ps_items.push_back(make_int2(k, I | J << 16));
     }
@@ -793,6 +801,8 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   db.tiles = reinterpret_cast<const int2*>(dmeta + o_ptiles);
   db.tbox = tbox.as<double4>(2 * tiles.size());
   db.band = pb.ps.count > 0 ? band.as<int>(nsys) : nullptr;
+  db.reach = pb.ps.count > 0 ? reach.as<unsigned long long>(reach_words) : nullptr;
+  db.reach_shift = pb.ps.side == 16 ? 4 : 3;
   pb.ps.items = reinterpret_cast<const int2*>(dmeta + o_ps);
   pb.pair_total = pair_total;
   pb.any_atm = any_atm;

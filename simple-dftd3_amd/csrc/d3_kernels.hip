@@ -185,6 +185,12 @@ __device__ __attribute__((noinline)) bool triple_in_range(const double4* __restr
   return rp <= cut2 && rp >= kEps && rq <= cut2 && rq >= kEps && rd <= cut2 && rd >= kEps;
 }
 
+// The row of DevBatch::reach of a tile of a system of the pair-sum route.
+__device__ __forceinline__ int reach_words(const SysGeom& g) { return (g.natoms + kWave - 1) / kWave; }
+__device__ __forceinline__ unsigned long long* reach_row(const DevBatch& b, const SysGeom& g, int tile) {
+  return b.reach + g.reach_begin + static_cast<long long>(tile) * reach_words(g);
+}
+
 // cutoff.f90:73-99 smooth_cutoff
 template <typename R>
 __device__ __forceinline__ void smooth_cutoff(R r, R cutoff, R width, R& sw, R& dswdr) {
@@ -335,6 +341,9 @@ __global__ __launch_bounds__(kBlock) void cn_kernel(DevBatch b, double* __restri
     cn[i] = acc;
     if (b.band && i == g.atom_begin) b.band[s] = 0;
   }
+  // pair_kernel sets the bits of the pair-sum route's reach
+  if (g.tri_begin >= 0 && (b.rank[i] & ((1 << b.reach_shift) - 1)) == 0)
+    for (int t = lane; t < reach_words(g); t += kWave) reach_row(b, g, b.rank[i] >> b.reach_shift)[t] = 0ull;
   static_assert(kMaxRef <= 8, "one reference per lane of a group of 8");
   constexpr double wf = 4.0, wf2 = 2.0 * wf;
   const int spi = b.sp[i], nr = b.nref[spi], r = lane & 7;
@@ -577,10 +586,15 @@ __device__ __forceinline__ double pow_m8_3(double x);
 // the pair's C6 is at hand (disp2_atom's terms): a separate kernel reads the
 // records again and, for a small molecule, is a launch more (whole calls, FP64:
 // planned batch of 1,024 molecules 2.95 -> 2.78 ms, 1,501-atom energy 0.593 ->
-// 0.562, 200 atoms from host arrays 0.143 -> 0.135).
+// 0.562, 200 atoms from host arrays 0.143 -> 0.135).  In molecules of more than
+// 8 tiles it leaves out the tiles beyond both cutoffs, whose three-body records
+// are then not written; DevBatch::reach keeps them from being read.  Three
+// wavefronts per SIMD with the gradient (at two, as the compiler took without
+// the hint, the FP64 instantiation has 171 registers; at three 168 and 12 bytes
+// of scratch).
 enum PairTwoBody { kNoTwoBody, kTwoBodyEnergy, kTwoBodyGrad };
 template <typename R, int kTwo>
-__global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* __restrict__ gw,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kTwo == kNoTwoBody ? 4 : 3))) void pair_kernel(DevBatch b, const double* __restrict__ gw,
                                                       const double* __restrict__ dgw,
                                                       const double* __restrict__ gwr, const int* __restrict__ spr,
                                                       R4<R>* __restrict__ pair, double4* __restrict__ tri,
@@ -636,6 +650,10 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* 
   const bool two = kTwo != kNoTwoBody && tri_row && two_body_active(p);
   const double cut2b = p.cut2 * p.cut2;
   const R r4r2i = R(b.r4r2[spi]);
+  // the tiles within the cutoffs (a bit each: this route ends at 64 tiles);
+  // beyond them there is no two-body term, and no record that is read
+  unsigned long long near = ~0ull;
+  if (tri_row) near = near_tiles(b, g, 0, xi, fmax(two ? cut2b : 0.0, cut3 * cut3 * (1.0 + kBand)));
   for (int jr = threadIdx.x; jr < n; jr += blockDim.x) {
     const int x = g.atom_begin + jr;  // position of partner j in the spatial order
     const int code = spr[x];
@@ -656,7 +674,7 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* 
     const double sc6 = sqrt(cc);
     const R4<R> q = make_r4<R>(R(sc6), R(di * ic), R(dj * ic), R(r0p_s[spj]));
     row[jr] = q;
-    if (!tri_row) continue;
+    if (!tri_row || !(near >> (jr >> 6) & 1ull)) continue;  // (uniform in the wavefront)
     if (two) {
       const int j = b.order[x];
       const double4 xj = b.posr[x];
@@ -715,6 +733,8 @@ __global__ __launch_bounds__(kBlock) void pair_kernel(DevBatch b, const double* 
       }
     }
     tri_row[jr] = t;
+    const unsigned long long partners = __ballot(t.y != 0.0);
+    if (partners && wave_lane() == 0) atomicOr(reach_row(b, g, ri >> b.reach_shift) + (jr >> 6), partners);
   }
   if constexpr (kTwo != kNoTwoBody) {
     if (!tri_row) return;  // (uniform) disp2_kernel sums this system's term
@@ -1893,9 +1913,16 @@ __global__ __launch_bounds__(kWave) void atm_pairs_kernel(DevBatch b, const long
 // A block owns a tile of (8 kT)^2 pairs, kT x kT per lane; its wavefronts
 // take the chunks of kC atoms c in turn, and their sums meet in the LDS.  The
 // records (c, a-tile) and (c, b-tile) of a chunk are 4 KB, staged by each
-// wavefront for itself one chunk ahead; atoms c beyond the cutoff of all of
-// a-tile or all of b-tile are skipped (their h are all zero).  The lists of
-// such systems spent most of their time on the distance tests, the LDS
+// wavefront for itself one chunk ahead.  Only atoms c with a record with both
+// tiles are visited, chunks without one are not fetched, and tile pairs
+// without a record end at once; pair_kernel leaves the bits of who has a
+// record with whom (DevBatch::reach).  Fetching every chunk to see so cost
+// extended molecules, and cutoffs shorter than the molecule, more than the
+// lists had (FP64 gradient of 3,500 atoms, this kernel: wire of 2 x 2 atoms
+// 715 -> 87 us, sheet of one layer 2,046 -> 435, cube with a cutoff of 12 bohr
+// 1,659 -> 180; whole calls 1,207 -> 446, 2,579 -> 841, 2,323 -> 850, by lists
+// 520, 895, 913).  The lists of compact
+// systems spent most of their time on the distance tests, the LDS
 // atomics and the gathers: 1,501-atom molecule, FP64 energy, whole call 1.82
 // -> 0.64 ms; planned batch of 1,024 molecules, FP64 gradient, 5.75 -> 3.30;
 // 200-atom molecule from host arrays 0.24 -> 0.17; the kernel is bound by
@@ -1927,12 +1954,22 @@ void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items, const double
   const double4* __restrict__ rec = tri + g.tri_begin;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = wave_lane();
   const int la = l >> 3, lb = l & 7;
+  const unsigned long long* __restrict__ reach_a = reach_row(b, g, I);
+  const unsigned long long* __restrict__ reach_b = reach_row(b, g, J);
+  // the atoms of the a-tile with a record with one of the b-tile, and the other way round
+  auto tile_bits = [](const unsigned long long* reach, int tile) {
+    return static_cast<unsigned>(reach[tile * kSide / kWave] >> (tile * kSide % kWave)) & ((1u << kSide) - 1u);
+  };
+  const unsigned a_bits = tile_bits(reach_b, I), b_bits = tile_bits(reach_a, J);
+  if (kMode != kPsPairs && (a_bits | b_bits) == 0u) return;  // no pair, and its sums are not read
   double A[kOwn], c38[kOwn], G6[kOwn], S[kOwn], Y[kOwn], Z[kOwn];
   unsigned own = 0;  // bit o: pair o has terms; bit 8 + o: it is near the cutoff
 #pragma unroll
   for (int o = 0; o < kOwn; ++o) {
     const int a = I * kSide + la + 8 * (o / kT), bb = J * kSide + lb + 8 * (o % kT);
-    const double4 q = a < n && bb < n ? rec[static_cast<long long>(a) * n + bb] : make_double4(1.0, 0.0, 0.0, 0.0);
+    const double4 q = bb < n && (a_bits >> (la + 8 * (o / kT)) & 1u)
+                          ? rec[static_cast<long long>(a) * n + bb]
+                          : make_double4(1.0, 0.0, 0.0, 0.0);
     A[o] = q.x;
     c38[o] = 0.375 / q.x;
     G6[o] = 6.0 * fabs(q.z);
@@ -1943,8 +1980,40 @@ void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items, const double
   const bool live = __ballot(own != 0u) != 0ull;
   if (kMode == kPsEnergy && !live) return;
 
-  const int nchunks = (n + kC - 1) / kC;
-  int ch = (kMode == kPsEnergy ? J * (kSide / kC) : 0) + w;
+  // The third atoms: those with a record with the a-tile and one with the
+  // b-tile, lane t holding the bits of positions 64 t .. 64 t + 63, of which
+  // this wavefront takes every fourth chunk.
+  constexpr unsigned long long kChunkBits = (1ull << kC) - 1ull;
+  unsigned long long third = 0;
+  if (l < reach_words(g)) {
+    third = reach_a[l] & reach_b[l];
+    if (kMode == kPsEnergy) {  // c > b
+      const int d = J * kSide - kWave * l;
+      third = d >= kWave ? 0ull : d > 0 ? third >> d << d : third;
+    }
+  }
+  {
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int k = 0; k < kWave; k += kC * kWavesPerBlock) mine |= kChunkBits << k;
+    third &= mine << (kC * w);
+  }
+  unsigned long long words = __ballot(third != 0ull), word = 0;
+  int word_at = 0;
+  // the next chunk of this wavefront (-1: none), its atoms with a term in act
+  auto next = [&](unsigned& act) {
+    if (!word) {
+      if (!words) return -1;
+      word_at = __builtin_ctzll(words);
+      words &= words - 1;
+      word = static_cast<unsigned long long>(__builtin_amdgcn_readlane(static_cast<int>(third >> 32), word_at)) << 32 |
+             static_cast<unsigned>(__builtin_amdgcn_readlane(static_cast<int>(third), word_at));
+    }
+    const int k = __builtin_ctzll(word) / kC;
+    act = static_cast<unsigned>(word >> (kC * k) & kChunkBits);
+    word &= ~(kChunkBits << (kC * k));
+    return word_at * (kWave / kC) + k;
+  };
   // 16-byte unit u = 64 k + l of a chunk: atom c = u / (2 kRecs), record
   // r = u / 2 mod kRecs (a-tile, then b-tile), half u mod 2
   double2 pre[4];
@@ -1961,22 +2030,16 @@ void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items, const double
   auto run = [&](auto banded) {
     constexpr bool kBanded = decltype(banded)::value;
     int buf = 0;
-    if (ch < nchunks) fetch(ch);
-    for (; ch < nchunks; ch += kWavesPerBlock, buf ^= 1) {
-      unsigned act = 0;  // atoms of the chunk with a term
+    unsigned act_next = 0;
+    int ch = next(act_next);
+    if (ch >= 0) fetch(ch);
+    for (; ch >= 0; buf ^= 1) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        stage[w][buf][kWave * k + l] = pre[k];
-        const unsigned long long nz = __ballot((l & 1) == 0 && pre[k].y != 0.0);
-        if (kT == 2) {
-          if ((nz & 0xffffffffull) && (nz >> 32)) act |= 1u << k;
-        } else {
-          if ((nz & 0xffffull) && (nz & 0xffff0000ull)) act |= 1u << (2 * k);
-          if (((nz >> 32) & 0xffffull) && (nz >> 48)) act |= 2u << (2 * k);
-        }
-      }
+      for (int k = 0; k < 4; ++k) stage[w][buf][kWave * k + l] = pre[k];
       const int chunk = ch;
-      if (ch + kWavesPerBlock < nchunks) fetch(ch + kWavesPerBlock);
+      unsigned act = act_next;  // atoms of the chunk with a term
+      ch = next(act_next);
+      if (ch >= 0) fetch(ch);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
       // energy: c > b within the b-tile
@@ -2101,7 +2164,11 @@ __global__ __launch_bounds__(kBlock) void pair_sum_finish_kernel(DevBatch b, con
   const double4 xi = b.pos[i];
   const bool smooth = p.width3 > 0.0;
   double v[11] = {0.0};
-  for (int x = wave_lane(); x < n; x += kWave) {
+  // (the sums of a pair of tiles without a record are not there)
+  const unsigned long long* __restrict__ reach = reach_row(b, g, b.rank[i] >> b.reach_shift);
+  for (int t = 0; t < reach_words(g); ++t) {
+    if (!(reach[t] >> wave_lane() & 1ull)) continue;
+    const int x = t * kWave + wave_lane();
     const double2 q = psum[g.tri_begin + row + x];
     const double qi = double(pair[g.c6_begin + row + x].y);
     const double4 xj = b.posr[g.atom_begin + x];

@@ -41,6 +41,11 @@ struct DevBatch {
   int rank_own;         // large molecules: three-body lists by storage order (energy evaluations)
   const int2* tiles;    // [ntiles] first position and count of each 64-position tile of that order
   int* band;            // [nsys] a pair of the system is within kBand of the three-body cutoff (pair-sum route)
+  // Pair-sum route: per tile of 2^reach_shift positions of a system's spatial
+  // order (rows from SysGeom::reach_begin) a bit per position, in 64-bit
+  // words: some atom of the tile has a three-body record with it.
+  unsigned long long* reach;
+  int reach_shift;
   const double4* tbox;  // [2 ntiles] lower and upper corner of each tile's positions (refreshed with pos)
 };
 
