@@ -362,21 +362,51 @@ AtmShape per_call_shape(bool mixed, bool periodic, long long items) {
 }
 
 // Three-body term by pair sums instead of lists: whole molecules (no lattice
-// images, no work partition) up to this many atoms.  The pair sums visit every
-// triple of atoms, three times with the gradient, at a third to a fifth of the
-// lists' cost a visit; the lists only the triples within the cutoff, so they
-// win once most atoms of a molecule are out of each other's range.  Ellipsoids
-// 1:1:2 at 0.1 atoms per cubic Angstrom, whole evaluations, ms, pair sums /
-// lists; FP64 gradient: 500 atoms 0.23 / 0.44, 1,000 0.64 / 1.08, 2,000 2.57 /
-// 3.91, 3,000 6.67 / 7.75, 4,000 12.6 / 12.5; FP64 energy: 1,000 0.31 / 0.78,
-// 4,000 4.83 / 8.56; mixed gradient: 1,000 0.62 / 0.91, 1,500 1.40 / 1.56,
-// 2,000 2.6 / 2.6 (a sphere 3.1 / 3.0); mixed energy: 4,000 4.75 / 4.88.
-// Extended molecules cost less on both sides; FP64 gradient of 3,500 atoms: a
-// wire of 2 x 2 atoms 0.45 / 0.52, a sheet of one layer 0.84 / 0.90, of three
-// layers 1.99 / 2.46.
+// images, no work partition) up to a number of atoms.  The pair sums visit
+// every triple of atoms within each other's range, three times with the
+// gradient, at a third to a fifth of the lists' cost a visit, and a few
+// beyond it; the lists visit each triple once.
+//
+// kPairSumAtoms: ellipsoids 1:1:2 at 0.1 atoms per cubic Angstrom, whole
+// evaluations, ms, pair sums / lists; FP64 gradient: 500 atoms 0.23 / 0.44,
+// 1,000 0.64 / 1.08, 2,000 2.57 / 3.91, 3,000 6.67 / 7.75, 4,000 12.6 / 12.5;
+// FP64 energy: 1,000 0.31 / 0.78, 4,000 4.83 / 8.56; mixed gradient: 1,000
+// 0.62 / 0.91, 1,500 1.40 / 1.56, 2,000 2.6 / 2.6 (a sphere 3.1 / 3.0); mixed
+// energy: 4,000 4.75 / 4.88.  Extended molecules cost less on both sides; FP64
+// gradient of 3,500 atoms: a wire of 2 x 2 atoms 0.45 / 0.52, a sheet of one
+// layer 0.84 / 0.90, of three layers 1.99 / 2.46.
 constexpr int kPairSumAtoms = 3500, kPairSumAtomsMixedGrad = 1750;
 static_assert(kPairSumAtoms <= 64 * kTile, "a bit per tile of 64 positions (pair_kernel, atm_pairsum_kernel)");
-int pair_sum_atoms(bool mixed, bool grad) { return mixed && grad ? kPairSumAtomsMixedGrad : kPairSumAtoms; }
+// With a three-body cutoff shorter than a molecule, fewer of the atoms that a
+// pair of tiles visits are in range of each pair: in batches of more than
+// kPairSumLatency atoms the gradient takes the pair sums only up to this many
+// atoms per cubed cutoff (the atoms within the cutoff are some 0.06 of it, in
+// bohr, at that density), and always up to kPairSumSmall atoms.  Cubes of n
+// atoms, 0.1 per cubic Angstrom, 30,000 atoms a batch, ms, pair sums / lists;
+// mixed gradient, 12 bohr: 200 atoms 0.76 / 0.96, 300 1.66 / 1.47; 20 bohr: 300
+// 2.44 / 2.39, 500 3.35 / 2.87; 26 bohr: 300 2.83 / 3.73, 1,000 7.54 / 6.17;
+// FP64 gradient, 16 bohr: 500 2.53 / 2.54, 1,000 2.94 / 2.84; 20 bohr: 500 3.47 /
+// 3.80, 1,000 4.48 / 4.22, 1,700 4.54 / 3.90; 26 bohr: 1,000 7.73 / 8.12, 1,700
+// 8.25 / 7.97.  In small batches the launches and waits of the lists weigh
+// more: one molecule of 1,700 atoms, FP64, 12 bohr 0.32 / 0.38, mixed, 20 bohr
+// 0.55 / 0.55; of 3,500 atoms, FP64, 12 bohr 0.85 / 0.95.  Energies are faster
+// by pair sums at every cutoff.
+constexpr double kPairSumPerCut3 = 0.0875, kPairSumPerCut3Mixed = 0.031;
+constexpr int kPairSumSmall = 500, kPairSumSmallMixed = 250;
+constexpr int kPairSumLatency = 4096;
+
+// Molecules of up to `atoms` atoms, and in larger batches of up to
+// max(small, per_cut3 cut3^3).
+struct PairSumRule {
+  int atoms = 0;  // 0: lists only
+  double per_cut3 = std::numeric_limits<double>::infinity();
+  int small = 0;
+};
+PairSumRule pair_sum_rule(bool mixed, bool grad) {
+  if (!grad) return {kPairSumAtoms};
+  return mixed ? PairSumRule{kPairSumAtomsMixedGrad, kPairSumPerCut3Mixed, kPairSumSmallMixed}
+               : PairSumRule{kPairSumAtoms, kPairSumPerCut3, kPairSumSmall};
+}
 // Tiles of 16 positions a side from this many tile pairs of the batch on, else
 // of 8, which spread a small batch over more wavefronts (gradient, ms, tiles of
 // 8 / 16: 300 atoms 0.155 / 0.158, 500 0.232 / 0.238, 600 (741 tile pairs)
@@ -452,9 +482,9 @@ struct Workspace {
   // Host planning of a batch: species of the batch, per-species tables,
   // lattice images per system and cutoff, pair-block offsets; one metadata
   // upload (stream-ordered).
-  // Molecules of up to max_pair_sum atoms take the pair-sum route.
+  // rule: the molecules that take the pair-sum route.
   Prepared upload(const std::vector<SystemDesc>& systems, const int* numbers, hipStream_t stream,
-                  const int* ghost_host, int max_pair_sum);
+                  const int* ghost_host, PairSumRule rule);
   // Packs the positions; with order_atoms also (re)computes the spatial order
   // of the atoms (the storage order of pair records and three-body lists).
   void pack(const Prepared& pb, const double* positions_dev, hipStream_t stream, bool order_atoms) {
@@ -495,7 +525,7 @@ void Engine::set_kernel_timing(bool enable) {
 std::pair<double, long long> Engine::kernel_time(const std::string& name) const { return ws_->timer.get(name); }
 
 Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* numbers, hipStream_t stream,
-                           const int* ghost_host, int max_pair_sum) {
+                           const int* ghost_host, PairSumRule rule) {
   Prepared pb;
   const int nsys = static_cast<int>(systems.size());
   int natoms = 0;
@@ -578,13 +608,16 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   long long pair_total = 0, slot_bound = 0, item_bound = 0, atm_atoms = 0;
   std::vector<int> ps_systems;  // pair-sum route
   auto pair_sum_route = [&](const SystemDesc& sd) {
-    return !(sd.periodic[0] || sd.periodic[1] || sd.periodic[2]) && sd.nparts == 1 && sd.natoms <= max_pair_sum;
+    if (sd.periodic[0] || sd.periodic[1] || sd.periodic[2] || sd.nparts != 1 || sd.natoms > rule.atoms) return false;
+    if (natoms <= kPairSumLatency || sd.natoms <= rule.small) return true;
+    const double c = sd.param.cut3;
+    return sd.natoms <= rule.per_cut3 * c * c * c;
   };
   {
     long long bytes = 0;
     for (const auto& sd : systems)
       if (pair_sum_route(sd)) bytes += static_cast<long long>(sd.natoms) * sd.natoms * (sizeof(double4) + sizeof(double2));
-    if (bytes > (arena ? kPairSumArenaBytes : kPairSumBytes)) max_pair_sum = 0;
+    if (bytes > (arena ? kPairSumArenaBytes : kPairSumBytes)) rule = PairSumRule{};
   }
   bool any_atm = false, smooth = false, periodic_atm = false;
   for (int k = 0, a = 0; k < nsys; ++k) {
@@ -1038,7 +1071,7 @@ void Engine::run(const std::vector<SystemDesc>& systems, const int* numbers, con
   Workspace& m = *ws_;
   const bool grad = out.gradient || out.sigma;
   const Prepared pb = m.upload(systems, numbers, stream, ghost_host,
-                               stats ? 0 : pair_sum_atoms(precision == kMixed, grad));
+                               stats ? PairSumRule{} : pair_sum_rule(precision == kMixed, grad));
   m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, out, debug, stats, -1, 0, kPerCallShape,
              stream);
   if (m.timer.enabled) m.timer.collect();
@@ -1074,18 +1107,18 @@ void run_noalloc(const std::vector<SystemDesc>& systems, const int* numbers, con
   BatchOutput inner = out;
   inner.gradient = nullptr;
   Prepared pb;
-  auto attempt = [&](int max_pair_sum) {
+  auto attempt = [&](const PairSumRule& rule) {
     m.reset_arena();
-    pb = m.upload(systems, numbers, stream, nullptr, max_pair_sum);
+    pb = m.upload(systems, numbers, stream, nullptr, rule);
     m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, inner, nullptr, nullptr, -1, 0,
                kPerCallShape, stream);
   };
   // pair sums take 48 bytes a pair of atoms where lists take 40: a batch that
   // only fits with lists gets them
   try {
-    attempt(pair_sum_atoms(precision == kMixed, grad));
+    attempt(pair_sum_rule(precision == kMixed, grad));
   } catch (const ArenaFull&) {
-    attempt(0);
+    attempt(PairSumRule{});
   }
   if (out.gradient)
     hip_check(hipMemcpyAsync(out.gradient, m.grad.as<double>(size_t(pb.db.natoms) * 3),
@@ -1102,10 +1135,10 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
     if (sd.lowrank && sd.periodic[0] && sd.periodic[1] && sd.periodic[2])
       throw Error("Pairwise analysis is only available for the real space summation");
   Workspace& m = *ws_;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, kPairSumAtoms);
+  const bool mixed = precision == kMixed;
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, pair_sum_rule(mixed, false));
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
-  const bool mixed = precision == kMixed;
   m.pack(pb, positions_dev, stream, true);
   const DevWork w = m.work(pb, mixed, false, BatchOutput{}, nullptr);
   m.timed("cn", stream, [&] { launch_cn(db, mixed, w.cn, w.gw, nullptr, w.gwr, w.spr, stream); });
@@ -1168,7 +1201,8 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
     lists = lists || sd.param.width3 > 0.0;
     bytes += static_cast<long long>(sd.natoms) * sd.natoms * static_cast<long long>(sizeof(double) * hess_pairsum_doubles());
   }
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, lists || bytes > kPairSumBytes ? 0 : kPairSumAtoms);
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host,
+                               lists || bytes > kPairSumBytes ? PairSumRule{} : PairSumRule{kPairSumAtoms});
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   double* e = energy ? energy : m.e_out.as<double>(static_cast<size_t>(db.nsys));
@@ -1218,7 +1252,7 @@ void Engine::count_terms(const std::vector<SystemDesc>& systems, const int* numb
   std::vector<SystemDesc> sys = systems;
   for (auto& s : sys)
     if (std::fabs(s.param.s9) < kEps) s.param.s9 = 1.0;  // triples are counted whatever s9 is
-  const Prepared pb = m.upload(sys, numbers, stream, nullptr, 0);
+  const Prepared pb = m.upload(sys, numbers, stream, nullptr, PairSumRule{});
   m.pack(pb, positions_dev, stream, true);
   const int natoms = pb.db.natoms;
   unsigned long long* dc = m.counts.as<unsigned long long>(size_t(pb.db.nsys) * 3);
@@ -1274,7 +1308,7 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
     State& s = *st_;
     s.mixed = precision == kMixed;
     s.grad = grad;
-    s.pb = s.ws.upload(systems, numbers_host, stream, ghost_host, pair_sum_atoms(s.mixed, grad));
+    s.pb = s.ws.upload(systems, numbers_host, stream, ghost_host, pair_sum_rule(s.mixed, grad));
     s.shape.num_cus = device_cu_count();
     const int natoms = s.pb.db.natoms;
     hip_check(hipMemsetAsync(s.ws.flag.as<int>(1), 0, sizeof(int), stream), "hipMemsetAsync");

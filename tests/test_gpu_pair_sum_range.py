@@ -114,3 +114,45 @@ def test_cost_follows_the_range():
         assert calls == 5
         ms.append(total)
     assert ms[0] < 0.05 * ms[1], ms
+
+
+# atoms of a molecule, three-body cutoff, precision, gradient, molecules in the
+# batch, lists: the edges of the rule by the cutoff (0.031 and 0.0875 atoms per
+# cubed cutoff, 250 and 500 atoms, 4,096 atoms a batch)
+ROUTES = [
+    (250, 12.0, "mixed", True, 17, False), (251, 12.0, "mixed", True, 17, True),
+    (251, 12.0, "mixed", True, 16, False), (251, 12.0, "mixed", False, 17, False),
+    (600, 27.0, "mixed", True, 7, False), (600, 26.8, "mixed", True, 7, True),
+    (500, 12.0, "fp64", True, 9, False), (501, 12.0, "fp64", True, 9, True),
+    (501, 12.0, "fp64", False, 9, False), (600, 19.1, "fp64", True, 7, False),
+    (600, 18.9, "fp64", True, 7, True), (600, 12.0, "fp64", True, 6, False),
+]
+
+
+@pytest.mark.parametrize("n,disp3,precision,grad,m,lists", ROUTES)
+def test_short_cutoffs_in_batches(n, disp3, precision, grad, m, lists):
+    """Which route a batch of equal molecules takes, and its results against
+    each molecule alone (pair sums)."""
+    from dftd3 import library, torch_api
+    _step(f"{m} x {n} atoms, cutoff {disp3}, {precision}, grad={grad}")
+    k = int(np.ceil(n ** (1.0 / 3.0)))
+    systems = []
+    for seed in range(m):
+        num, pos = _molecule(seed, n, (k, k, k))
+        systems.append(dict(numbers=num, positions=pos, param=BJ, cutoff=dict(disp3=disp3)))
+    spec, p = torch_api.batch_spec(systems)
+    p = torch.as_tensor(p, dtype=torch.float64, device="cuda").contiguous()
+    ws = library.new_workspace()
+    library.set_kernel_timing(ws, True)
+    out = torch_api.run_batch(spec, p, precision=precision, grad=grad, ws=ws)
+    assert (library.get_kernel_time(ws, "atm_list")[1] > 0) == lists
+    # mixed lists form the three-body term in FP32, the pair sums in FP64
+    mixed = precision == "mixed"
+    for q in (0, m - 1):
+        one = torch_api.get_dispersion_batch([systems[q]], precision=precision, grad=grad)
+        e, er = out["energy"][q].item(), one["energy"][0].item()
+        assert abs(e - er) <= (1e-8 * n if mixed else 1e-10 * abs(er)), (e, er)
+        if grad:
+            g, s = out["gradient"][q * n:(q + 1) * n], out["sigma"][q]
+            assert (g - one["gradient"]).abs().max().item() <= (1e-7 if mixed else 1e-9)
+            assert (s - one["sigma"][0]).abs().max().item() <= (1e-7 * n if mixed else 1e-9)
