@@ -592,9 +592,11 @@ __device__ __forceinline__ double pow_m8_3(double x);
 // wavefronts per SIMD with the gradient (at two, as the compiler took without
 // the hint, the FP64 instantiation has 171 registers; at three 168 and 12 bytes
 // of scratch).
-enum PairTwoBody { kNoTwoBody, kTwoBodyEnergy, kTwoBodyGrad };
+// kRecords, for batches without a system of that route, has none of this: the
+// registers for it cost the records alone 4,500 atoms, mixed, 144 -> 207 us.
+enum PairTwoBody { kRecords, kNoTwoBody, kTwoBodyEnergy, kTwoBodyGrad };
 template <typename R, int kTwo>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kTwo == kNoTwoBody ? 4 : 3))) void pair_kernel(DevBatch b, const double* __restrict__ gw,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kTwo <= kNoTwoBody ? 4 : 3))) void pair_kernel(DevBatch b, const double* __restrict__ gw,
                                                       const double* __restrict__ dgw,
                                                       const double* __restrict__ gwr, const int* __restrict__ spr,
                                                       R4<R>* __restrict__ pair, double4* __restrict__ tri,
@@ -637,17 +639,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kTwo == 
   const bool gi_ghost = b.ghost && b.ghost[i];
   const int ri = b.rank[i];
   R4<R>* row = pair + g.c6_begin + static_cast<long long>(ri) * n;
-  double4* tri_row = g.tri_begin >= 0 ? tri + g.tri_begin + static_cast<long long>(ri) * n : nullptr;
+  double4* tri_row = kTwo != kRecords && g.tri_begin >= 0 ? tri + g.tri_begin + static_cast<long long>(ri) * n : nullptr;
   const double4 xi = b.pos[i];
   const double cut3 = b.par[s].cut3, width3 = b.par[s].width3;
   const bool alp14 = b.par[s].alp == 14.0;
   const long long nat = b.natoms;
   // two-body sums: e, dE/dCN, gradient, virial
   constexpr bool kGrad = kTwo == kTwoBodyGrad;
-  constexpr int kSums = kTwo == kNoTwoBody ? 1 : (kGrad ? 11 : 1);
+  constexpr int kSums = kGrad ? 11 : 1;
   double v[kSums] = {0.0};
   const SysParam& p = b.par[s];
-  const bool two = kTwo != kNoTwoBody && tri_row && two_body_active(p);
+  const bool two = kTwo > kNoTwoBody && tri_row && two_body_active(p);
   const double cut2b = p.cut2 * p.cut2;
   const R r4r2i = R(b.r4r2[spi]);
   // the tiles within the cutoffs (a bit each: this route ends at 64 tiles);
@@ -736,7 +738,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kTwo == 
     const unsigned long long partners = __ballot(t.y != 0.0);
     if (partners && wave_lane() == 0) atomicOr(reach_row(b, g, ri >> b.reach_shift) + (jr >> 6), partners);
   }
-  if constexpr (kTwo != kNoTwoBody) {
+  if constexpr (kTwo > kNoTwoBody) {
     if (!tri_row) return;  // (uniform) disp2_kernel sums this system's term
     __shared__ double red[kWavesPerBlock][kSums];
 #pragma unroll
@@ -4048,12 +4050,14 @@ void launch_pair(const DevBatch& b, bool mixed, const DevWork& w, bool two_body,
   };
   if (mixed) {
     float4* pair = static_cast<float4*>(w.pair);
-    if (!two_body || !w.tri) launch(pair_kernel<float, kNoTwoBody>, pair);
+    if (!w.tri) launch(pair_kernel<float, kRecords>, pair);
+    else if (!two_body) launch(pair_kernel<float, kNoTwoBody>, pair);
     else if (grad) launch(pair_kernel<float, kTwoBodyGrad>, pair);
     else launch(pair_kernel<float, kTwoBodyEnergy>, pair);
   } else {
     double4* pair = static_cast<double4*>(w.pair);
-    if (!two_body || !w.tri) launch(pair_kernel<double, kNoTwoBody>, pair);
+    if (!w.tri) launch(pair_kernel<double, kRecords>, pair);
+    else if (!two_body) launch(pair_kernel<double, kNoTwoBody>, pair);
     else if (grad) launch(pair_kernel<double, kTwoBodyGrad>, pair);
     else launch(pair_kernel<double, kTwoBodyEnergy>, pair);
   }
