@@ -298,9 +298,12 @@ __global__ void spatial_rank_kernel(DevBatch b, const int* __restrict__ order, i
 // that order, reference-major: gwr[r][x], gwr[mref + r][x] (dw/dCN), and the
 // species with the ghost flag, spr[x].  Kernels of their own for the weights
 // and for that layout were two launches of 3 to 4 us in every evaluation.
+// Bound by the latency of the partners' loads: at four instead of five
+// wavefronts per SIMD (97 registers, FP32) it takes 53 instead of 40 us for a
+// molecule of 4,500 atoms.
 constexpr int kGhostBit = 1 << 20;
 template <typename R>
-__global__ __launch_bounds__(kBlock) void cn_kernel(DevBatch b, double* __restrict__ cn, double* __restrict__ gw,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 5 : 4))) void cn_kernel(DevBatch b, double* __restrict__ cn, double* __restrict__ gw,
                                                     double* __restrict__ dgw, double* __restrict__ gwr,
                                                     int* __restrict__ spr) {
   const int lane = wave_lane();
