@@ -1334,6 +1334,9 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
       // size every buffer now, so that an evaluation allocates nothing
       (void)s.ws.slots.get(std::max<long long>(cap, 1) * slot_record_bytes(s.mixed));
       (void)s.ws.items.as<int2>(std::max<long long>(s.max_items, 1));
+      (void)s.ws.cnt.as<long long>(natoms);
+      (void)s.ws.off.as<long long>(natoms + 1);
+      (void)s.ws.item_off.as<long long>(natoms + 1);
       (void)s.ws.counter.as<unsigned long long>(kXcd * kCounterStride);
     }
     // until set_shape or autotune
