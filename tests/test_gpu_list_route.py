@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import oracle as O
-from helpers import BJ
+from helpers import BJ, ZERO, cell
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +59,110 @@ def test_capture_without_an_evaluation_before(n, shape, disp3, m):
         for v in plan.out.values():
             v.zero_()
         _compare(plan.replay(), 0, 0, ref, n, True, True)
+
+
+def _noalloc(systems, precision, grad):
+    """The allocation-free entry point, which keeps the lists when the records
+    and sums of the pair sums (48 bytes a pair of atoms) exceed 16 MiB."""
+    from dftd3 import library, torch_api
+    assert 48 * sum(len(s["numbers"]) ** 2 for s in systems if "lattice" not in s) > 16 << 20
+    spec, pos = torch_api.batch_spec(systems)
+    p = torch.as_tensor(pos, dtype=torch.float64, device="cuda").contiguous()
+    out = dict(energy=torch.empty(len(spec), dtype=torch.float64, device="cuda"),
+               gradient=torch.empty(len(pos), 3, dtype=torch.float64, device="cuda"),
+               sigma=torch.empty(len(spec), 3, 3, dtype=torch.float64, device="cuda"))
+    prec = {"fp64": library.PRECISION_FP64, "mixed": library.PRECISION_MIXED}[precision]
+    library.get_dispersion_batch_noalloc(
+        spec.natoms, spec.numbers, spec.lattices, spec.periodic, spec.params, spec.cutoffs, prec, p.data_ptr(),
+        out["energy"].data_ptr(), out["gradient"].data_ptr() if grad else None,
+        out["sigma"].data_ptr() if grad else None, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("scale", [1.0, 1.0 + 3e-10, 1.0 - 3e-10])
+@pytest.mark.parametrize("k", [4, 54])
+def test_distances_at_the_cutoff(k, scale, precision, grad):
+    """A 10 x 9 x 8 grid of spacing 3 bohr in random order with a three-body
+    cutoff of 3 sqrt(k) bohr, at the cutoff to the last bit, or inside the band
+    that the reference's arithmetic decides, for listed pairs and for the third
+    side of the triples: short lists (4) and a cutoff that most tile pairs are
+    within (54, a distance of 10,144 pairs)."""
+    _step(f"cutoff band, k={k}, scale 1{scale - 1.0:+.0e}, {precision}, grad={grad}")
+    rng = np.random.default_rng(9)
+    g = np.array([[x, y, z] for x in range(10) for y in range(9) for z in range(8)], dtype=float)
+    pos = 3.0 * scale * rng.permutation(g) + np.array([0.1, 0.7, -0.3])
+    cut = 3.0 * np.sqrt(float(k))
+    s = dict(numbers=rng.choice([1, 6], size=len(pos)), positions=pos, param=BJ, cutoff=dict(disp3=cut))
+    _compare(_noalloc([s], precision, grad), 0, 0, _reference(s, grad), len(pos), precision == "mixed", grad)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n,kind,alp,width3", [(640, "rational", 14.0, 0.0), (641, "zero", 14.0, 8.0),
+                                               (703, "rational", 16.0, 0.0)])
+def test_long_lists_among_others(n, kind, alp, width3, precision, grad):
+    """One large molecule (whole tiles, one atom past them, a ragged last
+    tile) with a small molecule and a cell, whose lists keep the reference's
+    triangle."""
+    _step(f"{n} atoms {kind} alp={alp} width3={width3} {precision} grad={grad}")
+    num, pos = _molecule(n, n, (9, 9, 9))
+    cutoff = dict(width3=width3)
+    systems = [dict(numbers=num, positions=pos, param=dict(ZERO if kind == "zero" else BJ, alp=alp), kind=kind,
+                    cutoff=cutoff)]
+    num, pos = _molecule(3, 30, (4, 4, 4))
+    systems.append(dict(numbers=num, positions=pos, param=BJ, cutoff=cutoff))
+    num, pos, lat = cell(17, 12, 13.0)
+    systems.append(dict(numbers=num, positions=pos, lattice=lat, periodic=[True] * 3, param=BJ, cutoff=cutoff))
+    out, off = _noalloc(systems, precision, grad), 0
+    for k, s in enumerate(systems):
+        _compare(out, off, k, _reference(s, grad), len(s["numbers"]), precision == "mixed", grad)
+        off += len(s["numbers"])
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n,shape,cutoff", [(640, (4, 4, 40), dict(disp3=20.0, disp2=30.0)),
+                                            (611, (1, 25, 25), dict(disp3=15.0, disp2=12.0, width3=4.0)),
+                                            (777, (1, 1, 777), dict())])
+def test_tile_culling(n, shape, cutoff, precision, grad):
+    """Molecules longer than the cutoffs: tiles out of range in the loops of
+    the lists and of the two-body term, tile pairs mostly out of range."""
+    _step(f"{n} atoms {shape} {cutoff} {precision} grad={grad}")
+    num, pos = _molecule(n, n, shape)
+    s = dict(numbers=num, positions=pos, param=BJ, cutoff=cutoff)
+    _compare(_noalloc([s], precision, grad), 0, 0, _reference(s, grad), n, precision == "mixed", grad)
+
+
+@pytest.mark.parametrize("n,shape,disp3,runs", [(1751, (13, 13, 11), 40.0, [("mixed", True)]),
+                                                (3501, (16, 16, 14), 24.0, [("fp64", True), ("fp64", False),
+                                                                            ("mixed", False)])])
+def test_every_launch_shape(n, shape, disp3, runs):
+    """Every launch shape of the kernels with the dense form, through plans
+    above the sizes of the pair sums, and graph replays of the last."""
+    from dftd3 import library, torch_api
+    num, pos = _molecule(n, n, shape)
+    s = dict(numbers=num, positions=pos, param=BJ, cutoff=dict(disp3=disp3))
+    ref = _reference(s)
+    spec, p = torch_api.batch_spec([s])
+    p = torch.as_tensor(p, dtype=torch.float64, device="cuda").contiguous()
+    for precision, grad in runs:
+        ws = library.new_workspace()
+        library.set_kernel_timing(ws, True)
+        _compare(torch_api.run_batch(spec, p, precision=precision, grad=grad, ws=ws), 0, 0, ref, n,
+                 precision == "mixed", grad)
+        assert library.get_kernel_time(ws, "atm_list")[1] > 0
+        plan = torch_api.BatchPlan(spec, p, precision=precision, grad=grad)
+        for waves, bpc in library.plan_candidate_shapes():
+            _step(f"{n} atoms {precision} grad={grad} waves={waves} blocks/CU={bpc}")
+            plan.set_shape(waves, bpc)
+            out = {k: torch.zeros_like(v) for k, v in plan.out.items()}
+            _compare(plan.execute(out=out), 0, 0, ref, n, precision == "mixed", grad)
+        plan.capture()
+        for _ in range(3):
+            for v in plan.out.values():
+                v.zero_()
+            _compare(plan.replay(), 0, 0, ref, n, precision == "mixed", grad)
+        assert not plan.overflowed()
