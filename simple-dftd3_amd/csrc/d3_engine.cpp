@@ -456,6 +456,7 @@ struct Workspace {
   // allocation-free mode: every device buffer comes from the arena, the
   // metadata is copied from pageable host memory (no pinned staging)
   Arena* arena = nullptr;
+  bool pair_sums = false;  // the batch uploaded last has systems with pair sums
   std::vector<DeviceBuffer*> buffers() {
     return {&meta, &pos, &rank, &order, &sort_tmp, &cn, &gw, &dgw, &pair, &e_atom, &dedcn, &grad, &sig, &atm_acc, &cnt, &off,
             &item_off, &items, &slots, &tri, &psum, &band, &reach, &gw_rank, &sp_rank, &pos_rank, &tbox, &counts, &counter, &flag, &pair3s, &hbuf,
@@ -682,6 +683,7 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
       }
     }
   }
+  pair_sums = !ps_systems.empty();
   // Tile pairs of the pair-sum route, the largest systems (the longest sums) first
   std::vector<int2> ps_items;
   long long reach_words = 0;
@@ -1118,6 +1120,7 @@ void run_noalloc(const std::vector<SystemDesc>& systems, const int* numbers, con
   try {
     attempt(pair_sum_rule(precision == kMixed, grad));
   } catch (const ArenaFull&) {
+    if (!m.pair_sums) throw;
     attempt(PairSumRule{});
   }
   if (out.gradient)

@@ -61,11 +61,11 @@ def test_capture_without_an_evaluation_before(n, shape, disp3, m):
         _compare(plan.replay(), 0, 0, ref, n, True, True)
 
 
-def _noalloc(systems, precision, grad):
+def _noalloc(systems, precision, grad, lists=True):
     """The allocation-free entry point, which keeps the lists when the records
     and sums of the pair sums (48 bytes a pair of atoms) exceed 16 MiB."""
     from dftd3 import library, torch_api
-    assert 48 * sum(len(s["numbers"]) ** 2 for s in systems if "lattice" not in s) > 16 << 20
+    assert not lists or 48 * sum(len(s["numbers"]) ** 2 for s in systems if "lattice" not in s) > 16 << 20
     spec, pos = torch_api.batch_spec(systems)
     p = torch.as_tensor(pos, dtype=torch.float64, device="cuda").contiguous()
     out = dict(energy=torch.empty(len(spec), dtype=torch.float64, device="cuda"),
@@ -166,3 +166,29 @@ def test_every_launch_shape(n, shape, disp3, runs):
                 v.zero_()
             _compare(plan.replay(), 0, 0, ref, n, precision == "mixed", grad)
         assert not plan.overflowed()
+
+
+def test_work_area_that_holds_the_lists_only():
+    """A molecule and a cell that exceed the work area of the allocation-free
+    entry point (65 MiB) with the records and sums of the molecule's pair sums
+    (48 bytes a pair of atoms) and fit it with lists (72 bytes a slot)."""
+    _step("work area that holds the lists only")
+    n, nc = 590, 310
+    num, pos = _molecule(n, n, (9, 9, 9))
+    cnum, cpos, lat = cell(41, nc, 28.0)
+    img = np.array([[i, j, k] for i in range(-2, 3) for j in range(-2, 3) for k in range(-2, 3)]) @ lat
+    slots = 0
+    for t in img:
+        d2 = ((cpos[None] + t - cpos[:, None]) ** 2).sum(-1)
+        slots += int(np.tril((d2 <= 1600.0) & (d2 > 1e-12)).sum())
+    area, records = 65 << 20, 32 * (n * n + nc * nc)
+    assert 48 * n * n <= 16 << 20
+    assert records + 72 * (slots + n * (n - 1) // 2) + (1 << 20) < area < records + 72 * slots + 48 * n * n, slots
+    systems = [dict(numbers=num, positions=pos, param=BJ),
+               dict(numbers=cnum, positions=cpos, lattice=lat, periodic=[True] * 3, param=BJ)]
+    from dftd3 import torch_api
+    ref = torch_api.get_dispersion_batch(systems, precision="fp64")
+    out = _noalloc(systems, "fp64", True, lists=False)
+    assert ((out["energy"] - ref["energy"]).abs() <= 1e-12 * ref["energy"].abs()).all()
+    for key in ("gradient", "sigma"):
+        assert (out[key] - ref[key]).abs().max() <= 1e-11 * ref[key].abs().max(), key
