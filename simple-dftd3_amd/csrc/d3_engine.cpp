@@ -33,7 +33,9 @@ namespace {
 
 constexpr double kEps = 2.220446049250313e-16;
 
-struct ArenaFull : Error {
+// A device buffer that does not fit the device, or the work area of the
+// allocation-free entry point.
+struct OutOfMemory : Error {
   using Error::Error;
 };
 
@@ -51,8 +53,8 @@ class Arena {
   void* take(size_t bytes) {
     const size_t at = (used_ + 255) / 256 * 256;
     if (at > size_ || bytes > size_ - at)
-      throw ArenaFull("The batch needs more device memory than the fixed work area of the allocation-free entry point (" +
-                      std::to_string(size_ >> 20) + " MiB)");
+      throw OutOfMemory("The batch needs more device memory than the fixed work area of the allocation-free entry point (" +
+                        std::to_string(size_ >> 20) + " MiB)");
     used_ = at + bytes;
     return base_ + at;
   }
@@ -75,12 +77,12 @@ class DeviceBuffer {
     ptr_ = nullptr;
     cap_ = 0;
   }
-  // arena mode: forget the region (the arena is reset by its owner)
+  // Gives the memory back (arena mode: forgets the region, the arena is reset
+  // by its owner).
   void release() {
-    if (arena_) {
-      ptr_ = nullptr;
-      cap_ = 0;
-    }
+    if (ptr_ && !arena_) hip_check(hipFree(ptr_), "hipFree");
+    ptr_ = nullptr;
+    cap_ = 0;
   }
   void* get(size_t bytes) {
     if (bytes > cap_) {
@@ -93,7 +95,13 @@ class DeviceBuffer {
       ptr_ = nullptr;
       cap_ = 0;
       const size_t want = std::max<size_t>(bytes + bytes / 4, 256);
-      hip_check(hipMalloc(&ptr_, want), "hipMalloc");
+      const hipError_t err = hipMalloc(&ptr_, want);
+      if (err != hipSuccess) ptr_ = nullptr;
+      if (err == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // dealt with here, or reported by the exception
+        throw OutOfMemory(std::string("HIP error in hipMalloc: ") + hipGetErrorString(err));
+      }
+      hip_check(err, "hipMalloc");
       cap_ = want;
     }
     return ptr_;
@@ -413,9 +421,10 @@ PairSumRule pair_sum_rule(bool mixed, bool grad) {
 // 0.321 / 0.291, 1,000 0.80 / 0.67).
 constexpr size_t kPairSumWide = 650;
 // Above this many bytes of records and sums a batch keeps the lists, which
-// take less memory (28 or 40 bytes a pair of atoms, the sums 48, the Hessian's
-// 184 more), so that the batches that fit the device stay the same; and with
-// less in the fixed work area of the allocation-free entry point.
+// take less memory (at most 28 or 36 bytes a pair of atoms, the pair sums 48,
+// the Hessian's 184 more), and with less in the fixed work area of the
+// allocation-free entry point.  A batch below that whose records and sums do
+// not fit the free memory takes lists too (Workspace::with_pair_sums).
 constexpr long long kPairSumBytes = 32LL << 30;
 constexpr long long kPairSumArenaBytes = 16LL << 20;
 
@@ -463,6 +472,18 @@ struct Workspace {
             &e_out, &ew_tab, &ew_c6l, &ew_lc6l, &ew_ldc6l, &ew_part, &ew_phi, &ew_f, &ew_s, &sp_base, &sp_theta,
             &sp_dtheta, &sp_q, &sp_qh, &sp_th, &sp_k, &sp_dm, &sp_dmir};
   }
+  // Runs attempt(rule), and if it has pair sums whose records and sums do not
+  // fit the device or the work area, with lists, which take less.
+  template <typename F>
+  void with_pair_sums(const PairSumRule& rule, F&& attempt) {
+    try {
+      attempt(rule);
+    } catch (const OutOfMemory&) {
+      if (!pair_sums) throw;
+      for (DeviceBuffer* b : {&tri, &psum, &hbuf}) b->release();
+      attempt(PairSumRule{});
+    }
+  }
   void use_arena(Arena* a) {
     arena = a;
     for (DeviceBuffer* b : buffers()) b->use_arena(a);
@@ -507,6 +528,11 @@ struct Workspace {
   DevWork work(const Prepared& pb, bool mixed, bool grad, const BatchOutput& out, const BatchDebug* debug);
   // count -> scans of the list sizes and of their work items (three-body lists of every atom)
   void list_offsets(const DevBatch& db, const void* pair, bool mixed, double4* acc, int2* items, hipStream_t stream);
+  // The bodies of Engine::run_pairwise and Engine::run_hessian.
+  void pairwise(const std::vector<SystemDesc>& systems, const int* numbers, const double* positions_dev, bool mixed,
+                double* pair2, double* pair3, hipStream_t stream, const int* ghost_host, const PairSumRule& rule);
+  void hessian(const std::vector<SystemDesc>& systems, const int* numbers, const double* positions_dev, double* energy,
+               double* hessian, hipStream_t stream, const int* ghost_host, const PairSumRule& rule);
   // pack .. disp2; then the three-body lists and kernel; then the chain
   // rule and the reduction.  capacity < 0: read the list size back and size
   // the slot buffer to it; otherwise use the fixed capacity and item bound.
@@ -1072,10 +1098,11 @@ void Engine::run(const std::vector<SystemDesc>& systems, const int* numbers, con
   if (systems.empty()) return;
   Workspace& m = *ws_;
   const bool grad = out.gradient || out.sigma;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host,
-                               stats ? PairSumRule{} : pair_sum_rule(precision == kMixed, grad));
-  m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, out, debug, stats, -1, 0, kPerCallShape,
-             stream);
+  m.with_pair_sums(stats ? PairSumRule{} : pair_sum_rule(precision == kMixed, grad), [&](const PairSumRule& rule) {
+    const Prepared pb = m.upload(systems, numbers, stream, ghost_host, rule);
+    m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, out, debug, stats, -1, 0, kPerCallShape,
+               stream);
+  });
   if (m.timer.enabled) m.timer.collect();
 }
 
@@ -1109,20 +1136,12 @@ void run_noalloc(const std::vector<SystemDesc>& systems, const int* numbers, con
   BatchOutput inner = out;
   inner.gradient = nullptr;
   Prepared pb;
-  auto attempt = [&](const PairSumRule& rule) {
+  m.with_pair_sums(pair_sum_rule(precision == kMixed, grad), [&](const PairSumRule& rule) {
     m.reset_arena();
     pb = m.upload(systems, numbers, stream, nullptr, rule);
     m.evaluate(pb, positions_dev, true, precision == kMixed, grad, pb.smooth, inner, nullptr, nullptr, -1, 0,
                kPerCallShape, stream);
-  };
-  // pair sums take 48 bytes a pair of atoms where lists take 40: a batch that
-  // only fits with lists gets them
-  try {
-    attempt(pair_sum_rule(precision == kMixed, grad));
-  } catch (const ArenaFull&) {
-    if (!m.pair_sums) throw;
-    attempt(PairSumRule{});
-  }
+  });
   if (out.gradient)
     hip_check(hipMemcpyAsync(out.gradient, m.grad.as<double>(size_t(pb.db.natoms) * 3),
                              sizeof(double) * 3 * size_t(pb.db.natoms), hipMemcpyDeviceToDevice, stream),
@@ -1137,9 +1156,17 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
   for (const auto& sd : systems)  // disp.f90:429-433
     if (sd.lowrank && sd.periodic[0] && sd.periodic[1] && sd.periodic[2])
       throw Error("Pairwise analysis is only available for the real space summation");
-  Workspace& m = *ws_;
-  const bool mixed = precision == kMixed;
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, pair_sum_rule(mixed, false));
+  ws_->with_pair_sums(pair_sum_rule(precision == kMixed, false), [&](const PairSumRule& rule) {
+    ws_->pairwise(systems, numbers, positions_dev, precision == kMixed, pair2, pair3, stream, ghost_host, rule);
+  });
+  if (ws_->timer.enabled) ws_->timer.collect();
+}
+
+void Workspace::pairwise(const std::vector<SystemDesc>& systems, const int* numbers, const double* positions_dev,
+                         bool mixed, double* pair2, double* pair3, hipStream_t stream, const int* ghost_host,
+                         const PairSumRule& rule) {
+  Workspace& m = *this;
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, rule);
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   m.pack(pb, positions_dev, stream, true);
@@ -1183,7 +1210,6 @@ void Engine::run_pairwise(const std::vector<SystemDesc>& systems, const int* num
   }
   if (pb.ps.count > 0) m.timed("atm", stream, [&] { launch_atm_pairsum(db, mixed, false, pb.ps, w, pair3, stream); });
   hip_check(hipGetLastError(), "kernel launch");
-  if (m.timer.enabled) m.timer.collect();
 }
 
 void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numbers, const double* positions_dev,
@@ -1194,7 +1220,6 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
   if (systems.empty()) return;
   for (const auto& sd : systems)  // disp.f90:113-119
     if (sd.lowrank) throw Error("Hessian is only available for the real space summation");
-  Workspace& m = *ws_;
   // three-body term by pair sums for molecules without a switching width
   // (the visits are the gradient's, three per triple, at any size cheaper than
   // the lists' global atomics)
@@ -1204,8 +1229,18 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
     lists = lists || sd.param.width3 > 0.0;
     bytes += static_cast<long long>(sd.natoms) * sd.natoms * static_cast<long long>(sizeof(double) * hess_pairsum_doubles());
   }
-  const Prepared pb = m.upload(systems, numbers, stream, ghost_host,
-                               lists || bytes > kPairSumBytes ? PairSumRule{} : PairSumRule{kPairSumAtoms});
+  ws_->with_pair_sums(lists || bytes > kPairSumBytes ? PairSumRule{} : PairSumRule{kPairSumAtoms},
+                      [&](const PairSumRule& rule) {
+                        ws_->hessian(systems, numbers, positions_dev, energy, hessian, stream, ghost_host, rule);
+                      });
+  if (ws_->timer.enabled) ws_->timer.collect();
+}
+
+void Workspace::hessian(const std::vector<SystemDesc>& systems, const int* numbers, const double* positions_dev,
+                        double* energy, double* hessian, hipStream_t stream, const int* ghost_host,
+                        const PairSumRule& rule) {
+  Workspace& m = *this;
+  const Prepared pb = m.upload(systems, numbers, stream, ghost_host, rule);
   const DevBatch& db = pb.db;
   const int natoms = db.natoms;
   double* e = energy ? energy : m.e_out.as<double>(static_cast<size_t>(db.nsys));
@@ -1245,7 +1280,6 @@ void Engine::run_hessian(const std::vector<SystemDesc>& systems, const int* numb
                    stream);
   });
   hip_check(hipGetLastError(), "kernel launch");
-  if (m.timer.enabled) m.timer.collect();
 }
 
 void Engine::count_terms(const std::vector<SystemDesc>& systems, const int* numbers, const double* positions_dev,
@@ -1292,6 +1326,9 @@ struct Plan::State {
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
   }
+  // Uploads the batch and sizes every buffer of an evaluation.
+  void prepare(const std::vector<SystemDesc>& systems, const int* numbers_host, const double* positions_dev,
+               const int* ghost_host, hipStream_t stream, const PairSumRule& rule);
   void drop_graph() {
     if (exec) hip_check(hipGraphExecDestroy(exec), "hipGraphExecDestroy");
     if (graph) hip_check(hipGraphDestroy(graph), "hipGraphDestroy");
@@ -1311,48 +1348,56 @@ Plan::Plan(const std::vector<SystemDesc>& systems, const int* numbers_host, cons
     State& s = *st_;
     s.mixed = precision == kMixed;
     s.grad = grad;
-    s.pb = s.ws.upload(systems, numbers_host, stream, ghost_host, pair_sum_rule(s.mixed, grad));
-    s.shape.num_cus = device_cu_count();
-    const int natoms = s.pb.db.natoms;
-    hip_check(hipMemsetAsync(s.ws.flag.as<int>(1), 0, sizeof(int), stream), "hipMemsetAsync");
-    // the spatial order of the planning coordinates is kept for every evaluation
-    s.ws.pack(s.pb, positions_dev, stream, true);
-    if (s.pb.any_atm) {
-      long long cap = s.pb.slot_bound;
-      if (s.pb.periodic_atm) {
-        // lists of the initial coordinates, with headroom for later ones
-        const DevWork w = s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
-        launch_cn(s.pb.db, s.mixed, w.cn, w.gw, w.dgw, w.gwr, w.spr, stream);
-        launch_pair(s.pb.db, s.mixed, w, false, grad, stream);
-        s.ws.list_offsets(s.pb.db, w.pair, s.mixed, w.atm_acc, nullptr, stream);
-        long long total = 0;
-        hip_check(hipMemcpyAsync(&total, s.ws.off.as<long long>(natoms + 1) + natoms, sizeof total,
-                                 hipMemcpyDeviceToHost, stream),
-                  "list size");
-        hip_check(hipStreamSynchronize(stream), "list size sync");
-        cap = std::min(cap, std::max(total + total / 2, total + 64LL * s.pb.atm_atoms));
-      }
-      s.capacity = cap;
-      s.max_items = std::min(s.pb.item_bound, cap / kTile + natoms);
-      // size every buffer now, so that an evaluation allocates nothing
-      (void)s.ws.slots.get(std::max<long long>(cap, 1) * slot_record_bytes(s.mixed));
-      (void)s.ws.items.as<int2>(std::max<long long>(s.max_items, 1));
-      (void)s.ws.cnt.as<long long>(natoms);
-      (void)s.ws.off.as<long long>(natoms + 1);
-      (void)s.ws.item_off.as<long long>(natoms + 1);
-      (void)s.ws.counter.as<unsigned long long>(kXcd * kCounterStride);
-    }
-    // until set_shape or autotune
-    const AtmShape a =
-        per_call_shape(s.mixed, s.pb.periodic_atm, s.pb.any_atm ? s.max_items : s.pb.shape_items);
-    s.shape.waves = a.waves;
-    s.shape.blocks_per_cu = a.blocks_per_cu;
-    (void)s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
-    hip_check(hipStreamSynchronize(stream), "plan sync");
+    s.ws.with_pair_sums(pair_sum_rule(s.mixed, grad), [&](const PairSumRule& rule) {
+      s.prepare(systems, numbers_host, positions_dev, ghost_host, stream, rule);
+    });
   } catch (...) {
     delete st_;
     throw;
   }
+}
+
+void Plan::State::prepare(const std::vector<SystemDesc>& systems, const int* numbers_host, const double* positions_dev,
+                          const int* ghost_host, hipStream_t stream, const PairSumRule& rule) {
+  State& s = *this;
+  s.pb = s.ws.upload(systems, numbers_host, stream, ghost_host, rule);
+  s.shape.num_cus = device_cu_count();
+  const int natoms = s.pb.db.natoms;
+  hip_check(hipMemsetAsync(s.ws.flag.as<int>(1), 0, sizeof(int), stream), "hipMemsetAsync");
+  // the spatial order of the planning coordinates is kept for every evaluation
+  s.ws.pack(s.pb, positions_dev, stream, true);
+  if (s.pb.any_atm) {
+    long long cap = s.pb.slot_bound;
+    if (s.pb.periodic_atm) {
+      // lists of the initial coordinates, with headroom for later ones
+      const DevWork w = s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
+      launch_cn(s.pb.db, s.mixed, w.cn, w.gw, w.dgw, w.gwr, w.spr, stream);
+      launch_pair(s.pb.db, s.mixed, w, false, grad, stream);
+      s.ws.list_offsets(s.pb.db, w.pair, s.mixed, w.atm_acc, nullptr, stream);
+      long long total = 0;
+      hip_check(hipMemcpyAsync(&total, s.ws.off.as<long long>(natoms + 1) + natoms, sizeof total,
+                               hipMemcpyDeviceToHost, stream),
+                "list size");
+      hip_check(hipStreamSynchronize(stream), "list size sync");
+      cap = std::min(cap, std::max(total + total / 2, total + 64LL * s.pb.atm_atoms));
+    }
+    s.capacity = cap;
+    s.max_items = std::min(s.pb.item_bound, cap / kTile + natoms);
+    // size every buffer now, so that an evaluation allocates nothing
+    (void)s.ws.slots.get(std::max<long long>(cap, 1) * slot_record_bytes(s.mixed));
+    (void)s.ws.items.as<int2>(std::max<long long>(s.max_items, 1));
+    (void)s.ws.cnt.as<long long>(natoms);
+    (void)s.ws.off.as<long long>(natoms + 1);
+    (void)s.ws.item_off.as<long long>(natoms + 1);
+    (void)s.ws.counter.as<unsigned long long>(kXcd * kCounterStride);
+  }
+  // until set_shape or autotune
+  const AtmShape a =
+      per_call_shape(s.mixed, s.pb.periodic_atm, s.pb.any_atm ? s.max_items : s.pb.shape_items);
+  s.shape.waves = a.waves;
+  s.shape.blocks_per_cu = a.blocks_per_cu;
+  (void)s.ws.work(s.pb, s.mixed, grad, BatchOutput{}, nullptr);
+  hip_check(hipStreamSynchronize(stream), "plan sync");
 }
 
 Plan::~Plan() { delete st_; }
