@@ -221,7 +221,7 @@ struct Prepared {
   long long slot_bound = 0;    // sum over the systems with lists of (il + 1) * images
   long long atm_atoms = 0;     // atoms of these systems
   long long item_bound = 0;    // work items of those bounds
-  long long shape_items = 0;   // work items if every three-body system had lists (launch shape of a plan)
+  long long shape_items = 0;   // work items if every three-body system had lists (the shape a plan without lists reports)
   bool ewald = false;          // the (single) system sums its two-body term in reciprocal space
   EwaldBatch eb{};             // its vectors, expansion and species chunks (nk = 0: no two-body term)
   bool spme = false;           // ... on a particle mesh instead of the vectors
@@ -351,10 +351,10 @@ int device_cu_count() {
 // wavefronts idle at the end of an item: two wavefronts per block and 8
 // blocks per CU, or, for lists with lattice images in mixed precision, one
 // and 16.  Measured (whole evaluations, ms, this shape / four wavefronts and
-// one block per item / best of the ten shapes): 2,000-atom cell mixed 13.08 /
-// 14.13 / 13.08, FP64 19.01 / 20.51 / 19.01; 20,000-atom ellipsoid mixed
-// 109.8 / 116.5 / 109.2, FP64 161.0 / 177.3 / 161.0; 1,000- and 2,000-atom
-// molecules mixed 0.93 / 0.99 / 0.90 and 3.36 / 3.60 / 3.26.
+// one block per item / best of the ten shapes): 2,000-atom cell mixed 13.13 /
+// 14.17 / 13.13, FP64 18.74 / 20.28 / 18.74; 20,000-atom ellipsoid mixed
+// 77.2 / 86.5 / 77.2, FP64 119.9 / 132.0 / 119.9; cubes of 2,000 and 4,500
+// atoms, mixed, 2.49 / 2.96 / 2.47 and 9.44 / 10.50 / 9.40.
 constexpr long long kLargeAtmItems = 8192;
 const AtmShape kPerCallShape{0, 0, 0};
 
@@ -382,7 +382,7 @@ AtmShape per_call_shape(bool mixed, bool periodic, long long items) {
 // 0.62 / 0.91, 1,500 1.40 / 1.56, 2,000 2.6 / 2.6 (a sphere 3.1 / 3.0); mixed
 // energy: 4,000 4.75 / 4.88.  Extended molecules cost less on both sides; FP64
 // gradient of 3,500 atoms: a wire of 2 x 2 atoms 0.45 / 0.52, a sheet of one
-// layer 0.84 / 0.90, of three layers 1.99 / 2.46.
+// layer 0.84 / 0.90, of three layers 1.89 / 2.46.
 constexpr int kPairSumAtoms = 3500, kPairSumAtomsMixedGrad = 1750;
 static_assert(kPairSumAtoms <= 64 * kTile, "a bit per tile of 64 positions (pair_kernel, atm_pairsum_kernel)");
 // With a three-body cutoff shorter than a molecule, fewer of the atoms that a
@@ -397,7 +397,7 @@ static_assert(kPairSumAtoms <= 64 * kTile, "a bit per tile of 64 positions (pair
 // 3.80, 1,000 4.48 / 4.22, 1,700 4.54 / 3.90; 26 bohr: 1,000 7.73 / 8.12, 1,700
 // 8.25 / 7.97.  In small batches the launches and waits of the lists weigh
 // more: one molecule of 1,700 atoms, FP64, 12 bohr 0.32 / 0.38, mixed, 20 bohr
-// 0.55 / 0.55; of 3,500 atoms, FP64, 12 bohr 0.85 / 0.95.  Energies are faster
+// 0.55 / 0.55; of 3,500 atoms, FP64, 12 bohr 0.78 / 0.95.  Energies are faster
 // by pair sums at every cutoff.
 constexpr double kPairSumPerCut3 = 0.0875, kPairSumPerCut3Mixed = 0.031;
 constexpr int kPairSumSmall = 500, kPairSumSmallMixed = 250;
@@ -978,8 +978,8 @@ void Workspace::evaluate(const Prepared& pb, const double* positions_dev, bool o
   // the Hessian (stats) and the work partition go by the reference's triangle
   db.rank_own = pb.any_cull && !pb.partitioned && !stats;
   // lists of lattice images, taken atom by atom, gain nothing from an XCD's own
-  // range (2,000-atom cell, mixed: 14.1 ms with one queue, 14.7 with eight;
-  // batch of 1,024 molecules, FP64: 6.0 and 5.7 ms)
+  // range (gradient, mixed: 2,000-atom cell 13.2 ms with one queue, 13.8 with
+  // eight; 20,000-atom ellipsoid 80.5 and 77.8)
   db.xcd_queues = !pb.periodic_atm;
   const int natoms = db.natoms;
   pack(pb, positions_dev, stream, order_atoms);

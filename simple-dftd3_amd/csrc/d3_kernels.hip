@@ -1003,10 +1003,11 @@ __device__ __forceinline__ long long tiles_of(long long slots) { return (slots +
 // longest lists) first.  Systems without lattice images: the atoms in groups
 // of kWave positions, within a group P by P, so that items taken at about the
 // same time pair the same slots for neighbouring atoms and read the same pair
-// records (see atm_body; batch of 1,024 molecules, FP64: 5.7 against 6.0 ms
-// atom by atom).  Lists of lattice images: atom by atom (the records repeat
-// within a tile, and the group order makes the slot sums of 64 atoms meet in
-// the same cache lines: 2,000-atom cell, mixed 14.1 against 15.2 ms).
+// records (see atm_body; 20,000-atom ellipsoid, gradient, FP64: 121 against
+// 130 ms atom by atom, mixed 77.8 against 81.2).  Lists of lattice images: atom
+// by atom (the records repeat within a tile, and the group order makes the slot
+// sums of 64 atoms meet in the same cache lines: 2,000-atom cell, gradient,
+// FP64 18.9 against 19.6 ms, mixed 13.2 both ways).
 // Wavefront per 64-position tile.
 __device__ __forceinline__ void emit_items(const DevBatch& b, int t, const long long* count, const long long* item_off,
                                            long long total, int2* items) {
@@ -1036,8 +1037,10 @@ __device__ __forceinline__ void emit_items(const DevBatch& b, int t, const long 
 // exclusive scan of the list sizes count[i] over the atoms, item_off[0..n] =
 // exclusive scan of their tile counts ceil(count[order[x]] / 64) over the
 // storage positions x.  One thread per element; a block first sums all
-// elements before its own (coalesced, from the L2), so one launch without a
-// serial chain over the blocks does both scans.  With items (a launch of one
+// elements before its own, the counts in order and, for the items, through
+// order[], from the L2, so one launch without a serial chain over the blocks
+// does both scans.  It reads n^2 / 2048 elements in all (20,000 atoms: 20 us,
+// of an evaluation of 77 ms).  With items (a launch of one
 // block, kScanBlock atoms or fewer) it writes the item table too.
 constexpr int kScanBlock = 1024;
 __global__ __launch_bounds__(kScanBlock) void list_scan_kernel(DevBatch b, const long long* count, long long* offset,
@@ -1256,9 +1259,11 @@ template <> __device__ __forceinline__ float pow_pos<float>(float x, float y) {
 // x**(-8/3) for normal x > 0, the damping power of the default alp = 14
 // (alp + 2 = 16, (r0/r)^((alp + 2)/3) with x = r^2): the FP32 hardware
 // estimate scaled into range in FP64, then one third-order step on
-// h = 1 - t^3 x^8, t <- t (1 + h / 3 + 2 h^2 / 9) (the estimate is good to
-// 2e-6, so the h^3 term dropped is below 1e-17): 9 FP64 operations where two
-// Newton steps on t^6 x^16 took 16.  The general power costs the device
+// h = 1 - t^3 x^8, t <- t (1 + h / 3 + 2 h^2 / 9): 9 FP64 operations where two
+// Newton steps on t^6 x^16 took 16.  The estimate's error is that of e, which
+// FP32 rounds: at most 2.9e-6 for distances of 1 to 100 bohr, where the first
+// term dropped, 14/81 h^3, is at most 1.1e-16 of t (7.3e-6 and 1.8e-15 for
+// 1e-4 to 1e6 bohr).  The general power costs the device
 // library's log2 and exp2 in FP64.
 __device__ __forceinline__ double pow_m8_3(double x) {
   const float e = (-8.0f / 3.0f) * __builtin_amdgcn_logf(static_cast<float>(x));
@@ -1389,11 +1394,14 @@ __device__ __forceinline__ TripleTerm<R> triple_term(R A, R B, R C, const R4<R>&
 // In large molecules the gather of the pair records from beyond the L2 was
 // the limit (without it 56 of 99 ms, 20,000-atom ellipsoid, mixed); the
 // lists by storage order and the item order let neighbouring atoms share
-// lines.  20,000-atom ellipsoid, mixed, whole step 111.8 -> 78.1 ms;
-// 1,501-atom molecule, FP64 energy 2.55 -> 1.81 ms.  Where a tile pair is
+// lines.  20,000-atom ellipsoid, mixed, whole step 111.8 -> 77.8 ms; cube of
+// 4,500 atoms, FP64 energy 17.0 -> 10.3 ms, mixed gradient 12.6 -> 9.5.  A sheet
+// of one layer of 2,500 atoms, whose lists have few dense tile pairs, takes
+// 0.64 instead of 0.59 ms (mixed gradient), of 4,500 atoms 0.93 and 0.91.  Where a tile pair is
 // mostly out of range the ring's compaction is cheaper: the share at which
 // the dense form is taken, 0.6 of the sample, is the middle of a flat range
-// (0.45, 0.6, 0.75: 79.2, 78.3, 79.2 ms).  Batches of smaller molecules and
+// (0.45, 0.6, 0.75: 79.2, 78.3, 79.2 ms).  The dense form takes registers from
+// the gradient kernels (see atm_kernel).  Batches of smaller molecules and
 // of cells keep the ring alone, whose kernel needs fewer registers (2,000-atom
 // cell, mixed: 14.1 against 15.0 ms with both forms in one kernel).
 //
@@ -1410,8 +1418,11 @@ __device__ __forceinline__ TripleTerm<R> triple_term(R A, R B, R C, const R4<R>&
 // term, to a random line, was most of the cost (pair energies, FP64, whole call:
 // cells of 1,000 atoms 45.8 -> 7.7 ms, of 2,000 atoms 78 -> 24 ms).  The number of cells is chosen from the images per
 // atom (launch_atm_pairs); a tile pair of more pairs of atoms adds its terms
-// directly.  One wavefront per block, so that the cells are private to it.  The pair energy of (x, y) is then pair3s(rx, ry) + pair3s(ry, rx)
-// (pair3_finalize_kernel).
+// directly, as do all of molecules above the size of the pair sums, whose tile
+// pairs have 64 x 64 pairs of atoms (cube of 4,500 atoms, FP64: 72.2 ms, 70.5
+// before there were cells; wire of 2 x 2 atoms 1.91 and 1.94).  One wavefront
+// per block, so that the cells are private to it.  The pair energy of (x, y) is
+// then pair3s(rx, ry) + pair3s(ry, rx) (pair3_finalize_kernel).
 // A tile pair of which kDenseShare or more of the kSample * 64 sampled slot
 // pairs are within the cutoff is evaluated densely.
 constexpr int kSample = 8;
@@ -1869,7 +1880,12 @@ __device__ __forceinline__ void atm_body(DevBatch b, const long long* __restrict
 
 // At least three wavefronts per SIMD in FP64 (the E+grad instantiation
 // otherwise takes 184 VGPRs, two wavefronts, and runs 14 % slower; with the
-// hint it takes 168 and spills a few dozen bytes) and four in FP32.
+// hint it takes 168 and 44 to 68 bytes of scratch a lane) and four in FP32.
+// With the dense form the gradient kernels of two and four wavefronts per
+// block hold these at the price of more scratch, 208 bytes in FP64 and 176 in
+// FP32 (320 and 192 with a switching width); those of one wavefront per block
+// and FP32, which no call without a plan takes for molecules, have 178
+// registers and two wavefronts.
 template <typename R, bool kGrad, bool kSmooth, int kW, bool kPart, bool kDense>
 __global__ __launch_bounds__(kW * kWave) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 3))) void atm_kernel(DevBatch b, const long long* __restrict__ item_off,
                                                          const int2* __restrict__ items,
@@ -1928,7 +1944,7 @@ __global__ __launch_bounds__(kWave) void atm_pairs_kernel(DevBatch b, const long
 // extended molecules, and cutoffs shorter than the molecule, more than the
 // lists had (FP64 gradient of 3,500 atoms, this kernel: wire of 2 x 2 atoms
 // 715 -> 87 us, sheet of one layer 2,046 -> 435, cube with a cutoff of 12 bohr
-// 1,659 -> 180; whole calls 1,207 -> 446, 2,579 -> 841, 2,323 -> 850, by lists
+// 1,659 -> 180; whole calls 1,207 -> 446, 2,579 -> 841, 2,323 -> 780, by lists
 // 520, 895, 913).  The lists of compact
 // systems spent most of their time on the distance tests, the LDS
 // atomics and the gathers: 1,501-atom molecule, FP64 energy, whole call 1.82
@@ -1945,7 +1961,8 @@ enum PairSumMode { kPsEnergy, kPsGrad, kPsPairs };
 //
 // Three wavefronts per SIMD with the gradient, four without: four with the
 // gradient spill (planned batch of 1,024 molecules 2.93 and 3.17 ms;
-// 1,501-atom molecule, energy, three and four 0.613 and 0.594 ms).
+// 1,501-atom molecule, energy, three and four 0.613 and 0.594 ms, with 32 bytes
+// of scratch for the tiles of 16).
 template <int kMode, int kT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kMode == kPsGrad ? 3 : 4)))
 void atm_pairsum_kernel(DevBatch b, const int2* __restrict__ items, const double4* __restrict__ tri,
@@ -2401,7 +2418,7 @@ __global__ __launch_bounds__(kBlock) void count_triples_kernel(DevBatch b, const
 //                                                  d/dCN_i, d2/dCN_i^2, d2/dCN_i dCN_j
 //   dr, dEdcndr            3n x n at 3 c6_begin    [3i+c][k]: dCN_k/dR_ic, d2E/dR_ic dCN_k
 //   dEdcndcn               n x n at c6_begin       d2E/dCN_k dCN_l
-//   tmp                    n x 3n at 3 c6_begin    dEdcndcn dr^T
+//   tmp                    3n x n at 3 c6_begin    dEdcndr + dr dEdcndcn / 2
 //   hess                   3n x 3n at 9 c6_begin   [3i+a][3j+b]
 // The two-body, CN and dCN/dR kernels own the rows of their atom (ordered
 // pairs (i, j, T) with u = R_i - R_j - T; every pair term is even in u or

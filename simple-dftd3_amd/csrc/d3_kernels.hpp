@@ -38,7 +38,7 @@ struct DevBatch {
   const double4* posr;  // [N] positions in that order, posr[x] = pos[order[x]] (refreshed with pos)
   int ntiles;
   int xcd_queues;       // persistent three-body launch: a work queue per XCD
-  int rank_own;         // large molecules: three-body lists by storage order (energy evaluations)
+  int rank_own;         // large molecules: three-body lists by storage order (energies and gradients of whole systems)
   const int2* tiles;    // [ntiles] first position and count of each 64-position tile of that order
   int* band;            // [nsys] a pair of the system is within kBand of the three-body cutoff (pair-sum route)
   // Pair-sum route: per tile of 2^reach_shift positions of a system's spatial
@@ -111,10 +111,10 @@ void launch_disp2(const DevBatch& b, bool mixed, bool grad, const DevWork& w, do
 // The count pass also clears acc (DevWork::atm_acc, may be null).
 void launch_atm_count(const DevBatch& b, const void* pair, bool mixed, long long* count, double4* acc,
                       hipStream_t stream);
-// offset[0..n] and item_off[0..n]: exclusive scans of the list sizes and of
-// their 64-slot tile counts (one block).
-// items (batches small enough for it, else null): the item table is written
-// by the same launch
+// offset[0..n]: exclusive scan of the list sizes over the atoms, item_off[0..n]:
+// of their 64-slot tile counts over the storage positions.
+// items (batches of one block of the scan, else null): the item table is
+// written by the same launch
 bool list_scan_writes_items(const DevBatch& b);
 void launch_list_scan(const DevBatch& b, const long long* count, long long* offset, long long* item_off, int2* items,
                       hipStream_t stream);
@@ -153,12 +153,12 @@ struct AtmShape {
 // partitioned: some system has a work partition of more than one part.
 void launch_atm(const DevBatch& b, bool mixed, bool grad, bool smooth, bool partitioned, const AtmShape& shape,
                 const long long* item_off, const int2* items, long long max_items, const long long* offset,
-                const void* slots,                const DevWork& w, unsigned long long* counter, hipStream_t stream);
-// images: about how many images of an atom a list holds (the least of the
-// systems), by which the LDS cells per tile pair are sized.
+                const void* slots, const DevWork& w, unsigned long long* counter, hipStream_t stream);
 // Pairwise three-body energies: adds the pair sums of every triple term to
 // pair3s (per system an n x n block in storage order, zeroed by the caller);
 // pair3_finalize writes the symmetric pair energies in atom order to out.
+// images: about how many images of an atom a list holds (the least of the
+// systems), by which the LDS cells per tile pair are sized.
 void launch_atm_pairs(const DevBatch& b, bool mixed, bool smooth, const long long* item_off, const int2* items,
                       long long max_items,
                       const long long* offset, const void* slots, const DevWork& w, double* pair3s, double images,
