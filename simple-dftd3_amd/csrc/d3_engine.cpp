@@ -375,45 +375,44 @@ AtmShape per_call_shape(bool mixed, bool periodic, long long items) {
 // gradient, at a third to a fifth of the lists' cost a visit, and a few
 // beyond it; the lists visit each triple once.
 //
-// kPairSumAtoms: ellipsoids 1:1:2 at 0.1 atoms per cubic Angstrom, whole
-// evaluations, ms, pair sums / lists; FP64 gradient: 500 atoms 0.23 / 0.44,
-// 1,000 0.64 / 1.08, 2,000 2.57 / 3.91, 3,000 6.67 / 7.75, 4,000 12.6 / 12.5;
-// FP64 energy: 1,000 0.31 / 0.78, 4,000 4.83 / 8.56; mixed gradient: 1,000
-// 0.62 / 0.91, 1,500 1.40 / 1.56, 2,000 2.6 / 2.6 (a sphere 3.1 / 3.0); mixed
-// energy: 4,000 4.75 / 4.88.  Extended molecules cost less on both sides; FP64
-// gradient of 3,500 atoms: a wire of 2 x 2 atoms 0.45 / 0.52, a sheet of one
-// layer 0.84 / 0.90, of three layers 1.89 / 2.46.
+// kPairSumAtoms: cubes of n atoms, 0.1 per cubic Angstrom, whole evaluations,
+// ms, pair sums / lists; FP64 gradient: 1,300 atoms 1.10 / 1.67, 2,500 4.68 /
+// 5.73, 3,500 8.80 / 9.83; FP64 energy: 3,500 2.59 / 6.78; mixed gradient: 1,300
+// 1.09 / 1.19, 1,700 1.97 / 2.00, 2,500 4.63 / 3.61; mixed energy: 3,500 2.50 /
+// 3.76.  Extended molecules cost less on both sides; FP64 gradient of 3,500
+// atoms: a wire of 2 x 2 atoms 0.45 / 0.52, a sheet of one layer 0.84 / 0.92, of
+// three layers 1.89 / 2.23.
 constexpr int kPairSumAtoms = 3500, kPairSumAtomsMixedGrad = 1750;
 static_assert(kPairSumAtoms <= 64 * kTile, "a bit per tile of 64 positions (pair_kernel, atm_pairsum_kernel)");
 // With a three-body cutoff shorter than a molecule, fewer of the atoms that a
 // pair of tiles visits are in range of each pair: in batches of more than
-// kPairSumLatency atoms the gradient takes the pair sums only up to this many
-// atoms per cubed cutoff (the atoms within the cutoff are some 0.06 of it, in
-// bohr, at that density), and always up to kPairSumSmall atoms.  Cubes of n
-// atoms, 0.1 per cubic Angstrom, 30,000 atoms a batch, ms, pair sums / lists;
-// mixed gradient, 12 bohr: 200 atoms 0.76 / 0.96, 300 1.66 / 1.47; 20 bohr: 300
-// 2.44 / 2.39, 500 3.35 / 2.87; 26 bohr: 300 2.83 / 3.73, 1,000 7.54 / 6.17;
-// FP64 gradient, 16 bohr: 500 2.53 / 2.54, 1,000 2.94 / 2.84; 20 bohr: 500 3.47 /
-// 3.80, 1,000 4.48 / 4.22, 1,700 4.54 / 3.90; 26 bohr: 1,000 7.73 / 8.12, 1,700
-// 8.25 / 7.97.  In small batches the launches and waits of the lists weigh
-// more: one molecule of 1,700 atoms, FP64, 12 bohr 0.32 / 0.38, mixed, 20 bohr
-// 0.55 / 0.55; of 3,500 atoms, FP64, 12 bohr 0.78 / 0.95.  Energies are faster
-// by pair sums at every cutoff.
-constexpr double kPairSumPerCut3 = 0.0875, kPairSumPerCut3Mixed = 0.031;
+// kPairSumLatency atoms the gradient takes the pair sums only up to a number of
+// atoms that goes with the cutoff (in bohr), and always up to kPairSumSmall
+// atoms.  Cubes of n atoms, 30,000 atoms a batch, ms, pair sums / lists; mixed
+// (0.75 cut3^2): 12 bohr: 200 atoms 0.76 / 0.85, 300 1.66 / 1.27; 20 bohr: 200
+// 0.94 / 1.37, 300 2.39 / 2.30, 500 3.32 / 2.75; 26 bohr: 500 4.44 / 4.90, 700
+// 6.06 / 4.64; 40 bohr: 1,000 12.4 / 14.0, 1,700 19.5 / 16.9; FP64 (0.055
+// cut3^3): 16 bohr: 400 2.17 / 2.24, 500 2.52 / 2.48, 1,000 2.94 / 2.64; 20 bohr:
+// 500 3.45 / 3.66, 700 4.13 / 3.74; 26 bohr: 700 6.24 / 6.64, 1,000 7.63 / 7.19;
+// 32 bohr: 1,700 13.0 / 13.3, 2,500 10.4 / 10.2.  In small batches the launches
+// and waits of the lists weigh more: one molecule of 1,700 atoms, FP64, 16 bohr
+// 0.41 / 0.48, mixed 0.39 / 0.41 (20 bohr 0.55 / 0.54); 8 of 500, FP64, 16 bohr
+// 0.38 / 0.44.  Energies are faster by pair sums at every cutoff.
+constexpr double kPairSumPerCut3 = 0.055, kPairSumPerCut2Mixed = 0.75;
 constexpr int kPairSumSmall = 500, kPairSumSmallMixed = 250;
 constexpr int kPairSumLatency = 4096;
 
 // Molecules of up to `atoms` atoms, and in larger batches of up to
-// max(small, per_cut3 cut3^3).
+// max(small, factor cut3^power).
 struct PairSumRule {
   int atoms = 0;  // 0: lists only
-  double per_cut3 = std::numeric_limits<double>::infinity();
-  int small = 0;
+  double factor = std::numeric_limits<double>::infinity();
+  int power = 0, small = 0;
 };
 PairSumRule pair_sum_rule(bool mixed, bool grad) {
   if (!grad) return {kPairSumAtoms};
-  return mixed ? PairSumRule{kPairSumAtomsMixedGrad, kPairSumPerCut3Mixed, kPairSumSmallMixed}
-               : PairSumRule{kPairSumAtoms, kPairSumPerCut3, kPairSumSmall};
+  return mixed ? PairSumRule{kPairSumAtomsMixedGrad, kPairSumPerCut2Mixed, 2, kPairSumSmallMixed}
+               : PairSumRule{kPairSumAtoms, kPairSumPerCut3, 3, kPairSumSmall};
 }
 // Tiles of 16 positions a side from this many tile pairs of the batch on, else
 // of 8, which spread a small batch over more wavefronts (gradient, ms, tiles of
@@ -637,8 +636,7 @@ Prepared Workspace::upload(const std::vector<SystemDesc>& systems, const int* nu
   auto pair_sum_route = [&](const SystemDesc& sd) {
     if (sd.periodic[0] || sd.periodic[1] || sd.periodic[2] || sd.nparts != 1 || sd.natoms > rule.atoms) return false;
     if (natoms <= kPairSumLatency || sd.natoms <= rule.small) return true;
-    const double c = sd.param.cut3;
-    return sd.natoms <= rule.per_cut3 * c * c * c;
+    return sd.natoms <= rule.factor * std::pow(sd.param.cut3, rule.power);
   };
   {
     long long bytes = 0;

@@ -117,15 +117,15 @@ def test_cost_follows_the_range():
 
 
 # atoms of a molecule, three-body cutoff, precision, gradient, molecules in the
-# batch, lists: the edges of the rule by the cutoff (0.031 and 0.0875 atoms per
-# cubed cutoff, 250 and 500 atoms, 4,096 atoms a batch)
+# batch, lists: the edges of the rule by the cutoff (0.75 atoms per squared cutoff,
+# 0.055 per cubed cutoff, 250 and 500 atoms, 4,096 atoms a batch)
 ROUTES = [
     (250, 12.0, "mixed", True, 17, False), (251, 12.0, "mixed", True, 17, True),
     (251, 12.0, "mixed", True, 16, False), (251, 12.0, "mixed", False, 17, False),
-    (600, 27.0, "mixed", True, 7, False), (600, 26.8, "mixed", True, 7, True),
+    (600, 28.4, "mixed", True, 7, False), (600, 28.2, "mixed", True, 7, True),
     (500, 12.0, "fp64", True, 9, False), (501, 12.0, "fp64", True, 9, True),
-    (501, 12.0, "fp64", False, 9, False), (600, 19.1, "fp64", True, 7, False),
-    (600, 18.9, "fp64", True, 7, True), (600, 12.0, "fp64", True, 6, False),
+    (501, 12.0, "fp64", False, 9, False), (600, 22.3, "fp64", True, 7, False),
+    (600, 22.1, "fp64", True, 7, True), (600, 12.0, "fp64", True, 6, False),
 ]
 
 
