@@ -292,8 +292,8 @@ D3HIP_API void d3hip_get_kernel_time(dftd3_error error, dftd3_model model, const
  * host synchronisation or device allocation, and can be recorded into a HIP
  * graph (d3hip_plan_capture) and replayed (d3hip_plan_replay).
  * Three-body lists: molecules of up to 3,500 atoms (1,750 in mixed precision
- * with gradient, fewer in batches with a short three-body cutoff) have none,
- * larger ones get the exact bound; periodic systems get 1.5x
+ * with gradient; with gradient in batches of more than 4,096 atoms fewer, by
+ * the three-body cutoff) have none, larger ones get the exact bound; periodic systems get 1.5x
  * the list size at the planning coordinates (at least 64 more slots per
  * atom of a system with a three-body term).  An evaluation whose lists do
  * not fit adds no three-body terms, writes NaN into the energy, gradient and
